@@ -11,186 +11,22 @@
 // for the FP64 shape.  The k-slots of one instruction may map to any 4 (FP32/FP64) or
 // 32 (BF16, 8 per slot) distinct k values as long as A and B agree, so each
 // lane reads 4 (resp. 8) consecutive k from LDS in one vector access.
-#include "dmrg_common.h"
+#include "gemm_kernels.h"
 #include "tile_order.h"
 
 namespace dmrg {
 
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef float flt4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-template <typename T> struct Mfma;
-template <> struct Mfma<double> {
-  typedef dbl4 acc_t;
-  static __device__ __forceinline__ acc_t op(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mfma<float> {
-  typedef flt4 acc_t;
-  static __device__ __forceinline__ acc_t op(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
-
-struct GemmArgs {
-  int M, N, K, lda, ldb, ldc;
-  long long sA, sB, sC, pA, pB, pC;
-  double alpha, beta;
-  int conjA, conjB;
-  int vec;     // 16-byte vector loads allowed (aligned pointers and strides)
-  int lower;   // skip tiles strictly above the diagonal (Hermitian C)
-};
-
 // ---------------------------------------------------------------------------
-// FP64 / FP32 kernel
-// ---------------------------------------------------------------------------
-template <typename T, bool CX, int TM, int TN, bool TA, bool TB, int TAG>
-__global__ __launch_bounds__(256) void gemm_mfma(const T* __restrict__ A, const T* __restrict__ B,
-                                                 T* __restrict__ C, GemmArgs g) {
-  constexpr int BM = 32 * TM, BN = 32 * TN, BK = 16;
-  constexpr int PAD = (sizeof(T) == 8) ? 2 : 4;
-  constexpr int NP = CX ? 2 : 1;
-  constexpr int LA = BM * BK / 256, LB = BN * BK / 256;
-  typedef typename Mfma<T>::acc_t acc_t;
-
-  __shared__ T As[NP][BM][BK + PAD];
-  __shared__ T Bs[NP][BN][BK + PAD];
-
-  const long long bz = blockIdx.z;
-  A += bz * g.sA;
-  B += bz * g.sB;
-  C += bz * g.sC;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  if (g.lower && block_above_diagonal(m0, n0, BM)) return;   // whole block above the diagonal
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int li = lane & 15, lk = lane >> 4;
-  const int M = g.M, N = g.N, K = g.K;
-
-  acc_t acc[NP][TM][TN];
-#pragma unroll
-  for (int p = 0; p < NP; ++p)
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int b = 0; b < TN; ++b) acc[p][a][b] = acc_t{0, 0, 0, 0};
-
-  T ra[NP][LA], rb[NP][LB];
-  const T sgnA = (CX && g.conjA) ? T(-1) : T(1);
-  const T sgnB = (CX && g.conjB) ? T(-1) : T(1);
-
-  auto load_regs = [&](int k0) {
-#pragma unroll
-    for (int e = 0; e < LA; ++e) {
-      int idx = tid + 256 * e;
-      int r, c;
-      if (!TA) { r = idx / BK; c = idx % BK; } else { c = idx / BM; r = idx % BM; }
-      int gm = m0 + r, gk = k0 + c;
-      bool ok = (gm < M) && (gk < K);
-      long long off = TA ? (long long)gk * g.lda + gm : (long long)gm * g.lda + gk;
-#pragma unroll
-      for (int p = 0; p < NP; ++p) ra[p][e] = ok ? A[off + p * g.pA] : T(0);
-    }
-#pragma unroll
-    for (int e = 0; e < LB; ++e) {
-      int idx = tid + 256 * e;
-      int r, c;  // r: n within tile, c: k within tile
-      if (!TB) { c = idx / BN; r = idx % BN; } else { r = idx / BK; c = idx % BK; }
-      int gn = n0 + r, gk = k0 + c;
-      bool ok = (gn < N) && (gk < K);
-      long long off = TB ? (long long)gn * g.ldb + gk : (long long)gk * g.ldb + gn;
-#pragma unroll
-      for (int p = 0; p < NP; ++p) rb[p][e] = ok ? B[off + p * g.pB] : T(0);
-    }
-  };
-  auto store_regs = [&]() {
-#pragma unroll
-    for (int e = 0; e < LA; ++e) {
-      int idx = tid + 256 * e;
-      int r, c;
-      if (!TA) { r = idx / BK; c = idx % BK; } else { c = idx / BM; r = idx % BM; }
-      As[0][r][c] = ra[0][e];
-      if (CX) As[NP - 1][r][c] = sgnA * ra[NP - 1][e];
-    }
-#pragma unroll
-    for (int e = 0; e < LB; ++e) {
-      int idx = tid + 256 * e;
-      int r, c;
-      if (!TB) { c = idx / BN; r = idx % BN; } else { r = idx / BK; c = idx % BK; }
-      Bs[0][r][c] = rb[0][e];
-      if (CX) Bs[NP - 1][r][c] = sgnB * rb[NP - 1][e];
-    }
-  };
-
-  load_regs(0);
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    store_regs();
-    __syncthreads();
-    if (k0 + BK < K) load_regs(k0 + BK);
-    T fa[NP][TM][4], fb[NP][TN][4];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) fa[p][a][t] = As[p][wm * TM * 16 + a * 16 + li][lk * 4 + t];
-#pragma unroll
-      for (int b = 0; b < TN; ++b)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) fb[p][b][t] = Bs[p][wn * TN * 16 + b * 16 + li][lk * 4 + t];
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-#pragma unroll
-      for (int a = 0; a < TM; ++a) {
-#pragma unroll
-        for (int b = 0; b < TN; ++b) {
-          if (!CX) {
-            acc[0][a][b] = Mfma<T>::op(fa[0][a][t], fb[0][b][t], acc[0][a][b]);
-          } else {
-            acc[0][a][b] = Mfma<T>::op(fa[0][a][t], fb[0][b][t], acc[0][a][b]);
-            acc[0][a][b] = Mfma<T>::op(-fa[NP - 1][a][t], fb[NP - 1][b][t], acc[0][a][b]);
-            acc[NP - 1][a][b] = Mfma<T>::op(fa[0][a][t], fb[NP - 1][b][t], acc[NP - 1][a][b]);
-            acc[NP - 1][a][b] = Mfma<T>::op(fa[NP - 1][a][t], fb[0][b][t], acc[NP - 1][a][b]);
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-
-  const T alpha = T(g.alpha), beta = T(g.beta);
-#pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        // accumulator row of element r: FP32 16x16x4 holds rows 4*(l/16)+r,
-        // FP64 16x16x4 holds rows 4*r+(l/16) (measured lane layouts)
-        const int rr = (sizeof(T) == 8) ? (4 * r + lk) : (lk * 4 + r);
-        int row = m0 + wm * TM * 16 + a * 16 + rr;
-        int col = n0 + wn * TN * 16 + b * 16 + li;
-        if (row < M && col < N) {
-          long long off = (long long)row * g.ldc + col;
-#pragma unroll
-          for (int p = 0; p < NP; ++p) {
-            T v = alpha * acc[p][a][b][r];
-            if (g.beta != 0.0) v += beta * C[off + p * g.pC];
-            C[off + p * g.pC] = v;
-          }
-        }
-      }
-}
-
-// ---------------------------------------------------------------------------
-// Real FP64 / FP32 kernel (the H_eff and environment GEMMs): 16-byte global
-// loads when the host found base pointers, leading dimensions and batch
-// strides multiples of 16 bytes (g.vec), element loads otherwise;
-// double-buffered LDS (one barrier per k-tile) and an XCD-aware tile order
-// (xcd_tile, tile_order.h).
+// Real FP64 / FP32 kernel for products with enough output tiles to fill the
+// chip (the H_eff, environment and Gram GEMMs at large bond dimensions):
+// operand tiles in double-buffered LDS, one barrier per k-tile, the next
+// k-tile's 16-byte vectors loaded into registers while the current one is
+// multiplied, XCD-aware tile order (xcd_tile, tile_order.h).  MFMA bound.
+// The loads carry no per-element bounds check (see load_full); with a check
+// and a branch around every vector the same loop ran the FP32 products
+// 5070 x 3428 x 845 / 3918 x 11696 x 653 / 10448 x 731 x 4386 at 72 / 83 /
+// 73 TFLOP/s, now 103 / 115 / 116, and 6144 x 16384 x 1024 at 112, now 130
+// (a large library product reaches 148).
 // ---------------------------------------------------------------------------
 
 // Tile (row, column) of this workgroup in the XCD-grouped order of
@@ -198,10 +34,6 @@ __global__ __launch_bounds__(256) void gemm_mfma(const T* __restrict__ A, const 
 __device__ __forceinline__ void xcd_tile(int nbx, int nby, int& tr, int& tc) {
   xcd_tile_of(blockIdx.x, blockIdx.y, nbx, nby, tr, tc);
 }
-template <typename T> struct Vec;
-template <> struct Vec<float> { typedef flt4 type; static constexpr int W = 4; };
-template <> struct Vec<double> { typedef double dbl2 __attribute__((ext_vector_type(2))); typedef dbl2 type; static constexpr int W = 2; };
-
 template <typename T, int TM, int TN, bool TA, bool TB, int TAG, typename CT = T>
 __global__ __launch_bounds__(256) void gemm_fast(const T* __restrict__ A, const T* __restrict__ B,
                                                  CT* __restrict__ C, GemmArgs g) {
@@ -230,12 +62,11 @@ __global__ __launch_bounds__(256) void gemm_fast(const T* __restrict__ A, const 
   if (g.lower) {
     // Hermitian C: row-major tiles (every XCD gets an even share of the
     // lower-triangle tiles), those strictly above the diagonal exit at once
-    const int lin = blockIdx.y * gridDim.x + blockIdx.x;
-    tr = lin / gridDim.x;
-    tc = lin % gridDim.x;
+    tr = blockIdx.x / g.nbx;
+    tc = blockIdx.x % g.nbx;
     if (tile_above_diagonal(tr, tc, BM, BN)) return;
   } else {
-    xcd_tile(gridDim.x, gridDim.y, tr, tc);
+    xcd_tile_of(blockIdx.x, 0, g.nbx, g.nby, tr, tc);
   }
   const int m0 = tr * BM, n0 = tc * BN;
 
@@ -252,55 +83,72 @@ __global__ __launch_bounds__(256) void gemm_fast(const T* __restrict__ A, const 
 
   vec_t ra[NA], rb[NB];
 
-  auto load_regs = [&](int k0) {
+  // Each thread's vectors: a wave-uniform base per k-tile plus one byte
+  // offset per vector.  A vector along m / n may run over the edge of its row
+  // into the next one (what it picks up there is not stored); in an edge tile
+  // the k-tile that holds the last k (for rows shorter than a vector, the
+  // last few) is therefore read element by element with a mask, as is a
+  // partial k-tile; all others (up to kfull) without.  Rows and columns
+  // wholly past the edge repeat the tile's first.
+  const char* Ab = reinterpret_cast<const char*>(A + (TA ? (long long)m0 : (long long)m0 * g.lda));
+  const char* Bb = reinterpret_cast<const char*>(B + (TB ? (long long)n0 * g.ldb : (long long)n0));
+  const bool overA = TA && m0 + BM > M, overB = !TB && n0 + BN > N;
+  const int kfull = !(overA || overB) ? K : K - 1 - ((TA && g.lda < VW) || (!TB && g.ldb < VW) ? VW : 0);
+  long long oa[NA], ob[NB];
+#pragma unroll
+  for (int e = 0; e < NA; ++e) {
+    const int v = tid + 256 * e;
+    int r, c;  // element (m = m0 + r, k = k0 + c) is the first of the vector
+    if (!TA) { r = v / (BK / VW); c = (v % (BK / VW)) * VW; } else { c = v / (BM / VW); r = (v % (BM / VW)) * VW; }
+    if (m0 + r >= M) r = 0;
+    oa[e] = (TA ? (long long)c * g.lda + r : (long long)r * g.lda + c) * (long long)sizeof(T);
+  }
+#pragma unroll
+  for (int e = 0; e < NB; ++e) {
+    const int v = tid + 256 * e;
+    int r, c;  // element (n = n0 + r, k = k0 + c)
+    if (!TB) { c = v / (BN / VW); r = (v % (BN / VW)) * VW; } else { r = v / (BK / VW); c = (v % (BK / VW)) * VW; }
+    if (n0 + r >= N) r = 0;
+    ob[e] = (TB ? (long long)r * g.ldb + c : (long long)c * g.ldb + r) * (long long)sizeof(T);
+  }
+  const long long ka = (TA ? (long long)g.lda : 1LL) * (long long)sizeof(T);   // byte stride of one k
+  const long long kb = (TB ? 1LL : (long long)g.ldb) * (long long)sizeof(T);
+
+  auto load_full = [&](int k0) {
+    const char* pa = Ab + k0 * ka;
+    const char* pb = Bb + k0 * kb;
+#pragma unroll
+    for (int e = 0; e < NA; ++e) __builtin_memcpy(&ra[e], pa + oa[e], sizeof(vec_t));
+#pragma unroll
+    for (int e = 0; e < NB; ++e) __builtin_memcpy(&rb[e], pb + ob[e], sizeof(vec_t));
+  };
+  auto load_masked = [&](int k0) {
 #pragma unroll
     for (int e = 0; e < NA; ++e) {
       const int v = tid + 256 * e;
-      int r, c;  // element (m = m0 + r, k = k0 + c) is the first of the vector
+      int r, c;
       if (!TA) { r = v / (BK / VW); c = (v % (BK / VW)) * VW; } else { c = v / (BM / VW); r = (v % (BM / VW)) * VW; }
-      const int gm = m0 + r, gk = k0 + c;
-      if (!TA) {
-        const T* p = A + (long long)gm * g.lda + gk;
-        if (g.vec && gm < M && gk + VW <= K) {
-          ra[e] = *reinterpret_cast<const vec_t*>(p);
-        } else {
 #pragma unroll
-          for (int j = 0; j < VW; ++j) ra[e][j] = (gm < M && gk + j < K) ? p[j] : T(0);
-        }
-      } else {
-        const T* p = A + (long long)gk * g.lda + gm;
-        if (g.vec && gk < K && gm + VW <= M) {
-          ra[e] = *reinterpret_cast<const vec_t*>(p);
-        } else {
-#pragma unroll
-          for (int j = 0; j < VW; ++j) ra[e][j] = (gk < K && gm + j < M) ? p[j] : T(0);
-        }
+      for (int j = 0; j < VW; ++j) {
+        const int gm = m0 + r + (TA ? j : 0), gk = k0 + c + (TA ? 0 : j);
+        ra[e][j] = (gm < M && gk < K) ? A[TA ? (long long)gk * g.lda + gm : (long long)gm * g.lda + gk] : T(0);
       }
     }
 #pragma unroll
     for (int e = 0; e < NB; ++e) {
       const int v = tid + 256 * e;
-      int r, c;  // element (n = n0 + r, k = k0 + c)
+      int r, c;
       if (!TB) { c = v / (BN / VW); r = (v % (BN / VW)) * VW; } else { r = v / (BK / VW); c = (v % (BK / VW)) * VW; }
-      const int gn = n0 + r, gk = k0 + c;
-      if (!TB) {
-        const T* p = B + (long long)gk * g.ldb + gn;
-        if (g.vec && gk < K && gn + VW <= N) {
-          rb[e] = *reinterpret_cast<const vec_t*>(p);
-        } else {
 #pragma unroll
-          for (int j = 0; j < VW; ++j) rb[e][j] = (gk < K && gn + j < N) ? p[j] : T(0);
-        }
-      } else {
-        const T* p = B + (long long)gn * g.ldb + gk;
-        if (g.vec && gn < N && gk + VW <= K) {
-          rb[e] = *reinterpret_cast<const vec_t*>(p);
-        } else {
-#pragma unroll
-          for (int j = 0; j < VW; ++j) rb[e][j] = (gn < N && gk + j < K) ? p[j] : T(0);
-        }
+      for (int j = 0; j < VW; ++j) {
+        const int gn = n0 + r + (TB ? 0 : j), gk = k0 + c + (TB ? j : 0);
+        rb[e][j] = (gn < N && gk < K) ? B[TB ? (long long)gn * g.ldb + gk : (long long)gk * g.ldb + gn] : T(0);
       }
     }
+  };
+  auto load_regs = [&](int k0) {
+    if (k0 + BK <= kfull) load_full(k0);
+    else load_masked(k0);
   };
   auto store_regs = [&](int buf) {
 #pragma unroll
@@ -327,10 +175,9 @@ __global__ __launch_bounds__(256) void gemm_fast(const T* __restrict__ A, const 
     }
   };
 
-  // FP64 64 x 64 tiles with beta != 0 (among them the tridiagonalisation's
-  // trailing updates, inner dimension 64): the C tile is loaded before the
-  // k-loop, so its read does not wait behind the MFMA work in the epilogue
-  // (the larger FP64 tile keeps its two waves per SIMD without it)
+  // FP64 tiles with beta != 0 (among them the tridiagonalisation's trailing
+  // updates, inner dimension 64): the C tile is loaded before the k-loop, so
+  // its read does not wait behind the MFMA work in the epilogue
   constexpr bool CPRE = sizeof(T) == 8 && sizeof(CT) == 8 && TM * TN <= 4;
   CT cpre[CPRE ? TM : 1][CPRE ? TN : 1][4];
   const bool pre = CPRE && g.beta != 0.0;
@@ -734,59 +581,20 @@ void gemm_b3nt(Ctx* c, int M, int N, int K, const __bf16* Ah, const __bf16* Al, 
 // ---------------------------------------------------------------------------
 // host dispatch
 // ---------------------------------------------------------------------------
-static GemmArgs make_args(const GemmDesc& d) {
-  GemmArgs g;
-  g.M = d.M; g.N = d.N; g.K = d.K;
-  g.lda = d.lda; g.ldb = d.ldb; g.ldc = d.ldc;
-  g.sA = d.sA; g.sB = d.sB; g.sC = d.sC;
-  g.pA = d.pA; g.pB = d.pB; g.pC = d.pC;
-  g.alpha = d.alpha; g.beta = d.beta;
-  g.conjA = d.conjA; g.conjB = d.conjB;
-  g.vec = 0;
-  g.lower = d.lower ? 1 : 0;
-  return g;
-}
-
 static void check_desc(const GemmDesc& d) {
   DMRG_REQUIRE(d.M >= 0 && d.N >= 0 && d.K >= 0 && d.batch >= 1, "gemm: negative size");
   DMRG_REQUIRE(d.batch <= 65535, "gemm: batch too large");
+  DMRG_REQUIRE(d.M <= 65535 * (d.field == CPLX ? 64 : 128), "gemm: M too large for one launch");
   DMRG_REQUIRE(d.ldc >= d.N || d.M <= 1, "gemm: ldc < N");
   DMRG_REQUIRE(d.transA ? (d.lda >= d.M || d.K <= 1) : (d.lda >= d.K || d.M <= 1), "gemm: bad lda");
   DMRG_REQUIRE(d.transB ? (d.ldb >= d.K || d.N <= 1) : (d.ldb >= d.N || d.K <= 1), "gemm: bad ldb");
 }
 
-// Launch helper: picks the instantiation for (transA, transB, tag).
-#define DMRG_GEMM_TAGS(X) X(0) X(1) X(2) X(3) X(4) X(5)
-
-template <typename T, bool CX, int TM, int TN, bool TA, bool TB>
-static void launch_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, T* C) {
-  GemmArgs g = make_args(d);
-  dim3 grid((d.N + 32 * TN - 1) / (32 * TN), (d.M + 32 * TM - 1) / (32 * TM), d.batch);
-  DMRG_REQUIRE(grid.y <= 65535, "gemm: M too large for one launch");
-  switch (d.tag) {
-#define CASE(t) \
-  case t: gemm_mfma<T, CX, TM, TN, TA, TB, t><<<grid, 256, 0, c->stream>>>(A, B, C, g); break;
-    DMRG_GEMM_TAGS(CASE)
-#undef CASE
-    default: throw Error("gemm: bad tag");
-  }
-  DMRG_CHECK_HIP(hipGetLastError());
-}
-
-template <typename T, bool CX, int TM, int TN>
-static void launch_tt(Ctx* c, const GemmDesc& d, const T* A, const T* B, T* C) {
-  if (!d.transA && !d.transB) launch_tagged<T, CX, TM, TN, false, false>(c, d, A, B, C);
-  else if (d.transA && !d.transB) launch_tagged<T, CX, TM, TN, true, false>(c, d, A, B, C);
-  else if (!d.transA && d.transB) launch_tagged<T, CX, TM, TN, false, true>(c, d, A, B, C);
-  else launch_tagged<T, CX, TM, TN, true, true>(c, d, A, B, C);
-}
-
+// Launch helpers: pick the instantiation for (transA, transB, tag).
 template <typename T, int TM, int TN, bool TA, bool TB, typename CT = T>
-static void launch_fast_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, bool vec) {
-  GemmArgs g = make_args(d);
-  g.vec = vec ? 1 : 0;
-  dim3 grid((d.N + 32 * TN - 1) / (32 * TN), (d.M + 32 * TM - 1) / (32 * TM), d.batch);
-  DMRG_REQUIRE(grid.y <= 65535, "gemm: M too large for one launch");
+static void launch_fast_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C) {
+  const GemmArgs g = make_args(d, 32 * TM, 32 * TN);
+  const dim3 grid((unsigned)g.nbx * g.nby, 1, d.batch);
   switch (d.tag) {
 #define CASE(t) \
   case t: gemm_fast<T, TM, TN, TA, TB, t, CT><<<grid, 256, 0, c->stream>>>(A, B, C, g); break;
@@ -798,19 +606,39 @@ static void launch_fast_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B
 }
 
 template <typename T, int TM, int TN, typename CT = T>
-static void launch_fast(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, bool vec) {
-  if (!d.transA && !d.transB) launch_fast_tagged<T, TM, TN, false, false, CT>(c, d, A, B, C, vec);
-  else if (d.transA && !d.transB) launch_fast_tagged<T, TM, TN, true, false, CT>(c, d, A, B, C, vec);
-  else if (!d.transA && d.transB) launch_fast_tagged<T, TM, TN, false, true, CT>(c, d, A, B, C, vec);
-  else launch_fast_tagged<T, TM, TN, true, true, CT>(c, d, A, B, C, vec);
+static void launch_fast(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C) {
+  if (!d.transA && !d.transB) launch_fast_tagged<T, TM, TN, false, false, CT>(c, d, A, B, C);
+  else if (d.transA && !d.transB) launch_fast_tagged<T, TM, TN, true, false, CT>(c, d, A, B, C);
+  else if (!d.transA && d.transB) launch_fast_tagged<T, TM, TN, false, true, CT>(c, d, A, B, C);
+  else launch_fast_tagged<T, TM, TN, true, true, CT>(c, d, A, B, C);
 }
 
-// 16-byte vector loads are legal when every row start is 16-byte aligned
-template <typename T>
-static bool vec_ok(const GemmDesc& d, const T* A, const T* B) {
-  const int vw = 16 / (int)sizeof(T);
-  auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  return al(A) && al(B) && d.lda % vw == 0 && d.ldb % vw == 0 && d.sA % vw == 0 && d.sB % vw == 0;
+// Which kernel a real product takes.  The LDS kernel runs 128 x 128 (FP32)
+// or 64 x 64 tiles; products whose 64 x 64 tiles would leave the 256 CUs idle
+// or badly balanced go to the direct-load kernel (gemm_direct.hip), which
+// spreads 16 x 16 / 32 x 32 tiles and splits the inner dimension.  Measured
+// (LDS 64 x 64 / direct, us):
+//   FP64  760 x 187 x 935 (36 tiles) 54 / 18;  1024 x 256 x 1280 (64) 70 / 24;
+//         650^3 (121) 40 / 24;  950 x 748 x 190 (180) 15.0 / 15.7;
+//         650 x 2000 x 128 (352) 15.4 / 16.5;  1280 x 1024 x 256 (320) 25.9 / 24.7;
+//         650 x 2588 x 2612 (451) 215 / 203;  6400 x 400 x 2400 (700) 285 / 293;
+//         3000 x 3000 x 512 (2209) 184 / 213
+//   FP32  4800 x 300 x 1800 (375) 80 / 93;  131 x 1 x 200 (3) 8.6 / 5.1
+// so FP64 changes at 512 tiles (160 for short inner dimensions, where a
+// workgroup has little to hide), FP32 at 200.
+static bool use_direct(const GemmDesc& d, bool f64) {
+  const long long tiles64 = (long long)((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
+  return tiles64 < (f64 ? (d.K <= 200 ? 160 : 512) : 200);
+}
+
+// FP32 tile of the LDS kernel: 128 x 128 where its tiles fill whole rounds of
+// the 256 CUs to three quarters (3918 x 11696 x 653: 522 us against 571 with
+// 64 x 64; 10448 x 731 x 4386, 492 tiles: 578 against 663), 64 x 64 otherwise
+// (857 x 857 x 3380 x 6, 294 tiles: 325 against 458; 4800 x 300 x 1800, 114
+// tiles: 80 against 135).
+static bool use_tile128(const GemmDesc& d) {
+  const long long t = (long long)((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
+  return 4 * t >= 3 * 256 * ((t + 255) / 256);
 }
 
 // Real FP32 GEMM writing an FP64 result (the R-step of the FP32 H_eff apply
@@ -819,37 +647,24 @@ void gemm_f32_c64(Ctx* c, const GemmDesc& d, const float* A, const float* B, dou
   DMRG_REQUIRE(d.field == REAL && d.beta == 0.0, "gemm_f32_c64: real field and beta = 0 only");
   check_desc(d);
   if (d.M == 0 || d.N == 0) return;
-  const long long tiles128 = (long long)((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
-  const int vw = 4;
-  auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  const bool vec = al(A) && al(B) && d.lda % vw == 0 && d.ldb % vw == 0 && d.sA % vw == 0 && d.sB % vw == 0;
-  if (tiles128 >= 256) launch_fast<float, 4, 4, double>(c, d, A, B, C, vec);
-  else launch_fast<float, 2, 2, double>(c, d, A, B, C, vec);
+  if (use_direct(d, false)) gemm_direct_f32_c64(c, d, A, B, C);
+  else if (use_tile128(d)) launch_fast<float, 4, 4, double>(c, d, A, B, C);
+  else launch_fast<float, 2, 2, double>(c, d, A, B, C);
 }
 
-// Tile choice: large problems use 128x128 (real) / 64x64 (complex) tiles;
-// problems that would leave the 256 CUs mostly idle drop to 64x64 / 32x32.
-// Real operands always take the fast kernel; complex ones the planar one.
-template <typename T>
-static void gemm_any(Ctx* c, const GemmDesc& d, const T* A, const T* B, T* C) {
+void gemm_f64(Ctx* c, const GemmDesc& d, const double* A, const double* B, double* C) {
   check_desc(d);
   if (d.M == 0 || d.N == 0) return;
-  long long tiles128 = (long long)((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
-  if (d.field == REAL) {
-    const bool vec = vec_ok(d, A, B);
-    // FP64 uses 128x64 tiles: a 128x128 FP64 tile needs ~380 registers per
-    // lane (one wave per SIMD); 128x64 keeps two
-    if (tiles128 >= 256) {
-      if (sizeof(T) == 8) launch_fast<T, 4, 2>(c, d, A, B, C, vec);
-      else launch_fast<T, 4, 4>(c, d, A, B, C, vec);
-    } else {
-      launch_fast<T, 2, 2>(c, d, A, B, C, vec);
-    }
-    return;
-  }
-  long long tiles64 = (long long)((d.M + 63) / 64) * ((d.N + 63) / 64) * d.batch;
-  if (tiles64 >= 512) launch_tt<T, true, 2, 2>(c, d, A, B, C);
-  else launch_tt<T, true, 1, 1>(c, d, A, B, C);
+  if (d.field == CPLX || use_direct(d, true)) gemm_direct_f64(c, d, A, B, C);
+  else launch_fast<double, 2, 2>(c, d, A, B, C);
+}
+
+void gemm_f32(Ctx* c, const GemmDesc& d, const float* A, const float* B, float* C) {
+  check_desc(d);
+  if (d.M == 0 || d.N == 0) return;
+  if (d.field == CPLX || use_direct(d, false)) gemm_direct_f32(c, d, A, B, C);
+  else if (use_tile128(d)) launch_fast<float, 4, 4>(c, d, A, B, C);
+  else launch_fast<float, 2, 2>(c, d, A, B, C);
 }
 
 // C[i][j] = conj(C[j][i]) for j > i (n x n, row pitch ld, imaginary plane at
@@ -884,16 +699,9 @@ void mirror_lower(Ctx* c, double* C, int n, int ld, long long plane, int field) 
   DMRG_CHECK_HIP(hipGetLastError());
 }
 
-void gemm_f64(Ctx* c, const GemmDesc& d, const double* A, const double* B, double* C) {
-  gemm_any<double>(c, d, A, B, C);
-}
-void gemm_f32(Ctx* c, const GemmDesc& d, const float* A, const float* B, float* C) {
-  gemm_any<float>(c, d, A, B, C);
-}
-
 template <bool CX, int TM, int TN, bool TA, bool TB>
 static void launch_b3_tagged(Ctx* c, const GemmDesc& d, const float* A, const float* B, float* C) {
-  GemmArgs g = make_args(d);
+  GemmArgs g = make_args(d, 32 * TM, 32 * TN);
   dim3 grid((d.N + 32 * TN - 1) / (32 * TN), (d.M + 32 * TM - 1) / (32 * TM), d.batch);
   DMRG_REQUIRE(grid.y <= 65535, "gemm: M too large for one launch");
   switch (d.tag) {
