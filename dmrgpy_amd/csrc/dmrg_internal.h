@@ -75,6 +75,12 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
 // sytrd_lower, with the same early stop over both planes)
 int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, double stop_tol = 0.0,
                 double* dropped = nullptr);
+// The same reductions with the matrix in registers, one launch for all
+// columns (trd_resident.hip): A[s0:, s0:] of the n x n matrix; false with
+// nothing changed when it cannot run
+bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double* e, double* tau, double stop_tol,
+                  double total2, int* done, double* dropped);
+int trd_resident_max(int field);   // largest order it takes
 // rows of Zt (keep x n, row-major: eigenvectors of the tridiagonal) <- rows
 // of Q Y for the first nrefl reflectors sytrd_lower left in A (all n - 1 by
 // default; dormtr L/lower/N by blocked compact-WY GEMMs)

@@ -1,5 +1,9 @@
 // Householder tridiagonalisation of a real symmetric matrix (LAPACK dsytrd,
-// lower storage conventions), two kernel launches per column.
+// lower storage conventions), two kernel launches per column.  Orders whose
+// rows fit the register files (real 3072, complex 1792) are reduced there in
+// one launch instead (trd_resident.hip); this path reduces larger matrices
+// down to that order by panels, and any order when the resident kernel gives
+// up.
 //
 // The dense symmetric eigensolver behind every Gram-route split spends most
 // of its time reducing the matrix to tridiagonal form, one column at a time.
@@ -457,14 +461,40 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
   double* sq_out = part2 + gmax2;    // 8 spare doubles before the state (two used)
   double stop2 = 0.0;
   const int sq_cap = gmax1 * TRD_PS;   // partial sums the launch-1 buffer holds
-  if (early) {
-    trailing_sumsq_async(c, A, n, 0, 1, part1, sq_cap, sq_out, 0);
-    stop2 = stop_tol * stop_tol * trailing_sumsq_wait(c, 0);
-  }
   int done = n - 1;   // reflectors computed
   int pend = -1;      // slot of a trailing-norm check in flight
+  // up to the order whose rows fit the register files the matrix is reduced
+  // there (trd_resident.hip); larger ones by panels down to that order
+  bool resident = n <= trd_resident_max(REAL);
+  if (resident && trd_resident(c, REAL, A, n, 0, d, e, tau, early ? stop_tol : 0.0, -1.0, &done, dropped)) {
+    if (done < n - 1) {
+      trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 1);
+      DMRG_CHECK_HIP(hipGetLastError());
+    }
+    for (int j = 0; j < done; ++j) ps.bytes += 8.0 * (double)(n - j - 1) * (n - j) / 2.0;
+    return done;
+  }
+  resident = !resident;   // try once
+  double total2 = 0.0;
+  if (early) {
+    trailing_sumsq_async(c, A, n, 0, 1, part1, sq_cap, sq_out, 0);
+    total2 = trailing_sumsq_wait(c, 0);
+    stop2 = stop_tol * stop_tol * total2;
+  }
   int g2prev = 1;
+  bool in_registers = false;
   for (int j0 = 0; j0 < n - 1; j0 += TRD_NB) {
+    if (resident && n - j0 <= trd_resident_max(REAL)) {
+      resident = false;
+      if (trd_resident(c, REAL, A, n, j0, d, e, tau, early ? stop_tol : 0.0, total2, &done, dropped)) {
+        in_registers = true;
+        if (done < n - 1) {
+          trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 1);
+          DMRG_CHECK_HIP(hipGetLastError());
+        }
+        break;
+      }
+    }
     const int nbp = std::min(TRD_NB, n - 1 - j0);
     for (int jj = 0; jj < nbp; ++jj) {
       const int j = j0 + jj;
@@ -515,7 +545,7 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
       pend = slot;
     }
   }
-  if (done == n - 1)
+  if (done == n - 1 && !in_registers)
     DMRG_CHECK_HIP(hipMemcpyAsync(d + (n - 1), A + (size_t)(n - 1) * n + (n - 1), sizeof(double),
                                   hipMemcpyDeviceToDevice, c->stream));
   // algorithmic bytes: the lower triangle of the trailing matrix, once per reduced column
@@ -933,14 +963,39 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
   double* sq_out = part2 + 2 * (size_t)gmax2;   // 8 spare doubles before the state (two used)
   double stop2 = 0.0;
   const int sq_cap = gmax1 * TRC_PS;
-  if (early) {
-    trailing_sumsq_async(c, A, n, 0, 2, part1, sq_cap, sq_out, 0);
-    stop2 = stop_tol * stop_tol * trailing_sumsq_wait(c, 0);
-  }
   int done = n - 1;
   int pend = -1;
+  // as in sytrd_lower: in registers where the order allows, panels down to it
+  bool resident = n <= trd_resident_max(CPLX);
+  if (resident && trd_resident(c, CPLX, A, n, 0, d, e, tau, early ? stop_tol : 0.0, -1.0, &done, dropped)) {
+    if (done < n - 1) {
+      trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 2);
+      DMRG_CHECK_HIP(hipGetLastError());
+    }
+    for (int j = 0; j < done; ++j) ps.bytes += 16.0 * (double)(n - j - 1) * (n - j) / 2.0;
+    return done;
+  }
+  resident = !resident;   // try once
+  double total2 = 0.0;
+  if (early) {
+    trailing_sumsq_async(c, A, n, 0, 2, part1, sq_cap, sq_out, 0);
+    total2 = trailing_sumsq_wait(c, 0);
+    stop2 = stop_tol * stop_tol * total2;
+  }
   int g2prev = 1;
+  bool in_registers = false;
   for (int j0 = 0; j0 < n - 1; j0 += TRD_NB) {
+    if (resident && n - j0 <= trd_resident_max(CPLX)) {
+      resident = false;
+      if (trd_resident(c, CPLX, A, n, j0, d, e, tau, early ? stop_tol : 0.0, total2, &done, dropped)) {
+        in_registers = true;
+        if (done < n - 1) {
+          trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 2);
+          DMRG_CHECK_HIP(hipGetLastError());
+        }
+        break;
+      }
+    }
     const int nbp = std::min(TRD_NB, n - 1 - j0);
     for (int jj = 0; jj < nbp; ++jj) {
       const int j = j0 + jj;
@@ -988,7 +1043,7 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
       pend = slot;
     }
   }
-  if (done == n - 1)
+  if (done == n - 1 && !in_registers)
     DMRG_CHECK_HIP(hipMemcpyAsync(d + (n - 1), A + (size_t)(n - 1) * n + (n - 1), sizeof(double),
                                   hipMemcpyDeviceToDevice, c->stream));
   // algorithmic bytes: the lower triangle of the trailing matrix (both planes) once per reduced column

@@ -1,0 +1,610 @@
+// Householder tridiagonalisation with the matrix held in registers: one
+// launch reduces a symmetric (or Hermitian) matrix of order m to tridiagonal
+// form, unblocked (LAPACK dsytd2 / zhetd2, lower), with one exchange between
+// the workgroups per column.
+//
+// The launch-per-column reduction (sytrd.hip) is bound by latency -- two
+// dependent launches and their memory round trips per column, 9 ... 13 us --
+// and, from order ~2000 on, by streaming the trailing matrix.  Here each of G
+// workgroups keeps RW consecutive rows of the matrix in registers (the
+// chip's register files hold 128 MB; order 2588 takes 54), so a column costs
+// no memory traffic but the exchange of two vectors, and the rank-2 update
+// (free of memory traffic too) needs no panel.  Per column J, every
+// workgroup redundantly holds the column a = A[:, J] spread over its threads:
+//
+//   v, tau, beta from a and |a|;  q = A v for its own rows;  publish q;
+//   read all of q and row J+1 of A (published by its owner);
+//   w = tau q - (tau^2 (q.v) / 2) v;   next column  A[:, J+1] - v w_1 - w;
+//   A -= v w^T + w v^T on its own rows, fused with the next A x.
+//
+// Exchange: every published word goes to its own address in a buffer that a
+// preceding kernel filled with one NaN pattern; readers poll each word
+// (relaxed device-scope atomics) until it differs.  A word carries its own
+// validity, so no fence, flag or cache write-back is needed.  Measured with
+// 16 / 32 / 64 / 128 / 256 workgroups exchanging 760 words: 1.6 / 2.1 / 2.5 /
+// 3.0 / 3.2 us.  All waits are bounded: a workgroup that waits longer than
+// the limit (other work holding the CUs its peers need) gives up, as then do
+// the others, the input is untouched and the caller runs the
+// launch-per-column reduction instead.
+//
+// Measured per column, launch-per-column / resident (us): real order 128
+// 8.7 / 2.5, 380 9.8 / 3.2, 2588 (900 columns reduced) 16.2 / 8.4; complex
+// order 1200 14.5 / 6.6.  What bounds a column is the exchange (two thirds of
+// it at 216 workgroups), then the chain of two workgroup-wide reductions.
+#include "dmrg_internal.h"
+
+#include <algorithm>
+#include <cstring>
+
+namespace dmrg {
+
+constexpr unsigned long long RES_EMPTY = ~0ull;                  // a NaN no arithmetic produces; see publish()
+constexpr unsigned long long RES_NAN = 0x7FF8000000000000ull;
+constexpr long long RES_LIMIT = 5000000;                          // wall-clock ticks (100 MHz): 50 ms
+constexpr int RES_CHECK = 32, RES_CHECK_MIN = 64;                 // early-stop checks: every 32 columns from 64 on
+
+struct ResArgs {
+  const double* A;             // m x m, row pitch lda, imaginary plane at +pA
+  long long lda, pA;
+  int m, mp;                   // order, order padded to a multiple of 16
+  int col0, n;                 // absolute column of the first one, order of the whole matrix
+  unsigned long long* X;       // exchange: per column [2 (row, q)][planes][mp]
+  unsigned long long* chk;     // per early-stop check [2][gridDim.x]
+  double* R;                   // reflectors: row J, columns J+2 ... (m x m, planes m*m apart)
+  double *d, *e, *tau;         // at col0 (tau interleaved when complex)
+  int early;
+  double tol2, total2;         // stop when |trailing|_F^2 <= tol2 * total2 (total2 < 0: of this matrix)
+  int* status;                 // [0] 1 = gave up, [1] columns reduced
+  double* trace;               // trace of the block left when stopped early
+};
+
+__device__ __forceinline__ void publish(unsigned long long* p, double x) {
+  unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  if (u == RES_EMPTY) u = RES_NAN;
+  __hip_atomic_store(p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long peek(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double as_d(unsigned long long u) { return __longlong_as_double((long long)u); }
+
+// N words p[idx[i]] once they are all published; false after RES_LIMIT ticks
+template <int N>
+__device__ __forceinline__ bool await(const unsigned long long* p, const int (&idx)[N], double (&out)[N]) {
+  unsigned long long u[N];
+  long long t0 = 0;
+  for (int spin = 0;; ++spin) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) u[i] = peek(p + idx[i]);
+    bool miss = false;
+#pragma unroll
+    for (int i = 0; i < N; ++i) miss |= u[i] == RES_EMPTY;
+    if (!miss) break;
+    if ((spin & 63) == 63) {
+      const long long t = wall_clock64();
+      if (t0 == 0) t0 = t;
+      else if (t - t0 > RES_LIMIT) return false;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) out[i] = as_d(u[i]);
+  return true;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp(double x) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (unsigned)u, CTRL, 0xF, 0xF, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (unsigned)(u >> 32), CTRL, 0xF, 0xF, true);
+  return as_d(((unsigned long long)hi << 32) | lo);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;
+
+// a and b summed over lane pairs 32 (16) apart: the result holds a's sums in
+// the lanes with that bit clear and b's in the others
+__device__ __forceinline__ double fold32(double a, double b) {
+  const unsigned long long ua = (unsigned long long)__double_as_longlong(a), ub = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+  return as_d(((unsigned long long)hi[0] << 32) | lo[0]) + as_d(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+  const unsigned long long ua = (unsigned long long)__double_as_longlong(a), ub = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+  return as_d(((unsigned long long)hi[0] << 32) | lo[0]) + as_d(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+
+// Wave sums of 16 values at once, each stage halving the registers: lane l
+// ends with the sum of value bits (l>>2 & 1) + 2 (l>>3 & 1) + 4 (l>>4 & 1) +
+// 8 (l>>5 & 1).  A fixed order (63 instructions against 300 for 16 butterflies).
+__device__ __forceinline__ double wave_sums16(const double (&v)[16], int lane) {
+  double s[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) s[t] = fold32(v[t], v[t + 8]);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) s[t] = fold16(s[t], s[t + 4]);
+  const bool b3 = lane & 8, b2 = lane & 4;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const double keep = b3 ? s[t + 2] : s[t], send = b3 ? s[t] : s[t + 2];
+    s[t] = keep + dpp<DPP_MIRROR>(send);
+  }
+  const double keep = b2 ? s[1] : s[0], send = b2 ? s[0] : s[1];
+  double x = keep + dpp<DPP_HALF_MIRROR>(send);
+  x += dpp<DPP_XOR2>(x);
+  x += dpp<DPP_XOR1>(x);
+  return x;
+}
+__device__ __forceinline__ int sum_index(int lane) {
+  return ((lane >> 2) & 1) | ((lane >> 2) & 2) | ((lane >> 2) & 4) | ((lane >> 2) & 8);
+}
+
+// Wave sums of two values: lanes < 32 end with a's, the others with b's
+__device__ __forceinline__ double wave_sums2(double a, double b) {
+  double x = fold32(a, b);
+  x = fold16(x, x);      // both rows of a half: the same sum
+  x += dpp<DPP_MIRROR>(x);
+  x += dpp<DPP_HALF_MIRROR>(x);
+  x += dpp<DPP_XOR2>(x);
+  x += dpp<DPP_XOR1>(x);
+  return x;
+}
+
+__device__ __forceinline__ double lane_value(double x, int l) {   // wave-uniform
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, l), hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), l);
+  return as_d(((unsigned long long)hi << 32) | lo);
+}
+
+// T threads, thread t holds columns t, t + T, ... (CC of them) of RW rows.
+// At most 15 reduced values beside the norm (RW real, 2 RW complex).
+template <bool CX, int T, int CC, int RW>
+__global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
+  constexpr int NP = CX ? 2 : 1, NW = T / 64, NS = NP * RW;   // NS sums + the norm at index NS
+  static_assert(NS <= 15, "reduction holds 16 values");
+  __shared__ double red[NW * 16], red2[NW * 2];
+  __shared__ double sA1[NP][16], sa[2][NP][16], sq[NP][16];
+  __shared__ double2 svw[NW][NP][16];   // (v, w) of the own rows, one copy per wave
+  __shared__ double s_a0[NP], s_d;
+  __shared__ int s_bad;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wg = blockIdx.x, G = gridDim.x, m = g.m, mp = g.mp;
+  const int row0 = wg * RW, last = min(row0 + RW, m) - 1;
+  const bool writer = wg == G - 1;
+  if (tid == 0) s_bad = 0;
+
+  // own rows (conj(buffer) when complex: the reduction works on the column-major view)
+  double M[NP][RW][CC], a[NP][CC], v[NP][CC], w[NP][CC];
+#pragma unroll
+  for (int k = 0; k < CC; ++k) {
+    const int c = tid + T * k;
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const bool ok = c < m && row0 + i < m;
+      const long long o = (long long)(row0 + i) * g.lda + c;
+      M[0][i][k] = ok ? g.A[o] : 0.0;
+      if (CX) M[NP - 1][i][k] = ok ? -g.A[o + g.pA] : 0.0;
+    }
+    a[0][k] = c < m ? g.A[c] : 0.0;
+    if (CX) a[NP - 1][k] = c < m ? g.A[c + g.pA] : 0.0;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) v[p][k] = w[p][k] = 0.0;
+  }
+  double total2 = g.total2;
+  double tr = 0.0, ti = 0.0, Kr = 0.0, Ki = 0.0, scr = 0.0, sci = 0.0;   // tau, w = tau q + K v, v = scale a
+
+  for (int J = 0;; ++J) {
+    const int par = J & 1;
+    // ---- rank-2 update of column J-1 on the own rows, fused with A x for column J
+    double acc[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) acc[t] = 0.0;
+    double nrm = 0.0;
+#pragma unroll
+    for (int k = 0; k < CC; ++k) {
+      const int c = tid + T * k;
+      if (c == J) s_d = a[0][k];
+      if (c == J + 1) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) s_a0[p] = a[p][k];
+      }
+      if (c >= row0 && c < row0 + RW) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) sa[par][p][c - row0] = a[p][k];
+      }
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {   // from here on only a[J+2:] is wanted
+        a[p][k] = c >= J + 2 ? a[p][k] : 0.0;
+        nrm += a[p][k] * a[p][k];
+      }
+    }
+    if (J > 0) {
+      if (lane < RW) {   // v and w of the own rows (column J-1; rows from J on)
+        const int r = row0 + lane;
+        double vr = 0.0, vi = 0.0, wr = 0.0, wi = 0.0;
+        if (r >= J && r < m) {
+          const double ar = sa[par ^ 1][0][lane], ai = CX ? sa[par ^ 1][NP - 1][lane] : 0.0;
+          vr = r == J ? 1.0 : scr * ar - sci * ai;
+          vi = r == J ? 0.0 : scr * ai + sci * ar;
+          const double qr = sq[0][lane], qi = CX ? sq[NP - 1][lane] : 0.0;
+          wr = tr * qr - ti * qi + Kr * vr - Ki * vi;
+          wi = tr * qi + ti * qr + Kr * vi + Ki * vr;
+        }
+        svw[wave][0][lane] = double2{vr, wr};
+        if (CX) svw[wave][NP - 1][lane] = double2{vi, wi};
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      double2 pr = double2{0.0, 0.0}, pi = double2{0.0, 0.0};
+      if (J > 0) {
+        pr = svw[wave][0][i];
+        if (CX) pi = svw[wave][NP - 1][i];
+      }
+#pragma unroll
+      for (int k = 0; k < CC; ++k) {
+        if (!CX) {
+          const double t = M[0][i][k] - (pr.x * w[0][k] + pr.y * v[0][k]);
+          M[0][i][k] = t;
+          acc[i] += t * a[0][k];
+        } else {   // B -= v conj(w) + w conj(v)
+          const double wr = w[0][k], wi = w[NP - 1][k], vr = v[0][k], vi = v[NP - 1][k];
+          const double tre = M[0][i][k] - (pr.x * wr + pi.x * wi + pr.y * vr + pi.y * vi);
+          const double tim = M[NP - 1][i][k] - (pi.x * wr - pr.x * wi + pi.y * vr - pr.y * vi);
+          M[0][i][k] = tre;
+          M[NP - 1][i][k] = tim;
+          acc[i] += tre * a[0][k] - tim * a[NP - 1][k];
+          acc[RW + i] += tre * a[NP - 1][k] + tim * a[0][k];
+        }
+      }
+    }
+    acc[NS] = nrm;
+    // ---- row J+1 for everybody's next column; column J+1 of the own rows
+    unsigned long long* Xc = g.X + (long long)J * (2 * NP * mp);
+    unsigned long long* Xq = Xc + NP * mp;
+    const int i1 = J + 1 - row0;
+    if (i1 >= 0 && i1 < RW && J + 1 < m) {
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+        if (i == i1) {
+#pragma unroll
+          for (int k = 0; k < CC; ++k) {
+            const int c = tid + T * k;
+            if (c > J && c < m) {
+#pragma unroll
+              for (int p = 0; p < NP; ++p) publish(Xc + p * mp + c, M[p][i][k]);
+            }
+          }
+        }
+    }
+    const int k1 = (J + 1) / T;
+#pragma unroll
+    for (int k = 0; k < CC; ++k)
+      if (k == k1 && tid == J + 1 - T * k) {
+#pragma unroll
+        for (int i = 0; i < RW; ++i)
+#pragma unroll
+          for (int p = 0; p < NP; ++p) sA1[p][i] = M[p][i][k];
+      }
+    {
+      const double s = wave_sums16(acc, lane);
+      if ((lane & 3) == 0) red[wave * 16 + sum_index(lane)] = s;
+    }
+    __syncthreads();
+    // ---- early stop: |A[J:, J:]|_F^2 against the whole matrix's
+    const int s_abs = g.col0 + J;
+    const bool first = J == 0 && g.early && total2 < 0.0;
+    if (first || (g.early && J > 0 && s_abs >= RES_CHECK_MIN && s_abs % RES_CHECK == 0 && s_abs < g.n - 1)) {
+      double q2 = 0.0, dg = 0.0;
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+#pragma unroll
+        for (int k = 0; k < CC; ++k) {
+          const int c = tid + T * k, r = row0 + i;
+          if (r >= J && c >= J) {   // zero past the order
+#pragma unroll
+            for (int p = 0; p < NP; ++p) q2 += M[p][i][k] * M[p][i][k];
+            if (r == c) dg += M[0][i][k];
+          }
+        }
+      const double s = wave_sums2(q2, dg);
+      if (lane == 0) red2[wave * 2] = s;
+      if (lane == 32) red2[wave * 2 + 1] = s;
+      __syncthreads();
+      unsigned long long* ck = g.chk + (long long)(s_abs / RES_CHECK) * 2 * G;
+      if (tid < 2) {
+        double t = 0.0;
+#pragma unroll
+        for (int u = 0; u < NW; ++u) t += red2[u * 2 + tid];
+        publish(ck + tid * G + wg, t);
+      }
+      __syncthreads();
+      double f2 = 0.0, tc = 0.0;
+      for (int o = J / RW + tid; o < G; o += T) {   // the workgroups that hold rows from J on
+        const int idx[2] = {o, G + o};
+        double y[2] = {0.0, 0.0};
+        if (!await<2>(ck, idx, y)) s_bad = 1;
+        f2 += y[0];
+        tc += y[1];
+      }
+      const double ss = wave_sums2(f2, tc);
+      if (lane == 0) red2[wave * 2] = ss;
+      if (lane == 32) red2[wave * 2 + 1] = ss;
+      __syncthreads();
+      f2 = tc = 0.0;
+#pragma unroll
+      for (int u = 0; u < NW; ++u) {
+        f2 += red2[u * 2];
+        tc += red2[u * 2 + 1];
+      }
+      const bool bad = s_bad != 0;
+      __syncthreads();
+      if (bad) {
+        if (tid == 0) g.status[0] = 1;
+        return;
+      }
+      if (first) {
+        total2 = f2;
+      } else if (f2 <= g.tol2 * total2) {
+        if (writer && tid == 0) {
+          g.status[1] = J;
+          g.trace[0] = tc;
+        }
+        return;
+      }
+    }
+    // ---- reflector of column J (every workgroup, the same sums in the same order)
+    double tot = 0.0;
+    if (lane < 16) {
+#pragma unroll
+      for (int u = 0; u < NW; ++u) tot += red[u * 16 + lane];
+    }
+    const double xn2 = lane_value(tot, NS);
+    const double a0r = s_a0[0], a0i = CX ? s_a0[NP - 1] : 0.0;
+    double beta;
+    if (!CX) {
+      const double xn = sqrt(xn2);
+      tr = 0.0;
+      beta = a0r;
+      scr = 0.0;
+      if (xn != 0.0) {
+        beta = -copysign(hypot(a0r, xn), a0r);
+        tr = (beta - a0r) / beta;
+        scr = 1.0 / (a0r - beta);
+      }
+    } else {
+      // an exactly zero sub-column with a real a0 takes the reflection
+      // tau = 2, v = e_{J+1}, as in the launch-per-column reduction
+      tr = 2.0;
+      ti = 0.0;
+      beta = -a0r;
+      scr = sci = 0.0;
+      if (xn2 != 0.0 || a0i != 0.0) {
+        beta = -copysign(hypot(hypot(a0r, a0i), sqrt(xn2)), a0r);
+        tr = (beta - a0r) / beta;
+        ti = -a0i / beta;
+        const double dr = a0r - beta, di = a0i, den = dr * dr + di * di;
+        scr = dr / den;
+        sci = -di / den;
+      }
+    }
+    // ---- q = A v for the own rows
+    if (wave == 0) {
+      const double ti_ = CX ? __shfl(tot, RW + lane) : 0.0;
+      const int r = row0 + lane;
+      if (lane < RW) {
+        const double qr = sA1[0][lane] + scr * tot - sci * ti_;
+        const double qi = CX ? sA1[NP - 1][lane] + scr * ti_ + sci * tot : 0.0;
+        if (r > J && r < m) {
+          publish(Xq + r, qr);
+          if (CX) publish(Xq + mp + r, qi);
+        }
+        sq[0][lane] = qr;
+        if (CX) sq[NP - 1][lane] = qi;
+      }
+    }
+    double* Rj = g.R + (long long)J * m;
+#pragma unroll
+    for (int k = 0; k < CC; ++k) {
+      const int c = tid + T * k;
+      const double ar = a[0][k], ai = CX ? a[NP - 1][k] : 0.0;
+      v[0][k] = c >= J + 2 && c < m ? scr * ar - sci * ai : (c == J + 1 ? 1.0 : 0.0);
+      if (CX) v[NP - 1][k] = c >= J + 2 && c < m ? scr * ai + sci * ar : 0.0;
+      if (writer && c >= J + 2 && c < m) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) Rj[(long long)p * m * m + c] = v[p][k];
+      }
+    }
+    if (writer && tid == 0) {
+      g.d[J] = s_d;
+      g.e[J] = beta;
+      if (CX) {
+        g.tau[2 * J] = tr;
+        g.tau[2 * J + 1] = ti;
+      } else {
+        g.tau[J] = tr;
+      }
+    }
+    // ---- everybody's q, and row J+1
+    double cv[NP][CC], qv[NP][CC], q1[NP];
+    {
+      int idx[CC];
+#pragma unroll
+      for (int k = 0; k < CC; ++k) {
+        const int c = tid + T * k;
+        idx[k] = c > J && c < m ? c : J + 1;
+      }
+      const int one[1] = {J + 1};
+      bool ok = true;
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        double y1[1] = {0.0};
+        ok = ok && await<CC>(Xq + p * mp, idx, qv[p]);
+        ok = ok && await<1>(Xq + p * mp, one, y1);
+        ok = ok && await<CC>(Xc + p * mp, idx, cv[p]);
+        q1[p] = y1[0];
+      }
+      if (!ok) s_bad = 1;
+    }
+    // q^H v (conj(q) v summed over the rows past J)
+    double sr = 0.0, si = 0.0;
+#pragma unroll
+    for (int k = 0; k < CC; ++k) {   // v is zero up to J and past the order
+      sr += qv[0][k] * v[0][k];
+      if (CX) {
+        sr += qv[NP - 1][k] * v[NP - 1][k];
+        si += qv[0][k] * v[NP - 1][k] - qv[NP - 1][k] * v[0][k];
+      }
+    }
+    {
+      const double s = wave_sums2(sr, si);
+      if (lane == 0) red2[wave * 2] = s;
+      if (lane == 32) red2[wave * 2 + 1] = s;
+    }
+    __syncthreads();
+    if (s_bad) {
+      if (tid == 0) g.status[0] = 1;
+      return;
+    }
+    sr = si = 0.0;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+      sr += red2[u * 2];
+      if (CX) si += red2[u * 2 + 1];
+    }
+    // K = -(tau / 2) (w0^H v) with w0 = tau q:  w0^H v = conj(tau) q^H v
+    const double zr = tr * sr + ti * si, zi = tr * si - ti * sr;
+    Kr = -0.5 * (tr * zr - ti * zi);
+    Ki = -0.5 * (tr * zi + ti * zr);
+    const double q1r = q1[0], q1i = CX ? q1[NP - 1] : 0.0;
+    const double w1r = tr * q1r - ti * q1i + Kr, w1i = tr * q1i + ti * q1r + Ki;
+#pragma unroll
+    for (int k = 0; k < CC; ++k) {
+      const int c = tid + T * k;
+      const bool in = c > J && c < m;
+      const double vr = v[0][k], vi = CX ? v[NP - 1][k] : 0.0;
+      const double qr = qv[0][k], qi = CX ? qv[NP - 1][k] : 0.0;
+      w[0][k] = in ? tr * qr - ti * qi + Kr * vr - Ki * vi : 0.0;
+      if (CX) w[NP - 1][k] = in ? tr * qi + ti * qr + Kr * vi + Ki * vr : 0.0;
+      // column J+1: conj(row J+1) - v conj(w_1) - w
+      a[0][k] = in ? cv[0][k] - (vr * w1r + vi * w1i) - w[0][k] : 0.0;
+      if (CX) a[NP - 1][k] = in ? -cv[NP - 1][k] - (vi * w1r - vr * w1i) - w[NP - 1][k] : 0.0;
+      if (J == m - 2 && writer && c == m - 1) g.d[m - 1] = a[0][k];
+    }
+    if (J == m - 2 || last < J + 1) return;
+  }
+}
+
+// every word of the exchange and of the checks empty, status cleared
+__global__ void trd_resident_fill_k(unsigned long long* __restrict__ X, long long nx, unsigned long long* __restrict__ chk,
+                                    long long nc, int* __restrict__ status, int m) {
+  const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x, st = (long long)gridDim.x * blockDim.x;
+  for (long long i = i0; i < nx; i += st) X[i] = RES_EMPTY;
+  for (long long i = i0; i < nc; i += st) chk[i] = RES_EMPTY;
+  if (i0 == 0) {
+    status[0] = 0;
+    status[1] = m - 1;
+  }
+}
+
+// the reflectors into the rows of the matrix (row j, columns j+2 ...)
+__global__ __launch_bounds__(256) void trd_resident_store_k(const double* __restrict__ R, int m, int done,
+                                                            double* __restrict__ A, long long lda, long long pA,
+                                                            int planes) {
+  const int j = blockIdx.x;
+  if (j >= done) return;
+  for (int p = 0; p < planes; ++p)
+    for (int c = j + 2 + threadIdx.x; c < m; c += 256)
+      A[(long long)p * pA + (long long)j * lda + c] = R[((long long)p * m + j) * m + c];
+}
+
+template <bool CX, int T, int CC, int RW>
+static bool resident_launch(Ctx* c, const ResArgs& g, int G) {
+  // every workgroup must be resident at once: they wait for each other
+  int per_cu = 0, cus = 0;
+  DMRG_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trd_resident_k<CX, T, CC, RW>, T, 0));
+  DMRG_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
+  if ((long long)per_cu * cus < G) return false;
+  trd_resident_k<CX, T, CC, RW><<<G, T, 0, c->stream>>>(g);
+  DMRG_CHECK_HIP(hipGetLastError());
+  return true;
+}
+
+int trd_resident_max(int field) { return field == CPLX ? 256 * 7 : 256 * 12; }
+
+// Reduces A[s0:, s0:] of the n x n matrix A (in place: reflectors into its
+// rows) as sytrd_lower / hetrd_lower do; false (nothing changed) when the
+// order is out of range, the workgroups do not all fit, or a wait ran out.
+// *done: absolute number of columns reduced; *dropped: trace of the rest.
+bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double* e, double* tau, double stop_tol,
+                  double total2, int* done, double* dropped) {
+  const bool cx = field == CPLX;
+  const int m = n - s0, np = cx ? 2 : 1;
+  if (m < 3 || m > trd_resident_max(field)) return false;
+  // workgroup size and rows per workgroup: 15 rows (7 complex) fill the
+  // 16-value reduction; larger orders take 12 so that the rows fit the
+  // registers (512 threads, 256 registers each)
+  const int T = m <= 256 ? 256 : 512, CC = (m + T - 1) / T;
+  const int RW = cx ? 7 : (CC <= 2 ? 15 : 12);
+  const int G = (m + RW - 1) / RW;
+  ResArgs g;
+  g.A = A + (long long)s0 * n + s0;
+  g.lda = n;
+  g.pA = (long long)n * n;
+  g.m = m;
+  g.mp = (m + 15) / 16 * 16;
+  g.col0 = s0;
+  g.n = n;
+  const long long nx = (long long)(m - 1) * 2 * np * g.mp;
+  const long long nc = (long long)(n / RES_CHECK + 1) * 2 * G;
+  unsigned char* buf = (unsigned char*)ws_get(c, WS_TRD_X, 8 * (size_t)(nx + nc) + 64);
+  g.X = (unsigned long long*)buf;
+  g.chk = g.X + nx;
+  g.status = (int*)(g.chk + nc);
+  g.trace = (double*)(g.status + 2);
+  g.R = (double*)ws_get(c, WS_TRD_R, sizeof(double) * np * (size_t)m * m);
+  g.d = d + s0;
+  g.e = e + s0;
+  g.tau = tau + (size_t)np * s0;
+  g.early = stop_tol > 0.0 ? 1 : 0;
+  g.tol2 = stop_tol * stop_tol;
+  g.total2 = total2;
+  trd_resident_fill_k<<<2048, 256, 0, c->stream>>>(g.X, nx, g.chk, nc, g.status, m);
+  DMRG_CHECK_HIP(hipGetLastError());
+  bool ok = false;
+  if (!cx) {
+    if (T == 256) ok = resident_launch<false, 256, 1, 15>(c, g, G);
+    else switch (CC) {
+      case 1: ok = resident_launch<false, 512, 1, 15>(c, g, G); break;
+      case 2: ok = resident_launch<false, 512, 2, 15>(c, g, G); break;
+      case 3: ok = resident_launch<false, 512, 3, 12>(c, g, G); break;
+      case 4: ok = resident_launch<false, 512, 4, 12>(c, g, G); break;
+      case 5: ok = resident_launch<false, 512, 5, 12>(c, g, G); break;
+      case 6: ok = resident_launch<false, 512, 6, 12>(c, g, G); break;
+    }
+  } else {
+    if (T == 256) ok = resident_launch<true, 256, 1, 7>(c, g, G);
+    else switch (CC) {
+      case 1: ok = resident_launch<true, 512, 1, 7>(c, g, G); break;
+      case 2: ok = resident_launch<true, 512, 2, 7>(c, g, G); break;
+      case 3: ok = resident_launch<true, 512, 3, 7>(c, g, G); break;
+      case 4: ok = resident_launch<true, 512, 4, 7>(c, g, G); break;
+    }
+  }
+  if (!ok) return false;
+  DMRG_CHECK_HIP(hipMemcpyAsync(c->host_scalars + 36, g.status, 16, hipMemcpyDeviceToHost, c->stream));
+  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  int st[2];
+  std::memcpy(st, c->host_scalars + 36, sizeof(st));
+  if (st[0] != 0) return false;
+  trd_resident_store_k<<<st[1], 256, 0, c->stream>>>(g.R, m, st[1], A + (long long)s0 * n + s0, n, g.pA, np);
+  DMRG_CHECK_HIP(hipGetLastError());
+  *done = s0 + st[1];
+  if (st[1] < m - 1 && dropped) *dropped = std::max(0.0, c->host_scalars[37]);
+  return true;
+}
+
+}  // namespace dmrg
