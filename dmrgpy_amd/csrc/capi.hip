@@ -185,10 +185,12 @@ int dmrg_ctx_create(int device, void* stream, dmrg_ctx** out) {
   rocblas_set_stream(h->c.blas, h->c.stream);
   DMRG_CHECK_HIP(hipHostMalloc((void**)&h->c.host_scalars, 64 * sizeof(double), hipHostMallocDefault));
   std::memset(h->c.host_scalars, 0, 64 * sizeof(double));
+  DMRG_CHECK_HIP(hipHostMalloc((void**)&h->c.host_parts, (1024 + 8) * sizeof(double), hipHostMallocDefault));
   try {
     h->c.scratch = scratch_address(device);   // device current (hipSetDevice above)
   } catch (...) {
     (void)hipHostFree(h->c.host_scalars);
+    (void)hipHostFree(h->c.host_parts);
     rocblas_destroy_handle(h->c.blas);
     delete h;
     throw;
@@ -211,6 +213,7 @@ int dmrg_ctx_destroy(dmrg_ctx* ctx) {
     if (e) (void)hipEventDestroy(e);
   for (int i = 0; i < dmrg::WS_NSLOTS; ++i) c.ws[i].release();
   if (c.host_scalars) (void)hipHostFree(c.host_scalars);
+  if (c.host_parts) (void)hipHostFree(c.host_parts);
   if (c.blas) rocblas_destroy_handle(c.blas);
   delete ctx;
   API_END

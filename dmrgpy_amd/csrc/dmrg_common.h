@@ -87,6 +87,7 @@ struct Ctx {
   rocblas_handle blas = nullptr;
   DevBuf ws[WS_NSLOTS];
   double* host_scalars = nullptr;  // pinned, for scalar read-back
+  double* host_parts = nullptr;    // pinned, 1024 partial sums + 8 scalars kernels write directly
   // profiling: H_eff applies (kind 0), environment updates (1), SVDs (2),
   // Krylov vector work (3), tridiagonalisations (4)
   bool prof_on = false;

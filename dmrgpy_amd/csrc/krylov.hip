@@ -3,11 +3,13 @@
 // (FP64, planar complex); only the projected tridiagonal matrix and a handful
 // of scalars per iteration come to the host, once per iteration.
 //
-// Vector work per iteration k (n elements per plane, sizeof = 8):
-//   dot + axpy + block re-orthogonalisation (k dots, k axpys) + norm,
-//   about (2k + 6) * n * 8 bytes of HBM traffic: bandwidth bound.
+// Vector work per iteration k (n elements per plane, sizeof = 8): three
+// kernels after the apply (kry_alpha_k, kry_project_k, kry_clean_k), about
+// (2k + 7) * n * 8 bytes of HBM traffic -- bandwidth bound for long vectors,
+// launch bound for short ones.
 #include "dmrg_internal.h"
 #include "host_eig.h"
+#include "wave_reduce.h"
 
 #include <cfloat>
 #include <cmath>
@@ -185,6 +187,257 @@ static void scale_copy(Ctx* c, const double* src, double* dst, double s, long lo
   DMRG_CHECK_HIP(hipGetLastError());
 }
 
+// ---------------------------------------------------------------------------
+// One Krylov step's vector work.  With w = H q_k on entry:
+//   alpha = Re <q_k|w>;  w -= alpha q_k + beta q_{k-1};
+//   c_j = <q_j|w> for the basis vectors to re-orthogonalise against;
+//   w -= sum_j c_j q_j;  |w|^2.
+// A sum over workgroups ends one kernel and the next one's workgroups each
+// add up the partial sums (in the same fixed order: deterministic); the last
+// one's and alpha go straight to pinned host memory, where the host adds them
+// up after its one synchronisation per step.  The separate dot / reduce /
+// subtract kernels and scalar copies this replaces were 15 launches; the
+// block dot product walked the basis one vector at a time, with a
+// workgroup-wide sum after each (complex n = 16384, 20 vectors: 19 us, now 5).
+// ---------------------------------------------------------------------------
+constexpr int KRY_T = 256;
+constexpr int KRY_MAXBLK = 1024;
+
+// Workgroups: enough for short vectors to fill the chip (256 elements each),
+// few enough that re-reading the partial sums of every basis vector in every
+// workgroup stays small next to the vectors themselves (the larger counts are
+// for vectors of at least 2M / 8M elements).
+static int kry_blocks(long long n) {
+  const long long cap = n >= (8LL << 20) ? 1024 : (n >= (2LL << 20) ? 512 : 256);
+  return (int)std::max<long long>(1, std::min<long long>(cap, (n + KRY_T - 1) / KRY_T));
+}
+
+// this workgroup's elements [beg, end)
+__device__ __forceinline__ void kry_range(long long n, long long& beg, long long& end) {
+  long long chunk = (n + gridDim.x - 1) / gridDim.x;
+  chunk = (chunk + KRY_T - 1) / KRY_T * KRY_T;
+  beg = (long long)blockIdx.x * chunk;
+  end = beg + chunk < n ? beg + chunk : n;
+}
+
+// sum of one value per thread over the workgroup; valid in thread 0
+__device__ __forceinline__ double kry_block_sum(double x, double* sh) {
+  x = wave_sums2(x, 0.0);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return threadIdx.x == 0 ? sh[0] + sh[1] + sh[2] + sh[3] : 0.0;
+}
+
+// part[0..nb) added up by every wave (the same order everywhere)
+__device__ __forceinline__ double kry_sum_parts(const double* __restrict__ part, int nb) {
+  double x = 0.0;
+  for (int b = threadIdx.x & 63; b < nb; b += 64) x += part[b];
+  return lane_value(wave_sums2(x, 0.0), 0);
+}
+
+// part[block] = sum of Re(conj(a) b) over the workgroup's elements
+template <bool CX>
+__global__ __launch_bounds__(KRY_T) void kry_alpha_k(const double* __restrict__ a, const double* __restrict__ b,
+                                                     long long n, double* __restrict__ part) {
+  __shared__ double sh[4];
+  long long beg, end;
+  kry_range(n, beg, end);
+  double s = 0.0;
+#pragma unroll 4
+  for (long long i = beg + threadIdx.x; i < end; i += KRY_T) {
+    s += a[i] * b[i];
+    if (CX) s += a[i + n] * b[i + n];
+  }
+  s = kry_block_sum(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// Partial dot products of the NB basis vectors from j0 on (those past the
+// last: repeated, not stored) with this workgroup's elements of w
+template <bool CX, int NB>
+__device__ __forceinline__ void kry_dots(const double* __restrict__ Q, long long ldq, int j0, int k,
+                                         const double* __restrict__ w, long long n, long long beg, long long end,
+                                         double* red, double* __restrict__ part2) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double acc[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) acc[t] = 0.0;
+  for (long long i = beg + tid; i < end; i += KRY_T) {
+    const double wr = w[i], wi = CX ? w[i + n] : 0.0;
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      const double* v = Q + (long long)min(j0 + t, k - 1) * ldq;
+      const double vr = v[i];
+      if (CX) {
+        const double vi = v[i + n];
+        acc[t] += vr * wr + vi * wi;
+        acc[(NB + t) & 15] += vr * wi - vi * wr;
+      } else {
+        acc[t] += vr * wr;
+      }
+    }
+  }
+  const double s = wave_sums16(acc, lane);
+  __syncthreads();   // the previous batch's sums are read
+  if ((lane & 3) == 0) red[wave * 16 + sum_index(lane)] = s;
+  __syncthreads();
+  if (tid < (CX ? 2 * NB : NB)) {
+    const int j = j0 + tid % NB;
+    if (j < k)
+      part2[(long long)(tid < NB ? j : k + j) * gridDim.x + blockIdx.x] =
+          red[tid] + red[16 + tid] + red[32 + tid] + red[48 + tid];
+  }
+}
+
+// alpha from part1 (to host_alpha); w -= alpha q + beta qp (qp null: no second
+// term); then the partial dot products c_j of Q_0 .. Q_{k-1} with w, k x nblk
+// (imaginary parts after the k real rows), or with k = 0 the partial |w|^2
+template <bool CX>
+__global__ __launch_bounds__(KRY_T) void kry_project_k(const double* __restrict__ q, const double* __restrict__ qp,
+                                                       double beta, const double* __restrict__ part1, int nb1,
+                                                       const double* __restrict__ Q, long long ldq, int k, double* w,
+                                                       long long n, double* __restrict__ part2,
+                                                       double* __restrict__ host_alpha) {
+  __shared__ double red[4 * 16];
+  const int tid = threadIdx.x;
+  const double alpha = kry_sum_parts(part1, nb1);
+  if (blockIdx.x == 0 && tid == 0) *host_alpha = alpha;
+  long long beg, end;
+  kry_range(n, beg, end);
+  double nrm = 0.0;
+#pragma unroll 2
+  for (long long i = beg + tid; i < end; i += KRY_T) {   // each thread reads back only its own elements below
+    double wr = w[i] - alpha * q[i], wi = CX ? w[i + n] - alpha * q[i + n] : 0.0;
+    if (qp) {
+      wr -= beta * qp[i];
+      if (CX) wi -= beta * qp[i + n];
+    }
+    w[i] = wr;
+    nrm += wr * wr;
+    if (CX) {
+      w[i + n] = wi;
+      nrm += wi * wi;
+    }
+  }
+  if (k == 0) {
+    nrm = kry_block_sum(nrm, red);
+    if (tid == 0) part2[blockIdx.x] = nrm;
+    return;
+  }
+  // batches of up to 16 sums, the last one rounded up to a power of two
+  constexpr int MAXB = CX ? 8 : 16;
+  int j0 = 0;
+  for (; k - j0 > MAXB / 2; j0 += MAXB) kry_dots<CX, MAXB>(Q, ldq, j0, k, w, n, beg, end, red, part2);
+  const int rest = k - j0;
+  if (rest <= 0) return;
+  if (!CX && rest > 4) kry_dots<CX, CX ? 4 : 8>(Q, ldq, j0, k, w, n, beg, end, red, part2);
+  else if (rest > 2) kry_dots<CX, 4>(Q, ldq, j0, k, w, n, beg, end, red, part2);
+  else if (rest > 1) kry_dots<CX, 2>(Q, ldq, j0, k, w, n, beg, end, red, part2);
+  else kry_dots<CX, 1>(Q, ldq, j0, k, w, n, beg, end, red, part2);
+}
+
+// c_j from part2 (k x nb); w -= sum_j c_j Q_j; partial |w|^2 to host_norm
+constexpr int KRY_COEF = 512;   // coefficients held at a time
+template <bool CX>
+__global__ __launch_bounds__(KRY_T) void kry_clean_k(const double* __restrict__ Q, long long ldq, int k,
+                                                     const double* __restrict__ part2, int nb, double* w, long long n,
+                                                     double* __restrict__ host_norm) {
+  __shared__ double cr[KRY_COEF], ci[CX ? KRY_COEF : 1];
+  __shared__ double sh[4];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  long long beg, end;
+  kry_range(n, beg, end);
+  double nrm = 0.0;
+  for (int j0 = 0; j0 < k; j0 += KRY_COEF) {
+    const int kb = min(KRY_COEF, k - j0);
+    __syncthreads();   // the previous coefficients are used
+    for (int r = wave; r < (CX ? 2 * kb : kb); r += 4) {
+      const int row = r < kb ? j0 + r : k + j0 + (r - kb);
+      const double x = kry_sum_parts(part2 + (long long)row * nb, nb);
+      if ((tid & 63) == 0) {
+        if (r < kb) cr[r] = x;
+        else ci[CX ? r - kb : 0] = x;
+      }
+    }
+    __syncthreads();
+    const bool last = j0 + KRY_COEF >= k;
+    for (long long i = beg + tid; i < end; i += KRY_T) {
+      double wr = w[i], wi = CX ? w[i + n] : 0.0;
+#pragma unroll 8
+      for (int j = 0; j < kb; ++j) {
+        const double* v = Q + (long long)(j0 + j) * ldq;
+        const double vr = v[i];
+        if (CX) {
+          const double vi = v[i + n];
+          wr -= cr[j] * vr - ci[j] * vi;
+          wi -= cr[j] * vi + ci[j] * vr;
+        } else {
+          wr -= cr[j] * vr;
+        }
+      }
+      w[i] = wr;
+      if (CX) w[i + n] = wi;
+      if (last) {
+        nrm += wr * wr;
+        if (CX) nrm += wi * wi;
+      }
+    }
+  }
+  nrm = kry_block_sum(nrm, sh);
+  if (tid == 0) host_norm[blockIdx.x] = nrm;
+}
+
+static double sum_host(const double* p, int nb) {
+  double s = 0.0;
+  for (int b = 0; b < nb; ++b) s += p[b];
+  return s;
+}
+
+// |x| (one kernel, the partial sums added up on the host)
+static double krylov_norm(Ctx* c, int field, const double* x, long long n) {
+  const int nb = kry_blocks(n);
+  double* hp = c->host_parts;
+  {
+    ProfScope ps(c, 3, 0.0, 8.0 * (field == CPLX ? 2 : 1) * (double)n);
+    if (field == CPLX) kry_alpha_k<true><<<nb, KRY_T, 0, c->stream>>>(x, x, n, hp);
+    else kry_alpha_k<false><<<nb, KRY_T, 0, c->stream>>>(x, x, n, hp);
+    DMRG_CHECK_HIP(hipGetLastError());
+  }
+  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  return std::sqrt(std::max(sum_host(hp, nb), 0.0));
+}
+
+// The step above for basis vector `it`, re-orthogonalising against the first
+// k of Q; returns alpha, and |w| in *beta_new
+static double krylov_step(Ctx* c, int field, const double* Q, long long ldq, int it, int k, double beta, double* w,
+                          long long n, double* beta_new) {
+  const int nb = kry_blocks(n), np = field == CPLX ? 2 : 1;
+  double* part = (double*)ws_get(c, WS_KRYLOV_RED, sizeof(double) * ((size_t)np * std::max(k, 1) + 1) * nb);
+  double* part2 = part + nb;
+  double* hp = c->host_parts;   // [nb] |w|^2, then alpha
+  double* dst = k == 0 ? hp : part2;
+  const double* q = Q + (long long)it * ldq;
+  const double* qp = it > 0 ? q - ldq : nullptr;
+  {
+    // bytes: alpha reads q and w; the projection q, q_{k-1}, w, the basis, and
+    // writes w; the clean-up reads the basis and w and writes w
+    ProfScope ps(c, 3, 0.0, 8.0 * np * (double)n * (2 + (it > 0 ? 4 : 3) + (k > 0 ? 2 * k + 2 : 0)));
+    if (field == CPLX) {
+      kry_alpha_k<true><<<nb, KRY_T, 0, c->stream>>>(q, w, n, part);
+      kry_project_k<true><<<nb, KRY_T, 0, c->stream>>>(q, qp, beta, part, nb, Q, ldq, k, w, n, dst, hp + KRY_MAXBLK);
+      if (k > 0) kry_clean_k<true><<<nb, KRY_T, 0, c->stream>>>(Q, ldq, k, part2, nb, w, n, hp);
+    } else {
+      kry_alpha_k<false><<<nb, KRY_T, 0, c->stream>>>(q, w, n, part);
+      kry_project_k<false><<<nb, KRY_T, 0, c->stream>>>(q, qp, beta, part, nb, Q, ldq, k, w, n, dst, hp + KRY_MAXBLK);
+      if (k > 0) kry_clean_k<false><<<nb, KRY_T, 0, c->stream>>>(Q, ldq, k, part2, nb, w, n, hp);
+    }
+    DMRG_CHECK_HIP(hipGetLastError());
+  }
+  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  *beta_new = std::sqrt(std::max(sum_host(hp, nb), 0.0));
+  return hp[KRY_MAXBLK];
+}
+
 // Re <a|b> with a host round trip (used outside the hot loop)
 double vec_dot_real(Ctx* c, int field, const double* a, const double* b, long long n) {
   double* out = (double*)ws_get(c, WS_KRYLOV_COEF, sizeof(double) * 4);
@@ -258,16 +511,9 @@ void lanczos_ground(Ctx* c, const HeffOp& h, double* x, int maxiter, double tol,
   const long long ldq = ntot;
   double* Q = (double*)ws_get(c, WS_KRYLOV_Q, sizeof(double) * (size_t)ldq * m);
   double* w = (double*)ws_get(c, WS_KRYLOV_W, sizeof(double) * ntot);
-  // coefficient scratch: [0..2m) reorth coefficients, then scalars
-  double* coef = (double*)ws_get(c, WS_KRYLOV_COEF, sizeof(double) * (4 * (size_t)m + 16));
-  double* scal = coef + 4 * (size_t)m;  // scal[0] beta_prev, scal[1] alpha(re), scal[2] alpha(im), scal[4] |w|^2
-  double* hs = c->host_scalars;
+  double* coef = (double*)ws_get(c, WS_KRYLOV_COEF, sizeof(double) * 2 * (size_t)m);
 
-  // beta0 = |x|
-  vec_dot_block(c, field, x, 0, 1, x, n, scal + 4);
-  DMRG_CHECK_HIP(hipMemcpyAsync(hs, scal + 4, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  double beta0 = std::sqrt(std::max(hs[0], 0.0));
+  double beta0 = krylov_norm(c, field, x, n);
   if (beta0 == 0.0) {
     // zero start vector: seeded Gaussian restart (dmrg.py:102-105)
     std::mt19937_64 gen(0);
@@ -284,18 +530,9 @@ void lanczos_ground(Ctx* c, const HeffOp& h, double* x, int maxiter, double tol,
 
   std::vector<double> al, be;
   // first step
+  double beta = 0.0;
   heff_apply(c, h, Q, w);
-  vec_dot_block(c, field, Q, 0, 1, w, n, scal + 1);  // alpha (re, im)
-  if (field == CPLX) {
-    // only the real part of alpha enters (dmrg.py:109): zero the imaginary
-    DMRG_CHECK_HIP(hipMemsetAsync(scal + 2, 0, sizeof(double), c->stream));
-  }
-  vec_sub_block(c, field, Q, ldq, 1, scal + 1, w, n);
-  vec_dot_block(c, field, w, 0, 1, w, n, scal + 4);
-  DMRG_CHECK_HIP(hipMemcpyAsync(hs, scal, sizeof(double) * 5, hipMemcpyDeviceToHost, c->stream));
-  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  al.push_back(hs[1]);
-  double beta = std::sqrt(std::max(hs[4], 0.0));
+  al.push_back(krylov_step(c, field, Q, ldq, 0, 0, 0.0, w, n, &beta));
   double prev = al[0];
   int k = 1;
   for (int it = 1; it < m; ++it) {
@@ -304,27 +541,8 @@ void lanczos_ground(Ctx* c, const HeffOp& h, double* x, int maxiter, double tol,
     double* q = Q + (long long)it * ldq;
     scale_copy(c, w, q, 1.0 / beta, ntot);
     heff_apply(c, h, q, w);
-    // alpha; then w -= alpha q + beta q_prev  (coefficient pair [beta, alpha])
-    vec_dot_block(c, field, q, 0, 1, w, n, scal + 1);
-    if (field == CPLX) DMRG_CHECK_HIP(hipMemsetAsync(scal + 2, 0, sizeof(double), c->stream));
-    hs[0] = beta;
-    DMRG_CHECK_HIP(hipMemcpyAsync(scal, hs, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    {
-      // coefficient layout for sub_block with k=2 over (q_prev, q): re [beta, alpha], im [0, 0]
-      double* pair = coef + 4 * (size_t)m - 4;  // 4 doubles of scratch at the end of the coef block
-      DMRG_CHECK_HIP(hipMemcpyAsync(pair, scal, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      DMRG_CHECK_HIP(hipMemcpyAsync(pair + 1, scal + 1, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      DMRG_CHECK_HIP(hipMemsetAsync(pair + 2, 0, 2 * sizeof(double), c->stream));
-      vec_sub_block(c, field, Q + (long long)(it - 1) * ldq, ldq, 2, pair, w, n);
-    }
     // full re-orthogonalisation against q_0..q_{it-1} (dmrg.py:128-129)
-    vec_dot_block(c, field, Q, ldq, it, w, n, coef);
-    vec_sub_block(c, field, Q, ldq, it, coef, w, n);
-    vec_dot_block(c, field, w, 0, 1, w, n, scal + 4);
-    DMRG_CHECK_HIP(hipMemcpyAsync(hs + 8, scal, sizeof(double) * 5, hipMemcpyDeviceToHost, c->stream));
-    DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
-    al.push_back(hs[8 + 1]);
-    beta = std::sqrt(std::max(hs[8 + 4], 0.0));
+    al.push_back(krylov_step(c, field, Q, ldq, it, it, beta, w, n, &beta));
     k = it + 1;
     const double cur = lowest_tridiag(al, be);
     if (std::fabs(cur - prev) < tol * std::max(1.0, std::fabs(cur))) break;
@@ -376,14 +594,9 @@ void krylov_expm(Ctx* c, const HeffOp& h, double* x, std::complex<double> coeff,
   const long long ldq = ntot;
   double* Q = (double*)ws_get(c, WS_KRYLOV_Q, sizeof(double) * (size_t)ldq * m);
   double* w = (double*)ws_get(c, WS_KRYLOV_W, sizeof(double) * ntot);
-  double* coef = (double*)ws_get(c, WS_KRYLOV_COEF, sizeof(double) * (4 * (size_t)m + 16));
-  double* scal = coef + 4 * (size_t)m;
-  double* hs = c->host_scalars;
+  double* coef = (double*)ws_get(c, WS_KRYLOV_COEF, sizeof(double) * 2 * (size_t)m);
 
-  vec_dot_block(c, field, x, 0, 1, x, n, scal + 4);
-  DMRG_CHECK_HIP(hipMemcpyAsync(hs, scal + 4, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  const double beta0 = std::sqrt(std::max(hs[0], 0.0));
+  const double beta0 = krylov_norm(c, field, x, n);
   if (beta0 == 0.0) {
     if (iters) *iters = 0;
     return;
@@ -392,29 +605,9 @@ void krylov_expm(Ctx* c, const HeffOp& h, double* x, std::complex<double> coeff,
   std::vector<double> al, be;
   double beta = 0.0;
   for (int it = 0; it < m; ++it) {
-    double* q = Q + (long long)it * ldq;
-    heff_apply(c, h, q, w);
-    vec_dot_block(c, field, q, 0, 1, w, n, scal + 1);
-    if (field == CPLX) DMRG_CHECK_HIP(hipMemsetAsync(scal + 2, 0, sizeof(double), c->stream));
-    hs[0] = beta;
-    DMRG_CHECK_HIP(hipMemcpyAsync(scal, hs, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    double* pair = coef + 4 * (size_t)m - 4;
-    if (it > 0) {
-      DMRG_CHECK_HIP(hipMemcpyAsync(pair, scal, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      DMRG_CHECK_HIP(hipMemcpyAsync(pair + 1, scal + 1, sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-      DMRG_CHECK_HIP(hipMemsetAsync(pair + 2, 0, 2 * sizeof(double), c->stream));
-      vec_sub_block(c, field, Q + (long long)(it - 1) * ldq, ldq, 2, pair, w, n);
-    } else {
-      vec_sub_block(c, field, q, ldq, 1, scal + 1, w, n);
-    }
+    heff_apply(c, h, Q + (long long)it * ldq, w);
     // w -= Q_k (Q_k^dag w) over every basis vector so far (tdvp.py:138-139)
-    vec_dot_block(c, field, Q, ldq, it + 1, w, n, coef);
-    vec_sub_block(c, field, Q, ldq, it + 1, coef, w, n);
-    vec_dot_block(c, field, w, 0, 1, w, n, scal + 4);
-    DMRG_CHECK_HIP(hipMemcpyAsync(hs + 8, scal, sizeof(double) * 5, hipMemcpyDeviceToHost, c->stream));
-    DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
-    al.push_back(hs[8 + 1]);
-    beta = std::sqrt(std::max(hs[8 + 4], 0.0));
+    al.push_back(krylov_step(c, field, Q, ldq, it, it + 1, beta, w, n, &beta));
     // first column of exp(coeff T_k)
     const int k = it + 1;
     const std::vector<std::complex<double>> col = tridiag_expm_col0(al, be, coeff);
