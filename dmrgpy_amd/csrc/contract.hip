@@ -208,12 +208,46 @@ void to_prec_pitched(Ctx* c, int prec, const double* src, void* dst, long long r
   DMRG_CHECK_HIP(hipGetLastError());
 }
 
-// Uploads a small operator (W rows padded to a multiple of OCH_PAD), its
-// offset tables and, for a real W, its compressed rows into a workspace slot;
-// returns device pointers.
+// Small operators reach the device as arguments of a copy kernel: the call
+// neither waits for the stream nor keeps host memory alive, and the host runs
+// ahead of the GPU (a staged copy followed by a stream synchronisation made
+// up about a third of a small apply: S=1/2 D=64, 48 us per call in all).
+// The largest bulk operators of the supported chains take 2.6 KB; anything
+// beyond the largest blob takes the staged copy.
+template <int BYTES>
+struct OpBlob {
+  unsigned v[BYTES / 4];
+};
+
+template <int BYTES>
+__global__ __launch_bounds__(256) void put_blob_k(OpBlob<BYTES> blob, unsigned* __restrict__ dst, int words) {
+#pragma unroll
+  for (int u = 0; u < BYTES / 1024; ++u) {
+    const int i = u * 256 + threadIdx.x;
+    if (i < words) dst[i] = blob.v[i];
+  }
+}
+
+template <int BYTES>
+static bool put_blob(Ctx* c, const unsigned char* src, size_t bytes, void* dst) {
+  if (bytes > BYTES) return false;
+  OpBlob<BYTES> blob;
+  std::memcpy(blob.v, src, bytes);
+  put_blob_k<BYTES><<<1, 256, 0, c->stream>>>(blob, (unsigned*)dst, (int)((bytes + 3) / 4));
+  DMRG_CHECK_HIP(hipGetLastError());
+  return true;
+}
+
+// Uploads a small operator and its offset tables into a workspace slot and
+// returns device pointers: for a sparse real W its compressed rows (all that
+// run_smallop then reads), otherwise W itself, rows padded to a multiple of
+// OCH_PAD.
 SmallOp upload_smallop(Ctx* c, Slot slot, int prec, const std::vector<double>& wre,
                        const std::vector<double>& wim, bool wcplx, int Kin, int Kout,
                        const std::vector<int>& ioff, const std::vector<int>& ooff) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  DMRG_CHECK_HIP(hipStreamIsCapturing(c->stream, &cap));
+  DMRG_REQUIRE(cap == hipStreamCaptureStatusNone, "operator upload: the stream is being captured");
   SmallOp s;
   s.Kin = Kin;
   s.Kout = Kout;
@@ -228,21 +262,24 @@ SmallOp upload_smallop(Ctx* c, Slot slot, int prec, const std::vector<double>& w
   s.nnz = (int)col.size();
   int grp[5];
   wave_groups(rowptr, Kout, grp);
-  const size_t nw = (size_t)s.KoutPad * Kin * (wcplx ? 2 : 1);
+  const bool sparse = smallop_sparse_ok(s);
+  const size_t nw = sparse ? 0 : (size_t)s.KoutPad * Kin * (wcplx ? 2 : 1);
   const size_t bytes_w = up(nw * es);
-  const size_t bytes_o = up(sizeof(int) * (Kin + Kout + Kout + 1 + 5 + col.size()));
-  const size_t bytes = bytes_w + bytes_o + up(val.size() * es) + 256;
-  std::vector<unsigned char> host(bytes, 0);
-  for (int pl = 0; pl < (wcplx ? 2 : 1); ++pl) {
-    const std::vector<double>& src = pl ? wim : wre;
-    for (int o = 0; o < Kout; ++o)
-      for (int i = 0; i < Kin; ++i) {
-        size_t idx = (size_t)pl * s.KoutPad * Kin + (size_t)o * Kin + i;
-        double v = src[(size_t)o * Kin + i];
-        if (prec == P64) reinterpret_cast<double*>(host.data())[idx] = v;
-        else reinterpret_cast<float*>(host.data())[idx] = (float)v;
-      }
-  }
+  const size_t nint = (size_t)Kin + Kout + Kout + 1 + 5 + col.size();
+  const size_t bytes_o = (sizeof(int) * nint + 15) / 16 * 16;
+  const size_t bytes = bytes_w + bytes_o + val.size() * es;
+  std::vector<unsigned char> host(bytes + 16, 0);
+  if (!sparse)
+    for (int pl = 0; pl < (wcplx ? 2 : 1); ++pl) {
+      const std::vector<double>& src = pl ? wim : wre;
+      for (int o = 0; o < Kout; ++o)
+        for (int i = 0; i < Kin; ++i) {
+          size_t idx = (size_t)pl * s.KoutPad * Kin + (size_t)o * Kin + i;
+          double v = src[(size_t)o * Kin + i];
+          if (prec == P64) reinterpret_cast<double*>(host.data())[idx] = v;
+          else reinterpret_cast<float*>(host.data())[idx] = (float)v;
+        }
+    }
   int* ints = reinterpret_cast<int*>(host.data() + bytes_w);
   std::memcpy(ints, ioff.data(), sizeof(int) * Kin);
   std::memcpy(ints + Kin, ooff.data(), sizeof(int) * Kout);
@@ -254,12 +291,14 @@ SmallOp upload_smallop(Ctx* c, Slot slot, int prec, const std::vector<double>& w
     if (prec == P64) reinterpret_cast<double*>(vb)[k] = val[k];
     else reinterpret_cast<float*>(vb)[k] = (float)val[k];
   }
-  unsigned char* dev = (unsigned char*)ws_get(c, slot, bytes);
-  DMRG_CHECK_HIP(hipMemcpyAsync(dev, host.data(), bytes, hipMemcpyHostToDevice, c->stream));
-  // the host vector dies at return: make the copy complete first
-  DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  unsigned char* dev = (unsigned char*)ws_get(c, slot, bytes + 16);
+  if (!put_blob<1024>(c, host.data(), bytes, dev) && !put_blob<3072>(c, host.data(), bytes, dev)) {
+    DMRG_CHECK_HIP(hipMemcpyAsync(dev, host.data(), bytes, hipMemcpyHostToDevice, c->stream));
+    // the host vector dies at return: make the copy complete first
+    DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  }
   const int* di = reinterpret_cast<const int*>(dev + bytes_w);
-  s.W = dev;
+  s.W = sparse ? nullptr : dev;
   s.ioff = di;
   s.ooff = di + Kin;
   s.rowptr = di + Kin + Kout;
