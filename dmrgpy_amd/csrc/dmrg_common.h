@@ -70,7 +70,7 @@ enum Slot {
   WS_SVD_GRAM, WS_SVD_EV, WS_SVD_TMP, WS_SVD_TMP2, WS_SVD_INFO, WS_SVD_CPLX, WS_SVD_FIX, WS_SVD_RED, WS_PROJ, WS_B3_L, WS_B3_R,
   WS_BF16_A, WS_BF16_B, WS_REFINE,
   WS_GSV_Q, WS_GSV_B, WS_GSV_R, WS_GSV_S, WS_GSV_V, WS_GSV_T, WS_GSV_T2, WS_GSV_OU, WS_GSV_OV,
-  WS_TRD, WS_TRD_Z, WS_TRD_ZC, WS_BT_V, WS_BT_W, WS_TRD_ZS, WS_TRD_X, WS_TRD_R,
+  WS_TRD, WS_TRD_Z, WS_TRD_ZC, WS_BT_V, WS_BT_W, WS_TRD_ZS, WS_TRD_X, WS_TRD_R, WS_TRD_DC,
   WS_NSLOTS
 };
 
@@ -106,6 +106,7 @@ struct Ctx {
   // with rocSOLVER ormtr / unmtr for the back-transformation; 0 = rocSOLVER
   // syevd / heevd
   int eig_mode = 1;
+  int dc_n = 0;   // order of the tridiagonal whose divide and conquer the workspace holds
   hipEvent_t trd_ev[2] = {nullptr, nullptr};   // early-stop checks of the reduction in flight
   // allocation-free calls (dmrg_heff_apply_noalloc): while `noalloc` is set,
   // ws_get carves the workspace out of this device's static scratch array

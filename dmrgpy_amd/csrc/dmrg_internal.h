@@ -81,6 +81,12 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
 bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double* e, double* tau, double stop_tol,
                   double total2, int* done, double* dropped);
 int trd_resident_max(int field);   // largest order it takes
+// Divide and conquer on a real symmetric tridiagonal matrix (tridiag_dc.hip):
+// eigenvalues ascending into w (w may be d), then the rows of Zt (keep x n,
+// pitch ldz) as the eigenvectors of the `keep` largest ones, ascending
+bool tridiag_dc_ok(int n);
+void tridiag_dc_values(Ctx* c, int n, const double* d, const double* e, double* w);
+void tridiag_dc_vectors(Ctx* c, int n, const double* e, int keep, double* Zt, int ldz);
 // rows of Zt (keep x n, row-major: eigenvectors of the tridiagonal) <- rows
 // of Q Y for the first nrefl reflectors sytrd_lower left in A (all n - 1 by
 // default; dormtr L/lower/N by blocked compact-WY GEMMs)

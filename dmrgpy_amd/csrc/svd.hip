@@ -188,6 +188,14 @@ __global__ void scaled_copy_k(const double* __restrict__ x, long long n, const d
   for (; i < n; i += (long long)gridDim.x * 256) y[i] = f * x[i];
 }
 
+// X[r][c] = 0 for c >= m (rows x cols, pitch cols)
+__global__ void zero_tail_k(double* __restrict__ X, int rows, int m, int cols) {
+  const int w = cols - m;
+  const long long tot = (long long)rows * w;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < tot; i += (long long)gridDim.x * 256)
+    X[(i / w) * cols + m + i % w] = 0.0;
+}
+
 static unsigned g1(long long n) {
   long long b = (n + 255) / 256;
   if (b > 4096) b = 4096;
@@ -399,6 +407,21 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
   double *trd_Z = nullptr, *trd_tau = nullptr, *trd_refl = nullptr, *trd_Zs = nullptr;
   int trd_nrefl = g - 1, trd_m = g;   // reflectors computed, order of the tridiagonal solved
   double trd_dropped = 0.0;             // trace of the block a stopped reduction took as zero
+  bool own_dc = false;                  // tridiagonal problem solved by tridiag_dc (else rocSOLVER)
+  // eigenpairs of the reduced tridiagonal (d in ev, e in ework): the
+  // library's divide and conquer, whose vectors follow once keep is known;
+  // rocSOLVER's past the orders it takes
+  auto solve_tridiagonal = [&]() {
+    own_dc = tridiag_dc_ok(trd_m);
+    if (own_dc) {
+      tridiag_dc_values(c, trd_m, ev, ework, ev);
+    } else if (trd_m < g) {
+      trd_Zs = (double*)ws_get(c, WS_TRD_ZS, sizeof(double) * (size_t)trd_m * trd_m);
+      check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, trd_m, ev, ework, trd_Zs, trd_m, info), "dstedc");
+    } else {
+      check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, g, ev, ework, trd_Z, g, info), "dstedc");
+    }
+  };
   {
     ProfScope ps(c, 2, (cx ? 8.0 : 2.0) * (double)g * g * (left ? n : m));
     double* Gplanar = (double*)ws_get(c, WS_SVD_TMP2, sizeof(double) * es * (size_t)g * g);
@@ -427,13 +450,7 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
       trd_nrefl = hetrd_lower(c, Gplanar, g, ev, ework, trd_tau, c->eig_mode == 1 ? TRD_STOP_TOL : 0.0,
                               &trd_dropped);
       trd_m = trd_nrefl < g - 1 ? trd_nrefl + 1 : g;
-      if (trd_m < g) {
-        trd_Zs = (double*)ws_get(c, WS_TRD_ZS, sizeof(double) * (size_t)trd_m * trd_m);
-        check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, trd_m, ev, ework, trd_Zs, trd_m, info),
-                 "dstedc");
-      } else {
-        check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, g, ev, ework, trd_Z, g, info), "dstedc");
-      }
+      solve_tridiagonal();
       trd_refl = Gplanar;
     } else if (cx) {
       double* Gi = (double*)ws_get(c, WS_SVD_CPLX, sizeof(double) * 2 * (size_t)g * g);
@@ -455,13 +472,7 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
       trd_nrefl = sytrd_lower(c, Gplanar, g, ev, ework, trd_tau, c->eig_mode == 1 ? TRD_STOP_TOL : 0.0,
                               &trd_dropped);
       trd_m = trd_nrefl < g - 1 ? trd_nrefl + 1 : g;
-      if (trd_m < g) {
-        trd_Zs = (double*)ws_get(c, WS_TRD_ZS, sizeof(double) * (size_t)trd_m * trd_m);
-        check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, trd_m, ev, ework, trd_Zs, trd_m, info),
-                 "dstedc");
-      } else {
-        check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, g, ev, ework, trd_Z, g, info), "dstedc");
-      }
+      solve_tridiagonal();
       Gsolve = trd_Z;
       trd_refl = Gplanar;
     } else {
@@ -477,7 +488,7 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
   // below the trd_m computed values
   DMRG_CHECK_HIP(hipMemcpyAsync(evh.data() + (g - trd_m), ev, sizeof(double) * trd_m, hipMemcpyDeviceToHost,
                                 c->stream));
-  DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  if (!own_dc) DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipMemcpyAsync(&hmax, amax_dev, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
   DMRG_REQUIRE(hinfo == 0, "syevd/heevd did not converge");
@@ -497,7 +508,13 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
     // last keep eigenvector columns of the tridiagonal
     ProfScope ps(c, 2, 2.0 * (double)g * trd_nrefl * keep);
     double* Zt = trd_Z + (size_t)(g - keep) * g;
-    if (trd_m < g) {   // the kept eigenvectors of the leading block, zero beyond it
+    if (own_dc) {
+      tridiag_dc_vectors(c, trd_m, ework, keep, Zt, g);
+      if (trd_m < g) {   // zero beyond the leading block
+        zero_tail_k<<<g1((long long)keep * (g - trd_m)), 256, 0, c->stream>>>(Zt, keep, trd_m, g);
+        DMRG_CHECK_HIP(hipGetLastError());
+      }
+    } else if (trd_m < g) {   // the kept eigenvectors of the leading block, zero beyond it
       const long long tot = (long long)keep * g;
       embed_rows_k<<<g1(tot), 256, 0, c->stream>>>(trd_Zs + (size_t)(trd_m - keep) * trd_m, trd_m, keep, g, Zt);
       DMRG_CHECK_HIP(hipGetLastError());
@@ -517,7 +534,13 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
     const long long kg = (long long)keep * g;
     if (c->eig_mode != 2) {   // own blocked product on planar rows
       double* Et = (double*)ws_get(c, WS_SVD_CPLX, sizeof(double) * 2 * (size_t)kg);
-      if (trd_m < g) {   // the kept eigenvectors of the leading block, zero beyond it
+      if (own_dc) {
+        tridiag_dc_vectors(c, trd_m, ework, keep, Et, g);
+        if (trd_m < g) {   // zero beyond the leading block
+          zero_tail_k<<<g1((long long)keep * (g - trd_m)), 256, 0, c->stream>>>(Et, keep, trd_m, g);
+          DMRG_CHECK_HIP(hipGetLastError());
+        }
+      } else if (trd_m < g) {   // the kept eigenvectors of the leading block, zero beyond it
         embed_rows_k<<<g1(kg), 256, 0, c->stream>>>(trd_Zs + (size_t)(trd_m - keep) * trd_m, trd_m, keep, g, Et);
         DMRG_CHECK_HIP(hipGetLastError());
       } else {
@@ -530,6 +553,7 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
       DMRG_CHECK_HIP(hipGetLastError());
     } else {   // rocSOLVER zunmtr on interleaved reflectors
       double* Gi = (double*)ws_get(c, WS_SVD_CPLX, sizeof(double) * 2 * (size_t)g * g);
+      if (own_dc) tridiag_dc_vectors(c, trd_m, ework, keep, trd_Z + (size_t)(g - keep) * g, g);
       real_to_inter_k<<<g1(kg), 256, 0, c->stream>>>(trd_Z + (size_t)(g - keep) * g, kg, Zk);
       DMRG_CHECK_HIP(hipGetLastError());
       planar_to_inter_k<<<g1((long long)g * g), 256, 0, c->stream>>>(trd_refl, (long long)g * g, Gi);
@@ -921,9 +945,16 @@ int sym_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
   double* ework = (double*)ws_get(c, WS_SVD_EV, sizeof(double) * ((size_t)2 * n + 16));
   double* tauv = ework + n;
   rocblas_int* info = (rocblas_int*)ws_get(c, WS_SVD_INFO, 64);
+  bool own_dc = false;
   if (mode >= 1) {   // every eigenvector is wanted: always the full reduction
     sytrd_lower(c, A, n, w, ework, tauv);
-    check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, n, w, ework, Z, n, info), "dstedc");
+    own_dc = tridiag_dc_ok(n);
+    if (own_dc) {
+      tridiag_dc_values(c, n, w, ework, w);
+      tridiag_dc_vectors(c, n, ework, n, Z, n);
+    } else {
+      check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, n, w, ework, Z, n, info), "dstedc");
+    }
     if (mode != 2)
       ormtr_lower_rows(c, A, n, tauv, Z, n);
     else
@@ -936,7 +967,7 @@ int sym_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
     DMRG_CHECK_HIP(hipMemcpyAsync(Z, A, sizeof(double) * n * n, hipMemcpyDeviceToDevice, c->stream));
   }
   int hinfo = 0;
-  DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  if (!own_dc) DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
   DMRG_REQUIRE(hinfo == 0, "sym_eig: eigensolver did not converge");
   return 0;
@@ -956,10 +987,17 @@ int herm_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
   rocblas_int* info = (rocblas_int*)ws_get(c, WS_SVD_INFO, 64);
   double* Zc = (double*)ws_get(c, WS_TRD_ZC, sizeof(double) * 2 * (size_t)nn);
   double* Ai = (double*)ws_get(c, WS_SVD_CPLX, sizeof(double) * 2 * (size_t)nn);
+  bool own_dc = false;
   if (mode >= 1) {
     double* Zr = (double*)ws_get(c, WS_TRD_Z, sizeof(double) * (size_t)nn);
     hetrd_lower(c, A, n, w, ework, tauv);
-    check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, n, w, ework, Zr, n, info), "dstedc");
+    own_dc = tridiag_dc_ok(n);
+    if (own_dc) {
+      tridiag_dc_values(c, n, w, ework, w);
+      tridiag_dc_vectors(c, n, ework, n, Zr, n);
+    } else {
+      check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, n, w, ework, Zr, n, info), "dstedc");
+    }
     if (mode != 2) {   // Ai holds the planar rows of Q Y
       DMRG_CHECK_HIP(hipMemcpyAsync(Ai, Zr, sizeof(double) * nn, hipMemcpyDeviceToDevice, c->stream));
       DMRG_CHECK_HIP(hipMemsetAsync(Ai + nn, 0, sizeof(double) * nn, c->stream));
@@ -986,7 +1024,7 @@ int herm_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
   inter_to_planar_conj_k<<<g1(nn), 256, 0, c->stream>>>(Zc, nn, Z);
   DMRG_CHECK_HIP(hipGetLastError());
   int hinfo = 0;
-  DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  if (!own_dc) DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
   DMRG_REQUIRE(hinfo == 0, "herm_eig: eigensolver did not converge");
   return 0;
