@@ -28,9 +28,9 @@
 // launch-per-column reduction instead.
 //
 // Measured per column, launch-per-column / resident (us): real order 128
-// 8.7 / 2.5, 380 9.8 / 3.2, 2588 (900 columns reduced) 16.2 / 8.4; complex
-// order 1200 14.5 / 6.6.  What bounds a column is the exchange (two thirds of
-// it at 216 workgroups), then the chain of two workgroup-wide reductions.
+// 8.7 / 2.8, 380 9.8 / 2.9, 2588 (930 columns reduced) 16.2 / 6.3; complex
+// order 1200 14.5 / 5.7.  What bounds a column is the exchange (half of it at
+// 216 workgroups), then the chain of two workgroup-wide reductions.
 #include "dmrg_internal.h"
 #include "wave_reduce.h"
 
@@ -54,7 +54,7 @@ struct ResArgs {
   double* R;                   // reflectors: row J, columns J+2 ... (m x m, planes m*m apart)
   double *d, *e, *tau;         // at col0 (tau interleaved when complex)
   int early;
-  double tol2, total2;         // stop when |trailing|_F^2 <= tol2 * total2 (total2 < 0: of this matrix)
+  double tol2, total2;         // stop once |trailing|_F^2 <= tol2 * total2 (total2 < 0: of this matrix)
   int* status;                 // [0] 1 = gave up, [1] columns reduced
   double* trace;               // trace of the block left when stopped early
 };
@@ -68,28 +68,18 @@ __device__ __forceinline__ unsigned long long peek(const unsigned long long* p) 
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// N words p[idx[i]] once they are all published; false after RES_LIMIT ticks
-template <int N>
-__device__ __forceinline__ bool await(const unsigned long long* p, const int (&idx)[N], double (&out)[N]) {
-  unsigned long long u[N];
+// Words published by other workgroups, loaded in batches until all of a batch
+// are there; false after RES_LIMIT ticks
+struct Patience {
+  int spin = 0;
   long long t0 = 0;
-  for (int spin = 0;; ++spin) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) u[i] = peek(p + idx[i]);
-    bool miss = false;
-#pragma unroll
-    for (int i = 0; i < N; ++i) miss |= u[i] == RES_EMPTY;
-    if (!miss) break;
-    if ((spin & 63) == 63) {
-      const long long t = wall_clock64();
-      if (t0 == 0) t0 = t;
-      else if (t - t0 > RES_LIMIT) return false;
-    }
+  __device__ __forceinline__ bool over() {
+    if ((++spin & 63) != 0) return false;
+    const long long t = wall_clock64();
+    if (t0 == 0) t0 = t;
+    return t - t0 > RES_LIMIT;
   }
-#pragma unroll
-  for (int i = 0; i < N; ++i) out[i] = as_d(u[i]);
-  return true;
-}
+};
 
 // T threads, thread t holds columns t, t + T, ... (CC of them) of RW rows.
 // At most 15 reduced values beside the norm (RW real, 2 RW complex).
@@ -127,6 +117,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
     for (int p = 0; p < NP; ++p) v[p][k] = w[p][k] = 0.0;
   }
   double total2 = g.total2;
+  bool passed = false;   // the last early-stop check
   double tr = 0.0, ti = 0.0, Kr = 0.0, Ki = 0.0, scr = 0.0, sci = 0.0;   // tau, w = tau q + K v, v = scale a
 
   for (int J = 0;; ++J) {
@@ -258,11 +249,19 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       __syncthreads();
       double f2 = 0.0, tc = 0.0;
       for (int o = J / RW + tid; o < G; o += T) {   // the workgroups that hold rows from J on
-        const int idx[2] = {o, G + o};
-        double y[2] = {0.0, 0.0};
-        if (!await<2>(ck, idx, y)) s_bad = 1;
-        f2 += y[0];
-        tc += y[1];
+        unsigned long long y0, y1;
+        Patience wait;
+        for (;;) {
+          y0 = peek(ck + o);
+          y1 = peek(ck + G + o);
+          if (y0 != RES_EMPTY && y1 != RES_EMPTY) break;
+          if (wait.over()) {
+            s_bad = 1;
+            break;
+          }
+        }
+        f2 += as_d(y0);
+        tc += as_d(y1);
       }
       const double ss = wave_sums2(f2, tc);
       if (lane == 0) red2[wave * 2] = ss;
@@ -282,12 +281,14 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       }
       if (first) {
         total2 = f2;
-      } else if (f2 <= g.tol2 * total2) {
+      } else if (passed) {   // one check after the first to pass, as the panel path stops
         if (writer && tid == 0) {
           g.status[1] = J;
           g.trace[0] = tc;
         }
         return;
+      } else {
+        passed = f2 <= g.tol2 * total2;
       }
     }
     // ---- reflector of column J (every workgroup, the same sums in the same order)
@@ -300,12 +301,12 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
     const double a0r = s_a0[0], a0i = CX ? s_a0[NP - 1] : 0.0;
     double beta;
     if (!CX) {
-      const double xn = sqrt(xn2);
       tr = 0.0;
       beta = a0r;
       scr = 0.0;
-      if (xn != 0.0) {
-        beta = -copysign(hypot(a0r, xn), a0r);
+      if (xn2 != 0.0) {
+        const double h2 = a0r * a0r + xn2;
+        beta = -copysign(h2 > 1e-280 && h2 < 1e280 ? sqrt(h2) : hypot(a0r, sqrt(xn2)), a0r);
         tr = (beta - a0r) / beta;
         scr = 1.0 / (a0r - beta);
       }
@@ -317,7 +318,8 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       beta = -a0r;
       scr = sci = 0.0;
       if (xn2 != 0.0 || a0i != 0.0) {
-        beta = -copysign(hypot(hypot(a0r, a0i), sqrt(xn2)), a0r);
+        const double h2 = a0r * a0r + a0i * a0i + xn2;
+        beta = -copysign(h2 > 1e-280 && h2 < 1e280 ? sqrt(h2) : hypot(hypot(a0r, a0i), sqrt(xn2)), a0r);
         tr = (beta - a0r) / beta;
         ti = -a0i / beta;
         const double dr = a0r - beta, di = a0i, den = dr * dr + di * di;
@@ -363,6 +365,8 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       }
     }
     // ---- everybody's q, and row J+1
+    // (row J+1 was published well before: its words are loaded once, with the
+    // first try for q, and looked at last -- one round trip for both)
     double cv[NP][CC], qv[NP][CC], q1[NP];
     {
       int idx[CC];
@@ -371,17 +375,51 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
         const int c = tid + T * k;
         idx[k] = c > J && c < m ? c : J + 1;
       }
-      const int one[1] = {J + 1};
-      bool ok = true;
+      unsigned long long uc[NP][CC], uq[NP][CC], u1[NP];
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int k = 0; k < CC; ++k) uc[p][k] = peek(Xc + p * mp + idx[k]);
+      Patience wait;
+      bool ok = true, miss;
+      do {
+        miss = false;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          u1[p] = peek(Xq + p * mp + J + 1);
+#pragma unroll
+          for (int k = 0; k < CC; ++k) uq[p][k] = peek(Xq + p * mp + idx[k]);
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          miss |= u1[p] == RES_EMPTY;
+#pragma unroll
+          for (int k = 0; k < CC; ++k) miss |= uq[p][k] == RES_EMPTY;
+        }
+        if (miss && wait.over()) ok = false;
+      } while (miss && ok);
+      do {
+        miss = false;
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+          for (int k = 0; k < CC; ++k)
+            if (uc[p][k] == RES_EMPTY) {
+              miss = true;
+              uc[p][k] = peek(Xc + p * mp + idx[k]);
+            }
+        if (miss && wait.over()) ok = false;
+      } while (miss && ok);
+      if (!ok) s_bad = 1;
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
-        double y1[1] = {0.0};
-        ok = ok && await<CC>(Xq + p * mp, idx, qv[p]);
-        ok = ok && await<1>(Xq + p * mp, one, y1);
-        ok = ok && await<CC>(Xc + p * mp, idx, cv[p]);
-        q1[p] = y1[0];
+        q1[p] = as_d(u1[p]);
+#pragma unroll
+        for (int k = 0; k < CC; ++k) {
+          qv[p][k] = as_d(uq[p][k]);
+          cv[p][k] = as_d(uc[p][k]);
+        }
       }
-      if (!ok) s_bad = 1;
     }
     // q^H v (conj(q) v summed over the rows past J)
     double sr = 0.0, si = 0.0;
