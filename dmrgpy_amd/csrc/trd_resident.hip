@@ -12,10 +12,16 @@
 // (free of memory traffic too) needs no panel.  Per column J, every
 // workgroup redundantly holds the column a = A[:, J] spread over its threads:
 //
-//   v, tau, beta from a and |a|;  q = A v for its own rows;  publish q;
-//   read all of q and row J+1 of A (published by its owner);
-//   w = tau q - (tau^2 (q.v) / 2) v;   next column  A[:, J+1] - v w_1 - w;
-//   A -= v w^T + w v^T on its own rows, fused with the next A x.
+//   x = a[J+2:];  A x and |x|^2 for its own rows;  publish A x;
+//   tau, beta, scale from |x|, v = e_{J+1} + scale x, and the previous column's
+//   A -= v w^T + w v^T on its own rows, while the exchange is under way;
+//   read all of A x and row J+1 of A (published by its owner): q = A v;
+//   w = tau q - (tau^2 (q.v) / 2) v;   next column  A[:, J+1] - v w_1 - w.
+//
+// A x is taken with the matrix before the previous column's update and
+// corrected by v (w.x) + w (v.x), as in the blocked reduction's panels, so
+// that neither the update nor the reflector's divisions sit between one
+// exchange and the next.
 //
 // Exchange: every published word goes to its own address in a buffer that a
 // preceding kernel filled with one NaN pattern; readers poll each word
@@ -28,9 +34,10 @@
 // launch-per-column reduction instead.
 //
 // Measured per column, launch-per-column / resident (us): real order 128
-// 8.7 / 2.8, 380 9.8 / 2.9, 2588 (930 columns reduced) 16.2 / 6.3; complex
-// order 1200 14.5 / 5.7.  What bounds a column is the exchange (half of it at
-// 216 workgroups), then the chain of two workgroup-wide reductions.
+// 8.7 / 2.45, 380 9.8 / 2.6, 2588 (930 columns reduced) 16.2 / 6.0; complex
+// order 1200 14.5 / 5.6 (with the update and the reflector before the
+// publication: 2.8, 2.9, 6.3, 5.7).  What bounds a column is the exchange,
+// then the chain of two workgroup-wide reductions.
 #include "dmrg_internal.h"
 #include "wave_reduce.h"
 
@@ -82,13 +89,14 @@ struct Patience {
 };
 
 // T threads, thread t holds columns t, t + T, ... (CC of them) of RW rows.
-// At most 15 reduced values beside the norm (RW real, 2 RW complex).
 template <bool CX, int T, int CC, int RW>
 __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
-  constexpr int NP = CX ? 2 : 1, NW = T / 64, NS = NP * RW;   // NS sums + the norm at index NS
-  static_assert(NS <= 15, "reduction holds 16 values");
-  __shared__ double red[NW * 16], red2[NW * 2];
-  __shared__ double sA1[NP][16], sa[2][NP][16], sq[NP][16];
+  constexpr int NP = CX ? 2 : 1, NW = T / 64, NS = NP * RW;
+  // 16 sums per column: A x of the own rows, |x|^2 at NS and, real, w.x and v.x
+  // of the previous column after it (complex: four more, reduced apart)
+  static_assert(CX ? NS <= 15 : NS <= 13, "reduction holds 16 values");
+  __shared__ double red[NW * 16], red2[NW * 4], red4[NW * 4];
+  __shared__ double sa[2][NP][16], sq[NP][16];
   __shared__ double2 svw[NW][NP][16];   // (v, w) of the own rows, one copy per wave
   __shared__ double s_a0[NP], s_d;
   __shared__ int s_bad;
@@ -120,13 +128,58 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
   bool passed = false;   // the last early-stop check
   double tr = 0.0, ti = 0.0, Kr = 0.0, Ki = 0.0, scr = 0.0, sci = 0.0;   // tau, w = tau q + K v, v = scale a
 
+  // On entry to column J: a = column J; v, w = column J-1's, not yet applied to M.
   for (int J = 0;; ++J) {
     const int par = J & 1;
-    // ---- rank-2 update of column J-1 on the own rows, fused with A x for column J
+    unsigned long long* Xc = g.X + (long long)J * (2 * NP * mp);
+    unsigned long long* Xq = Xc + NP * mp;
+    // ---- v and w of the own rows (column J-1; rows from J on), lane i for row i
+    double ovr = 0.0, ovi = 0.0, owr = 0.0, owi = 0.0;
+    if (J > 0 && lane < RW) {
+      const int r = row0 + lane;
+      if (r >= J && r < m) {
+        const double ar = sa[par ^ 1][0][lane], ai = CX ? sa[par ^ 1][NP - 1][lane] : 0.0;
+        ovr = r == J ? 1.0 : scr * ar - sci * ai;
+        ovi = r == J ? 0.0 : scr * ai + sci * ar;
+        const double qr = sq[0][lane], qi = CX ? sq[NP - 1][lane] : 0.0;
+        owr = tr * qr - ti * qi + Kr * ovr - Ki * ovi;
+        owi = tr * qi + ti * qr + Kr * ovi + Ki * ovr;
+      }
+    }
+    if (lane < RW) {
+      svw[wave][0][lane] = double2{ovr, owr};
+      if (CX) svw[wave][NP - 1][lane] = double2{ovi, owi};
+    }
+    // ---- row J+1 for everybody (with column J-1 applied)
+    const int i1 = J + 1 - row0;
+    if (i1 >= 0 && i1 < RW && J + 1 < m) {
+      const double pvr = lane_value(ovr, i1), pwr = lane_value(owr, i1);
+      const double pvi = CX ? lane_value(ovi, i1) : 0.0, pwi = CX ? lane_value(owi, i1) : 0.0;
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+        if (i == i1) {
+#pragma unroll
+          for (int k = 0; k < CC; ++k) {
+            const int c = tid + T * k;
+            if (c > J && c < m) {
+              if (!CX) {
+                publish(Xc + c, M[0][i][k] - (pvr * w[0][k] + pwr * v[0][k]));
+              } else {
+                const double wr = w[0][k], wi = w[NP - 1][k], vr = v[0][k], vi = v[NP - 1][k];
+                publish(Xc + c, M[0][i][k] - (pvr * wr + pvi * wi + pwr * vr + pwi * vi));
+                publish(Xc + mp + c, M[NP - 1][i][k] - (pvi * wr - pvr * wi + pwi * vr - pwr * vi));
+              }
+            }
+          }
+        }
+    }
+    // ---- A x of the own rows, x = a[J+2:], with the A before column J-1:
+    // column J-1's update is taken off the sums below and applied to M later,
+    // while the exchange is under way
     double acc[16];
 #pragma unroll
     for (int t = 0; t < 16; ++t) acc[t] = 0.0;
-    double nrm = 0.0;
+    double wxr = 0.0, wxi = 0.0, vxr = 0.0, vxi = 0.0;   // w^H x, v^H x
 #pragma unroll
     for (int k = 0; k < CC; ++k) {
       const int c = tid + T * k;
@@ -142,83 +195,79 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
 #pragma unroll
       for (int p = 0; p < NP; ++p) {   // from here on only a[J+2:] is wanted
         a[p][k] = c >= J + 2 ? a[p][k] : 0.0;
-        nrm += a[p][k] * a[p][k];
+        acc[NS] += a[p][k] * a[p][k];
+        wxr += w[p][k] * a[p][k];
+        vxr += v[p][k] * a[p][k];
       }
-    }
-    if (J > 0) {
-      if (lane < RW) {   // v and w of the own rows (column J-1; rows from J on)
-        const int r = row0 + lane;
-        double vr = 0.0, vi = 0.0, wr = 0.0, wi = 0.0;
-        if (r >= J && r < m) {
-          const double ar = sa[par ^ 1][0][lane], ai = CX ? sa[par ^ 1][NP - 1][lane] : 0.0;
-          vr = r == J ? 1.0 : scr * ar - sci * ai;
-          vi = r == J ? 0.0 : scr * ai + sci * ar;
-          const double qr = sq[0][lane], qi = CX ? sq[NP - 1][lane] : 0.0;
-          wr = tr * qr - ti * qi + Kr * vr - Ki * vi;
-          wi = tr * qi + ti * qr + Kr * vi + Ki * vr;
-        }
-        svw[wave][0][lane] = double2{vr, wr};
-        if (CX) svw[wave][NP - 1][lane] = double2{vi, wi};
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
-#pragma unroll
-    for (int i = 0; i < RW; ++i) {
-      double2 pr = double2{0.0, 0.0}, pi = double2{0.0, 0.0};
-      if (J > 0) {
-        pr = svw[wave][0][i];
-        if (CX) pi = svw[wave][NP - 1][i];
+      if (CX) {
+        wxi += w[0][k] * a[NP - 1][k] - w[NP - 1][k] * a[0][k];
+        vxi += v[0][k] * a[NP - 1][k] - v[NP - 1][k] * a[0][k];
       }
 #pragma unroll
-      for (int k = 0; k < CC; ++k) {
+      for (int i = 0; i < RW; ++i) {
         if (!CX) {
-          const double t = M[0][i][k] - (pr.x * w[0][k] + pr.y * v[0][k]);
-          M[0][i][k] = t;
-          acc[i] += t * a[0][k];
-        } else {   // B -= v conj(w) + w conj(v)
-          const double wr = w[0][k], wi = w[NP - 1][k], vr = v[0][k], vi = v[NP - 1][k];
-          const double tre = M[0][i][k] - (pr.x * wr + pi.x * wi + pr.y * vr + pi.y * vi);
-          const double tim = M[NP - 1][i][k] - (pi.x * wr - pr.x * wi + pi.y * vr - pr.y * vi);
-          M[0][i][k] = tre;
-          M[NP - 1][i][k] = tim;
-          acc[i] += tre * a[0][k] - tim * a[NP - 1][k];
-          acc[RW + i] += tre * a[NP - 1][k] + tim * a[0][k];
+          acc[i] += M[0][i][k] * a[0][k];
+        } else {
+          acc[i] += M[0][i][k] * a[0][k] - M[NP - 1][i][k] * a[NP - 1][k];
+          acc[RW + i] += M[0][i][k] * a[NP - 1][k] + M[NP - 1][i][k] * a[0][k];
         }
       }
     }
-    acc[NS] = nrm;
-    // ---- row J+1 for everybody's next column; column J+1 of the own rows
-    unsigned long long* Xc = g.X + (long long)J * (2 * NP * mp);
-    unsigned long long* Xq = Xc + NP * mp;
-    const int i1 = J + 1 - row0;
-    if (i1 >= 0 && i1 < RW && J + 1 < m) {
-#pragma unroll
-      for (int i = 0; i < RW; ++i)
-        if (i == i1) {
-#pragma unroll
-          for (int k = 0; k < CC; ++k) {
-            const int c = tid + T * k;
-            if (c > J && c < m) {
-#pragma unroll
-              for (int p = 0; p < NP; ++p) publish(Xc + p * mp + c, M[p][i][k]);
-            }
-          }
-        }
+    if (!CX) {
+      acc[14] = wxr;
+      acc[15] = vxr;
+    } else {
+      wave_sums4(wxr, wxi, vxr, vxi);
+      if (lane < 4) red4[wave * 4 + lane] = lane == 0 ? wxr : (lane == 1 ? wxi : (lane == 2 ? vxr : vxi));
     }
-    const int k1 = (J + 1) / T;
-#pragma unroll
-    for (int k = 0; k < CC; ++k)
-      if (k == k1 && tid == J + 1 - T * k) {
-#pragma unroll
-        for (int i = 0; i < RW; ++i)
-#pragma unroll
-          for (int p = 0; p < NP; ++p) sA1[p][i] = M[p][i][k];
-      }
     {
       const double s = wave_sums16(acc, lane);
       if ((lane & 3) == 0) red[wave * 16 + sum_index(lane)] = s;
     }
     __syncthreads();
+    double tot = 0.0;
+    if (lane < 16) {
+#pragma unroll
+      for (int u = 0; u < NW; ++u) tot += red[u * 16 + lane];
+    }
+    if (wave == 0) {   // publish A x; q = A v = (row J+1) + scale (A x) is formed by the readers
+      double yr = tot, yi = CX ? __shfl(tot, (RW + lane) & 63) : 0.0;
+      if (!CX) {
+        yr -= ovr * lane_value(tot, 14) + owr * lane_value(tot, 15);
+      } else {
+        double t4 = 0.0;
+        if (lane < 4) {
+#pragma unroll
+          for (int u = 0; u < NW; ++u) t4 += red4[u * 4 + lane];
+        }
+        const double xr = lane_value(t4, 0), xi = lane_value(t4, 1), zr = lane_value(t4, 2), zi = lane_value(t4, 3);
+        yr -= ovr * xr - ovi * xi + owr * zr - owi * zi;
+        yi -= ovr * xi + ovi * xr + owr * zi + owi * zr;
+      }
+      const int r = row0 + lane;
+      if (lane < RW && r > J && r < m) {
+        publish(Xq + r, yr);
+        if (CX) publish(Xq + mp + r, yi);
+      }
+    }
+    // ---- column J-1's rank-2 update
+    if (J > 0) {
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const double2 pr = svw[wave][0][i];
+        const double2 pi = CX ? svw[wave][NP - 1][i] : double2{0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < CC; ++k) {
+          if (!CX) {
+            M[0][i][k] -= pr.x * w[0][k] + pr.y * v[0][k];
+          } else {   // B -= v conj(w) + w conj(v)
+            const double wr = w[0][k], wi = w[NP - 1][k], vr = v[0][k], vi = v[NP - 1][k];
+            M[0][i][k] -= pr.x * wr + pi.x * wi + pr.y * vr + pi.y * vi;
+            M[NP - 1][i][k] -= pi.x * wr - pr.x * wi + pi.y * vr - pr.y * vi;
+          }
+        }
+      }
+    }
     // ---- early stop: |A[J:, J:]|_F^2 against the whole matrix's
     const int s_abs = g.col0 + J;
     const bool first = J == 0 && g.early && total2 < 0.0;
@@ -292,11 +341,6 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       }
     }
     // ---- reflector of column J (every workgroup, the same sums in the same order)
-    double tot = 0.0;
-    if (lane < 16) {
-#pragma unroll
-      for (int u = 0; u < NW; ++u) tot += red[u * 16 + lane];
-    }
     const double xn2 = lane_value(tot, NS);
     const double a0r = s_a0[0], a0i = CX ? s_a0[NP - 1] : 0.0;
     double beta;
@@ -327,28 +371,13 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
         sci = -di / den;
       }
     }
-    // ---- q = A v for the own rows
-    if (wave == 0) {
-      const double ti_ = CX ? __shfl(tot, RW + lane) : 0.0;
-      const int r = row0 + lane;
-      if (lane < RW) {
-        const double qr = sA1[0][lane] + scr * tot - sci * ti_;
-        const double qi = CX ? sA1[NP - 1][lane] + scr * ti_ + sci * tot : 0.0;
-        if (r > J && r < m) {
-          publish(Xq + r, qr);
-          if (CX) publish(Xq + mp + r, qi);
-        }
-        sq[0][lane] = qr;
-        if (CX) sq[NP - 1][lane] = qi;
-      }
-    }
     double* Rj = g.R + (long long)J * m;
 #pragma unroll
     for (int k = 0; k < CC; ++k) {
       const int c = tid + T * k;
-      const double ar = a[0][k], ai = CX ? a[NP - 1][k] : 0.0;
-      v[0][k] = c >= J + 2 && c < m ? scr * ar - sci * ai : (c == J + 1 ? 1.0 : 0.0);
-      if (CX) v[NP - 1][k] = c >= J + 2 && c < m ? scr * ai + sci * ar : 0.0;
+      const double ar = a[0][k], ai = CX ? a[NP - 1][k] : 0.0;   // zero up to J+1 and past the order
+      v[0][k] = c == J + 1 ? 1.0 : scr * ar - sci * ai;
+      if (CX) v[NP - 1][k] = scr * ai + sci * ar;
       if (writer && c >= J + 2 && c < m) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) Rj[(long long)p * m * m + c] = v[p][k];
@@ -364,10 +393,9 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
         g.tau[J] = tr;
       }
     }
-    // ---- everybody's q, and row J+1
-    // (row J+1 was published well before: its words are loaded once, with the
-    // first try for q, and looked at last -- one round trip for both)
-    double cv[NP][CC], qv[NP][CC], q1[NP];
+    // ---- everybody's A x, and row J+1, loaded together (the row was published
+    // well before and is looked at last: one round trip for both)
+    double cv[NP][CC], qv[NP][CC], q1[NP], c1[NP];
     {
       int idx[CC];
 #pragma unroll
@@ -375,11 +403,13 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
         const int c = tid + T * k;
         idx[k] = c > J && c < m ? c : J + 1;
       }
-      unsigned long long uc[NP][CC], uq[NP][CC], u1[NP];
+      unsigned long long uc[NP][CC], uq[NP][CC], u1[NP], e1[NP];
 #pragma unroll
-      for (int p = 0; p < NP; ++p)
+      for (int p = 0; p < NP; ++p) {
+        e1[p] = peek(Xc + p * mp + J + 1);
 #pragma unroll
         for (int k = 0; k < CC; ++k) uc[p][k] = peek(Xc + p * mp + idx[k]);
+      }
       Patience wait;
       bool ok = true, miss;
       do {
@@ -401,34 +431,49 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       do {
         miss = false;
 #pragma unroll
-        for (int p = 0; p < NP; ++p)
+        for (int p = 0; p < NP; ++p) {
+          if (e1[p] == RES_EMPTY) {
+            miss = true;
+            e1[p] = peek(Xc + p * mp + J + 1);
+          }
 #pragma unroll
           for (int k = 0; k < CC; ++k)
             if (uc[p][k] == RES_EMPTY) {
               miss = true;
               uc[p][k] = peek(Xc + p * mp + idx[k]);
             }
+        }
         if (miss && wait.over()) ok = false;
       } while (miss && ok);
       if (!ok) s_bad = 1;
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
+        const double sg = p ? -1.0 : 1.0;   // column J+1 is the conjugate of row J+1
         q1[p] = as_d(u1[p]);
+        c1[p] = sg * as_d(e1[p]);
 #pragma unroll
         for (int k = 0; k < CC; ++k) {
           qv[p][k] = as_d(uq[p][k]);
-          cv[p][k] = as_d(uc[p][k]);
+          cv[p][k] = sg * as_d(uc[p][k]);
         }
       }
     }
-    // q^H v (conj(q) v summed over the rows past J)
+    // q = A v = A e_{J+1} + scale A x;  q^H v (v is zero up to J and past the order)
     double sr = 0.0, si = 0.0;
 #pragma unroll
-    for (int k = 0; k < CC; ++k) {   // v is zero up to J and past the order
+    for (int k = 0; k < CC; ++k) {
+      const double yr = qv[0][k], yi = CX ? qv[NP - 1][k] : 0.0;
+      qv[0][k] = cv[0][k] + scr * yr - sci * yi;
       sr += qv[0][k] * v[0][k];
       if (CX) {
+        qv[NP - 1][k] = cv[NP - 1][k] + scr * yi + sci * yr;
         sr += qv[NP - 1][k] * v[NP - 1][k];
         si += qv[0][k] * v[NP - 1][k] - qv[NP - 1][k] * v[0][k];
+      }
+      const int c = tid + T * k;
+      if (c >= row0 && c < row0 + RW) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) sq[p][c - row0] = qv[p][k];
       }
     }
     {
@@ -451,7 +496,8 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
     const double zr = tr * sr + ti * si, zi = tr * si - ti * sr;
     Kr = -0.5 * (tr * zr - ti * zi);
     Ki = -0.5 * (tr * zi + ti * zr);
-    const double q1r = q1[0], q1i = CX ? q1[NP - 1] : 0.0;
+    const double y1r = q1[0], y1i = CX ? q1[NP - 1] : 0.0;
+    const double q1r = c1[0] + scr * y1r - sci * y1i, q1i = CX ? c1[NP - 1] + scr * y1i + sci * y1r : 0.0;
     const double w1r = tr * q1r - ti * q1i + Kr, w1i = tr * q1i + ti * q1r + Ki;
 #pragma unroll
     for (int k = 0; k < CC; ++k) {
@@ -461,9 +507,9 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       const double qr = qv[0][k], qi = CX ? qv[NP - 1][k] : 0.0;
       w[0][k] = in ? tr * qr - ti * qi + Kr * vr - Ki * vi : 0.0;
       if (CX) w[NP - 1][k] = in ? tr * qi + ti * qr + Kr * vi + Ki * vr : 0.0;
-      // column J+1: conj(row J+1) - v conj(w_1) - w
+      // column J+1 - v conj(w_1) - w
       a[0][k] = in ? cv[0][k] - (vr * w1r + vi * w1i) - w[0][k] : 0.0;
-      if (CX) a[NP - 1][k] = in ? -cv[NP - 1][k] - (vi * w1r - vr * w1i) - w[NP - 1][k] : 0.0;
+      if (CX) a[NP - 1][k] = in ? cv[NP - 1][k] - (vi * w1r - vr * w1i) - w[NP - 1][k] : 0.0;
       if (J == m - 2 && writer && c == m - 1) g.d[m - 1] = a[0][k];
     }
     if (J == m - 2 || last < J + 1) return;
@@ -516,11 +562,11 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
   const bool cx = field == CPLX;
   const int m = n - s0, np = cx ? 2 : 1;
   if (m < 3 || m > trd_resident_max(field)) return false;
-  // workgroup size and rows per workgroup: 15 rows (7 complex) fill the
+  // workgroup size and rows per workgroup: 13 rows (7 complex) fill the
   // 16-value reduction; larger orders take 12 so that the rows fit the
   // registers (512 threads, 256 registers each)
   const int T = m <= 256 ? 256 : 512, CC = (m + T - 1) / T;
-  const int RW = cx ? 7 : (CC <= 2 ? 15 : 12);
+  const int RW = cx ? 7 : (CC <= 2 ? 13 : 12);
   const int G = (m + RW - 1) / RW;
   ResArgs g;
   g.A = A + (long long)s0 * n + s0;
@@ -548,10 +594,10 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
   DMRG_CHECK_HIP(hipGetLastError());
   bool ok = false;
   if (!cx) {
-    if (T == 256) ok = resident_launch<false, 256, 1, 15>(c, g, G);
+    if (T == 256) ok = resident_launch<false, 256, 1, 13>(c, g, G);
     else switch (CC) {
-      case 1: ok = resident_launch<false, 512, 1, 15>(c, g, G); break;
-      case 2: ok = resident_launch<false, 512, 2, 15>(c, g, G); break;
+      case 1: ok = resident_launch<false, 512, 1, 13>(c, g, G); break;
+      case 2: ok = resident_launch<false, 512, 2, 13>(c, g, G); break;
       case 3: ok = resident_launch<false, 512, 3, 12>(c, g, G); break;
       case 4: ok = resident_launch<false, 512, 4, 12>(c, g, G); break;
       case 5: ok = resident_launch<false, 512, 5, 12>(c, g, G); break;

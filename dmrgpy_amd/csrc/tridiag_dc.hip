@@ -338,19 +338,6 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
   }
 }
 
-// sums of four values over the wave
-__device__ __forceinline__ void wave_sums4(double& a, double& b, double& c, double& d) {
-  double t = fold16(fold32(a, c), fold32(b, d));
-  t += dpp<DPP_MIRROR>(t);
-  t += dpp<DPP_HALF_MIRROR>(t);
-  t += dpp<DPP_XOR2>(t);
-  t += dpp<DPP_XOR1>(t);
-  a = lane_value(t, 0);
-  b = lane_value(t, 16);
-  c = lane_value(t, 32);
-  d = lane_value(t, 48);
-}
-
 // Root j of 1/rho + sum_i z_i^2 / (d_i - x): between poles j and j + 1 (the last
 // one past the last pole), as the distance tau from the nearer pole, so that
 // every difference d_i - x is formed without cancellation.  Two-pole rational

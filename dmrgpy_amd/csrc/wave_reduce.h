@@ -74,4 +74,17 @@ __device__ __forceinline__ double lane_value(double x, int l) {   // wave-unifor
   return as_d(((unsigned long long)hi << 32) | lo);
 }
 
+// sums of four values over the wave
+__device__ __forceinline__ void wave_sums4(double& a, double& b, double& c, double& d) {
+  double t = fold16(fold32(a, c), fold32(b, d));
+  t += dpp<DPP_MIRROR>(t);
+  t += dpp<DPP_HALF_MIRROR>(t);
+  t += dpp<DPP_XOR2>(t);
+  t += dpp<DPP_XOR1>(t);
+  a = lane_value(t, 0);
+  b = lane_value(t, 16);
+  c = lane_value(t, 32);
+  d = lane_value(t, 48);
+}
+
 }  // namespace dmrg
