@@ -32,6 +32,7 @@
 // ready for rocsolver_dstedc and the back-transformation below.  All sums
 // run in a fixed order (deterministic).
 #include "dmrg_internal.h"
+#include "gemm_kernels.h"
 
 namespace dmrg {
 
@@ -1060,12 +1061,12 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
 // triangular, LAPACK dlarft forward/columnwise), and each block is applied
 // to the eigenvectors as three GEMMs, last block first.  The eigenvectors
 // are the rows of Zt (keep x n, row-major), so a block is Zt <- Zt Q_b^T:
-//   Y = Zt V_b (split along its long inner dimension into BT_SPLIT partial
-//   products written side by side), Y2 = [Y_0 .. Y_{S-1}] [T_b^T; ..; T_b^T],
+//   Y = Zt V_b (a long inner dimension split into up to BT_SPLIT partial
+//   products written side by side, then added up), Y2 = Y T_b^T,
 //   Zt -= Y2 V_b^T.
 // ---------------------------------------------------------------------------
 constexpr int BT_NB = 128;
-constexpr int BT_SPLIT = 8;
+constexpr int BT_SPLIT = 8, BT_CHUNK = 128;
 
 // Vall[j][r] = v_j[r] for rows j < n - 1 (0 for r <= j, 1 at r = j + 1, the
 // stored entry A[j][r] beyond), zero rows up to the block multiple
@@ -1082,108 +1083,141 @@ __global__ void bt_vall_k(const double* __restrict__ A, int n, int nrefl, long l
   }
 }
 
-// T_b from S_b = V_b V_b^T and tau (one workgroup of 256 threads per block),
-// then BT_SPLIT stacked copies of T_b^T.  T is built by blocked recursion:
-// its 16 x 16 diagonal blocks by the column recurrence (thread k owns row
-// k: T[k][k] = tau_k, T[k][i] = -tau_i sum_{l=k}^{i-1} T[k][l] S[l][i]),
-// then pairs of diagonal blocks of size h = 16, 32, 64 are joined by the
-// compact-WY identity T12 = -T1 (S12 T2) (LAPACK dlarft's recursive form:
-// (I - V1 T1 V1^T)(I - V2 T2 V2^T) = I - V T V^T with that T12), every
-// output an independent dot product.  The serial recurrence over the whole
-// block made row 0 a chain of 127 dependent steps (279 us per call).  The
-// strict upper triangle of S (column-packed) and the upper triangle of T
-// (row-packed) sit in LDS; X = S12 T2 is kept in T12's slots until
-// T12 = -T1 X replaces it (through registers, so no slot is read after it
-// is overwritten).
-constexpr int BT_TRI = BT_NB * (BT_NB + 1) / 2;
-__device__ __forceinline__ int bt_s_idx(int l, int i) { return i * (i - 1) / 2 + l; }            // l < i
-__device__ __forceinline__ int bt_t_idx(int k, int l) { return k * BT_NB - k * (k - 1) / 2 + (l - k); }  // l >= k
+// T_b^T from S_b = V_b^H V_b and tau, one workgroup per block of NB
+// reflectors, T in LDS (row pitch NB + 2: the 16 rows of an operand fall on
+// different banks; 133 KB at NB = 128).  Blocked recursion:
+// - 16 x 16 diagonal blocks: T[k][k] = tau_k, T[k][i] = -tau_i sum_{l<i}
+//   T[k][l] S[l][i].  The rows are independent: one thread per row, its 16
+//   values in registers, each new value added to the later sums at once.
+// - pairs of diagonal blocks of size h = 16, 32, 64 are joined by
+//   T12 = -T1 (S12 T2) (LAPACK dlarft's recursive form: (I - V1 T1 V1^H)
+//   (I - V2 T2 V2^H) = I - V T V^H with that T12) on the matrix cores, one
+//   wave per 16 x 16 output tile and NB / 8 waves for the NB / 8 tiles of the
+//   last level; S12 comes from memory, X = S12 T2 is kept in T12's place.
+// What bounds it is the chain of the levels (the last one 2 x 16 MFMAs per
+// wave, four waves to a SIMD).  Per call, order 128: 130 us with packed
+// triangles and one dot product per output, 18.6 us so.
 constexpr int BT_LEAF = 16;
 
-__global__ __launch_bounds__(256) void bt_larft_k(const double* __restrict__ S, const double* __restrict__ tau,
-                                                  int nrefl, double* __restrict__ TtS) {
-  __shared__ double sS[BT_NB * (BT_NB - 1) / 2];
-  __shared__ double sT[BT_TRI];
-  __shared__ double stau[BT_NB];
-  const int b = blockIdx.x, tid = threadIdx.x;
-  const int j0 = b * BT_NB;
-  const double* Sb = S + (size_t)b * BT_NB * BT_NB;
-  if (tid < BT_NB) stau[tid] = j0 + tid < nrefl ? tau[j0 + tid] : 0.0;
-  for (int idx = tid; idx < BT_NB * BT_NB; idx += 256) {   // S[t][k], kept for t < k
-    const int t = idx / BT_NB, k = idx % BT_NB;
-    if (t < k) sS[bt_s_idx(t, k)] = Sb[idx];
+template <bool CX, int NB>
+__global__ __launch_bounds__(NB * 8) void bt_larft_k(const double* __restrict__ S, long long pS,
+                                                     const double* __restrict__ tau, int nrefl,
+                                                     double* __restrict__ Tt, long long pT) {
+  constexpr int NP = CX ? 2 : 1, P = NB + 2, NT = NB * 8;
+  extern __shared__ double sT[];   // [NP][NB][P]
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j0 = blockIdx.x * NB;
+  const double* Sb = S + (size_t)blockIdx.x * NB * NB;
+  double tr = 0.0, ti = 0.0;
+  if (tid < NB && j0 + tid < nrefl) {
+    tr = CX ? tau[2 * (j0 + tid)] : tau[j0 + tid];
+    if (CX) ti = tau[2 * (j0 + tid) + 1];
+  }
+  // S on the diagonal blocks, zero elsewhere
+  for (int o = tid; o < NB * NB; o += NT) {
+    const int r = o / NB, c = o % NB;
+    const bool dg = r / BT_LEAF == c / BT_LEAF;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) sT[(p * NB + r) * P + c] = dg ? Sb[o + p * pS] : 0.0;
   }
   __syncthreads();
-  if (tid < BT_NB) {   // diagonal blocks of BT_LEAF by the recurrence
-    const int k = tid, end = (k / BT_LEAF + 1) * BT_LEAF;
-    const int tk = bt_t_idx(k, 0);   // row k of T is contiguous
-    sT[tk + k] = stau[k];
-    for (int i = k + 1; i < end; ++i) {
-      const int si = bt_s_idx(0, i);   // column i of S is contiguous
-      double a = 0.0;
-      for (int l = k; l < i; ++l) a += sT[tk + l] * sS[si + l];
-      sT[tk + i] = -stau[i] * a;
+  if (tid < NB) {   // whole waves: NB is a multiple of 64
+    const int k = tid & (BT_LEAF - 1), base = tid - k;
+    double x[NP][BT_LEAF];
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int i = 0; i < BT_LEAF; ++i) x[p][i] = 0.0;
+#pragma unroll
+    for (int i = 0; i < BT_LEAF; ++i) {
+      const double tir = __shfl(tr, (lane & 48) + i), tii = CX ? __shfl(ti, (lane & 48) + i) : 0.0;
+      const double ar = x[0][i], ai = CX ? x[NP - 1][i] : 0.0;   // sum_{l < i} T[k][l] S[l][i]
+      const double vr = i == k ? tir : (i < k ? 0.0 : -(tir * ar - tii * ai));
+      const double vi = i == k ? tii : (i < k ? 0.0 : -(tir * ai + tii * ar));
+      x[0][i] = vr;
+      if (CX) x[NP - 1][i] = vi;
+#pragma unroll
+      for (int j = i + 1; j < BT_LEAF; ++j) {
+        const double sr = sT[(base + i) * P + base + j];
+        if (!CX) {
+          x[0][j] += vr * sr;
+        } else {
+          const double si = sT[(NB + base + i) * P + base + j];
+          x[0][j] += vr * sr - vi * si;
+          x[NP - 1][j] += vr * si + vi * sr;
+        }
+      }
     }
+    // a block's 16 rows belong to one wave: its reads are done
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int i = 0; i < BT_LEAF; ++i) sT[(p * NB + tid) * P + base + i] = x[p][i];
   }
   __syncthreads();
-  constexpr int MAXPER = BT_NB * (BT_NB / 2) / 2 / 256;   // outputs per thread at the last level (16)
-  for (int h = BT_LEAF; h < BT_NB; h *= 2) {
-    const int per = BT_NB * h / 2 / 256;   // (BT_NB / 2h) pairs x h x h outputs over 256 threads
-    double x[MAXPER];
-    // X = S12 T2 into the T12 slots (T2 is read, T12 only written: disjoint)
+  typedef Mfma<double>::acc_t acc_t;
+  for (int h = BT_LEAF; h < NB; h *= 2) {
+    const int ht = h / BT_LEAF, tiles = NB / (2 * h) * ht * ht;
+    const bool mine = wave < tiles;
+    const int pr = wave / (ht * ht), tr16 = wave % (ht * ht) / ht * BT_LEAF, tc16 = wave % ht * BT_LEAF;
+    const int r0 = 2 * h * pr, c0 = r0 + h;   // T1 at (r0, r0), T2 at (c0, c0), T12 at (r0, c0)
+    acc_t acc[NP];
+    for (int step = 0; step < 2; ++step) {   // X = S12 T2, then T1 X
 #pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        double a = 0.0;
-        for (int l = b0 + h; l <= i; ++l) a += sS[bt_s_idx(k, l)] * sT[bt_t_idx(l, i)];
-        x[e] = a;
+      for (int p = 0; p < NP; ++p) acc[p] = acc_t{0.0, 0.0, 0.0, 0.0};
+      if (mine) {
+        // T2 is zero below its diagonal tiles, T1 left of them
+        const int k0 = step ? tr16 : 0, k1 = step ? h : tc16 + BT_LEAF;
+        const int bo = step ? r0 : c0;   // first row of the right factor
+        for (int k = k0; k < k1; k += 4) {
+          const int kk = k + lk;
+          const double ar = step ? sT[(r0 + tr16 + li) * P + r0 + kk] : Sb[(r0 + tr16 + li) * NB + c0 + kk];
+          const double br = sT[(bo + kk) * P + c0 + tc16 + li];
+          acc[0] = Mfma<double>::op(ar, br, acc[0]);
+          if (CX) {
+            const double ai = step ? sT[(NB + r0 + tr16 + li) * P + r0 + kk] : Sb[(r0 + tr16 + li) * NB + c0 + kk + pS];
+            const double bi = sT[(NB + bo + kk) * P + c0 + tc16 + li];
+            acc[0] = Mfma<double>::op(-ai, bi, acc[0]);
+            acc[NP - 1] = Mfma<double>::op(ar, bi, acc[NP - 1]);
+            acc[NP - 1] = Mfma<double>::op(ai, br, acc[NP - 1]);
+          }
+        }
       }
-    }
+      if (step) __syncthreads();   // T12's place holds X until every wave has read it
+      if (mine) {
 #pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        sT[bt_t_idx(k, i)] = x[e];
-      }
-    }
-    __syncthreads();
-    // T12 = -T1 X
+        for (int p = 0; p < NP; ++p)
 #pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        const int tk = bt_t_idx(k, 0);
-        double a = 0.0;
-        for (int l = k; l < b0 + h; ++l) a += sT[tk + l] * sT[bt_t_idx(l, i)];
-        x[e] = -a;
+          for (int e = 0; e < 4; ++e)
+            sT[(p * NB + r0 + tr16 + 4 * e + lk) * P + c0 + tc16 + li] = step ? -acc[p][e] : acc[p][e];
       }
+      __syncthreads();
     }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        sT[bt_t_idx(k, i)] = x[e];
-      }
-    }
-    __syncthreads();
   }
-  double* out = TtS + (size_t)b * BT_SPLIT * BT_NB * BT_NB;
-  for (int idx = tid; idx < BT_NB * BT_NB; idx += 256) {   // row k of T^T = column k of T
-    const int k = idx / BT_NB, i = idx % BT_NB;
-    const double v = i <= k ? sT[bt_t_idx(i, k)] : 0.0;
-    for (int s = 0; s < BT_SPLIT; ++s) out[((size_t)s * BT_NB + k) * BT_NB + i] = v;
+  double* out = Tt + (size_t)blockIdx.x * NB * NB;
+  for (int o = tid; o < NB * NB; o += NT) {   // row r of T^T = column r of T
+    const int r = o / NB, c = o % NB;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) out[o + p * pT] = c <= r ? sT[(p * NB + c) * P + r] : 0.0;
   }
 }
+
+template <bool CX, int NB>
+void bt_larft(Ctx* c, const double* S, long long pS, const double* tau, int nrefl, double* Tt, long long pT) {
+  const int nblk = (nrefl + NB - 1) / NB;
+  constexpr int lds = (CX ? 2 : 1) * NB * (NB + 2) * (int)sizeof(double);
+  if (lds > 65536) {
+    DMRG_CHECK_HIP(hipFuncSetAttribute((const void*)bt_larft_k<CX, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  }
+  bt_larft_k<CX, NB><<<nblk, NB * 8, lds, c->stream>>>(S, pS, tau, nrefl, Tt, pT);
+  DMRG_CHECK_HIP(hipGetLastError());
+}
+
+// partial products along an inner dimension of len: chunks of BT_CHUNK or
+// longer, at most BT_SPLIT (short ones are split inside the GEMM, with no
+// pass to add them up)
+int bt_splits(int len) { return std::max(1, std::min(BT_SPLIT, len / BT_CHUNK)); }
 
 // Y[c][i] = sum_s Ycat[c][s nb + i] (the split inner products of a block, in
 // order), for every plane: rows*nb outputs per plane, plane strides pin/pout
@@ -1211,11 +1245,11 @@ void ormtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
   const int nblk = (nrefl + BT_NB - 1) / BT_NB;
   const size_t vrows = (size_t)nblk * BT_NB;
   double* Vall = (double*)ws_get(c, WS_BT_V, sizeof(double) * vrows * n);
-  const size_t nS = (size_t)nblk * BT_NB * BT_NB, nT = (size_t)nblk * BT_SPLIT * BT_NB * BT_NB;
+  const size_t nS = (size_t)nblk * BT_NB * BT_NB, nT = nS;
   const size_t nY = (size_t)keep * (BT_SPLIT + 1) * BT_NB, nY2 = (size_t)keep * BT_NB;   // S partials + their sum
   double* Sm = (double*)ws_get(c, WS_BT_W, sizeof(double) * (nS + nT + nY + nY2));
-  double* TtS = Sm + nS;
-  double* Ycat = TtS + nT;
+  double* Tt = Sm + nS;
+  double* Ycat = Tt + nT;
   double* Y2 = Ycat + nY;
   const long long total = (long long)vrows * n;
   bt_vall_k<<<(int)std::min<long long>((total + 255) / 256, 65536), 256, 0, c->stream>>>(A, n, nrefl, total, Vall);
@@ -1228,13 +1262,12 @@ void ormtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
     g.sC = (long long)BT_NB * BT_NB;
     gemm_f64(c, g, Vall, Vall, Sm);
   }
-  bt_larft_k<<<nblk, 256, 0, c->stream>>>(Sm, tau, nrefl, TtS);
-  DMRG_CHECK_HIP(hipGetLastError());
+  bt_larft<false, BT_NB>(c, Sm, 0, tau, nrefl, Tt, 0);
   for (int b = nblk - 1; b >= 0; --b) {
     const int b0 = b * BT_NB;
     const int len = n - b0 - 1;   // columns b0 + 1 .. n - 1 carry block b
     if (len <= 0) continue;
-    int S = BT_SPLIT, kc = len, start = b0 + 1;
+    int S = bt_splits(len), kc = len, start = b0 + 1;
     for (; S >= 1; --S) {   // S equal chunks ending at column n; columns left of b0 + 1 meet zero rows of V_b
       kc = (len + S - 1) / S;
       start = n - S * kc;
@@ -1258,7 +1291,7 @@ void ormtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
       Y = Ys;
     }
     GemmDesc g2 = gdesc(keep, BT_NB, BT_NB, BT_NB, BT_NB, BT_NB, REAL, 4);
-    gemm_f64(c, g2, Y, TtS + (size_t)b * BT_SPLIT * BT_NB * BT_NB, Y2);
+    gemm_f64(c, g2, Y, Tt + (size_t)b * BT_NB * BT_NB, Y2);
     GemmDesc g3 = gdesc(keep, len, BT_NB, BT_NB, n, n, REAL, 4);
     g3.alpha = -1.0;
     g3.beta = 1.0;
@@ -1274,7 +1307,6 @@ void ormtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
 // Et = (Q Y)^T as Et <- Et - (Et conj(V_b)) T_b^T V_b^T, last block first.
 // ---------------------------------------------------------------------------
 constexpr int BTC_NB = 64;
-constexpr int BTC_TRI = BTC_NB * (BTC_NB + 1) / 2;
 
 __global__ void btc_vall_k(const double* __restrict__ A, int n, int nrefl, long long total,
                            double* __restrict__ Vall) {
@@ -1295,126 +1327,6 @@ __global__ void btc_vall_k(const double* __restrict__ A, int n, int nrefl, long 
   }
 }
 
-__device__ __forceinline__ int btc_s_idx(int l, int i) { return i * (i - 1) / 2 + l; }
-__device__ __forceinline__ int btc_t_idx(int k, int l) { return k * BTC_NB - k * (k - 1) / 2 + (l - k); }
-
-// S planar (plane stride pS), tau interleaved; TtS planar (plane stride pT).
-// The same blocked recursion as bt_larft_k in complex arithmetic
-// (S[l][i] = v_l^H v_i, T12 = -T1 S12 T2 from (I - V1 T1 V1^H)(I - V2 T2 V2^H)),
-// 256 threads: 16 x 16 diagonal blocks by the recurrence, then levels 16, 32.
-__global__ __launch_bounds__(256) void btc_larft_k(const double* __restrict__ S, long long pS,
-                                                  const double* __restrict__ tau, int nrefl,
-                                                  double* __restrict__ TtS, long long pT) {
-  __shared__ double sSr[BTC_TRI], sSi[BTC_TRI], sTr[BTC_TRI], sTi[BTC_TRI];
-  __shared__ double str[BTC_NB], sti[BTC_NB];
-  const int b = blockIdx.x, tid = threadIdx.x;
-  const int j0 = b * BTC_NB;
-  const double* Sb = S + (size_t)b * BTC_NB * BTC_NB;
-  if (tid < BTC_NB) {
-    str[tid] = j0 + tid < nrefl ? tau[2 * (j0 + tid)] : 0.0;
-    sti[tid] = j0 + tid < nrefl ? tau[2 * (j0 + tid) + 1] : 0.0;
-  }
-  for (int idx = tid; idx < BTC_NB * BTC_NB; idx += 256) {   // S[t][k], kept for t < k
-    const int t = idx / BTC_NB, k = idx % BTC_NB;
-    if (t < k) {
-      sSr[btc_s_idx(t, k)] = Sb[idx];
-      sSi[btc_s_idx(t, k)] = Sb[idx + pS];
-    }
-  }
-  __syncthreads();
-  if (tid < BTC_NB) {   // diagonal blocks of BT_LEAF by the recurrence
-    const int k = tid, end = (k / BT_LEAF + 1) * BT_LEAF;
-    const int tk = btc_t_idx(k, 0);
-    sTr[tk + k] = str[k];
-    sTi[tk + k] = sti[k];
-    for (int i = k + 1; i < end; ++i) {
-      const int si = btc_s_idx(0, i);
-      double ar = 0.0, ai = 0.0;
-      for (int l = k; l < i; ++l) {
-        const double xr = sTr[tk + l], xi = sTi[tk + l], yr = sSr[si + l], yi = sSi[si + l];
-        ar += xr * yr - xi * yi;
-        ai += xr * yi + xi * yr;
-      }
-      sTr[tk + i] = -(str[i] * ar - sti[i] * ai);
-      sTi[tk + i] = -(str[i] * ai + sti[i] * ar);
-    }
-  }
-  __syncthreads();
-  constexpr int MAXPER = BTC_NB * (BTC_NB / 2) / 2 / 256;   // 4
-  for (int h = BT_LEAF; h < BTC_NB; h *= 2) {
-    const int per = BTC_NB * h / 2 / 256;
-    double xr[MAXPER], xi[MAXPER];
-#pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {   // X = S12 T2 into the T12 slots
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        double ar = 0.0, ai = 0.0;
-        for (int l = b0 + h; l <= i; ++l) {
-          const double sr = sSr[btc_s_idx(k, l)], si = sSi[btc_s_idx(k, l)];
-          const double tr = sTr[btc_t_idx(l, i)], ti = sTi[btc_t_idx(l, i)];
-          ar += sr * tr - si * ti;
-          ai += sr * ti + si * tr;
-        }
-        xr[e] = ar;
-        xi[e] = ai;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        sTr[btc_t_idx(k, i)] = xr[e];
-        sTi[btc_t_idx(k, i)] = xi[e];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {   // T12 = -T1 X
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        const int tk = btc_t_idx(k, 0);
-        double ar = 0.0, ai = 0.0;
-        for (int l = k; l < b0 + h; ++l) {
-          const double ur = sTr[tk + l], ui = sTi[tk + l];
-          const double vr = sTr[btc_t_idx(l, i)], vi = sTi[btc_t_idx(l, i)];
-          ar += ur * vr - ui * vi;
-          ai += ur * vi + ui * vr;
-        }
-        xr[e] = -ar;
-        xi[e] = -ai;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < MAXPER; ++e) {
-      if (e < per) {
-        const int o = tid + 256 * e;
-        const int p = o / (h * h), r = o % (h * h);
-        const int b0 = 2 * h * p, k = b0 + r / h, i = b0 + h + r % h;
-        sTr[btc_t_idx(k, i)] = xr[e];
-        sTi[btc_t_idx(k, i)] = xi[e];
-      }
-    }
-    __syncthreads();
-  }
-  double* out = TtS + (size_t)b * BT_SPLIT * BTC_NB * BTC_NB;
-  for (int idx = tid; idx < BTC_NB * BTC_NB; idx += 256) {   // row r of T^T (column r of T)
-    const int r = idx / BTC_NB, k = idx % BTC_NB;
-    const double vr = k <= r ? sTr[btc_t_idx(k, r)] : 0.0, vi = k <= r ? sTi[btc_t_idx(k, r)] : 0.0;
-    for (int s = 0; s < BT_SPLIT; ++s) {
-      const size_t o = ((size_t)s * BTC_NB + r) * BTC_NB + k;
-      out[o] = vr;
-      out[o + pT] = vi;
-    }
-  }
-}
-
 // Et (keep x n planar, plane stride keep*n) <- rows of Q Y for hetrd_lower's
 // reflectors in A (planar, plane stride n*n) and tau (interleaved); nrefl
 // reflectors (n - 1 when negative)
@@ -1426,11 +1338,11 @@ void unmtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
   const size_t vrows = (size_t)nblk * NB;
   const long long pV = (long long)vrows * n;
   double* Vall = (double*)ws_get(c, WS_BT_V, sizeof(double) * 2 * (size_t)pV);
-  const size_t nS = (size_t)nblk * NB * NB, nT = (size_t)nblk * BT_SPLIT * NB * NB;
+  const size_t nS = (size_t)nblk * NB * NB, nT = nS;
   const size_t nY = (size_t)keep * (BT_SPLIT + 1) * NB, nY2 = (size_t)keep * NB;   // S partials + their sum
   double* Sm = (double*)ws_get(c, WS_BT_W, sizeof(double) * 2 * (nS + nT + nY + nY2));
-  double* TtS = Sm + 2 * nS;
-  double* Ycat = TtS + 2 * nT;
+  double* Tt = Sm + 2 * nS;
+  double* Ycat = Tt + 2 * nT;
   double* Y2 = Ycat + 2 * nY;
   btc_vall_k<<<(int)std::min<long long>((pV + 255) / 256, 65536), 256, 0, c->stream>>>(A, n, nrefl, pV, Vall);
   DMRG_CHECK_HIP(hipGetLastError());
@@ -1445,14 +1357,13 @@ void unmtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
     g.pC = (long long)nS;
     gemm_f64(c, g, Vall, Vall, Sm);
   }
-  btc_larft_k<<<nblk, 256, 0, c->stream>>>(Sm, (long long)nS, tau, nrefl, TtS, (long long)nT);
-  DMRG_CHECK_HIP(hipGetLastError());
+  bt_larft<true, BTC_NB>(c, Sm, (long long)nS, tau, nrefl, Tt, (long long)nT);
   const long long pE = (long long)keep * n;
   for (int b = nblk - 1; b >= 0; --b) {
     const int b0 = b * NB;
     const int len = n - b0 - 1;
     if (len <= 0) continue;
-    int S = BT_SPLIT, kc = len, start = b0 + 1;
+    int S = bt_splits(len), kc = len, start = b0 + 1;
     for (; S >= 1; --S) {
       kc = (len + S - 1) / S;
       start = n - S * kc;
@@ -1483,7 +1394,7 @@ void unmtr_lower_rows(Ctx* c, const double* A, int n, const double* tau, double*
     g2.pA = (long long)nY;
     g2.pB = (long long)nT;
     g2.pC = (long long)nY2;
-    gemm_f64(c, g2, Y, TtS + (size_t)b * BT_SPLIT * NB * NB, Y2);
+    gemm_f64(c, g2, Y, Tt + (size_t)b * NB * NB, Y2);
     GemmDesc g3 = gdesc(keep, len, NB, NB, n, n, CPLX, 4);   // Et -= Y2 V_b^T
     g3.alpha = -1.0;
     g3.beta = 1.0;
