@@ -81,6 +81,11 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
 bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double* e, double* tau, double stop_tol,
                   double total2, int* done, double* dropped);
 int trd_resident_max(int field);   // largest order it takes
+
+// Real orders up to trd_single_max() in one workgroup (trd_single.hip)
+void trd_single(Ctx* c, double* A, int n, double* d, double* e, double* tau, double stop_tol, int* done,
+                double* dropped);
+int trd_single_max();
 // Divide and conquer on a real symmetric tridiagonal matrix (tridiag_dc.hip):
 // eigenvalues ascending into w (w may be d), then the rows of Zt (keep x n,
 // pitch ldz) as the eigenvectors of the `keep` largest ones, ascending

@@ -1,6 +1,6 @@
 // Householder tridiagonalisation of a real symmetric matrix (LAPACK dsytrd,
-// lower storage conventions), two kernel launches per column.  Orders whose
-// rows fit the register files (real 3072, complex 1792) are reduced there in
+// lower storage conventions), two kernel launches per column.  Real orders up
+// to 128 are reduced by one workgroup (trd_single.hip).  Orders whose rows fit the register files (real 3072, complex 1792) are reduced there in
 // one launch instead (trd_resident.hip); this path reduces larger matrices
 // down to that order by panels, and any order when the resident kernel gives
 // up.
@@ -441,6 +441,17 @@ static double trailing_sumsq_wait(Ctx* c, int slot) {
 constexpr int TRD_STOP_MIN = 64;
 int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, double stop_tol, double* dropped) {
   DMRG_REQUIRE(n >= 2, "sytrd: order must be at least 2");
+  if (n <= trd_single_max()) {   // one workgroup holds the matrix (trd_single.hip)
+    ProfScope ps(c, 4, 0.0, 0.0);
+    int done = n - 1;
+    trd_single(c, A, n, d, e, tau, n > TRD_STOP_MIN + TRD_NB ? stop_tol : 0.0, &done, dropped);
+    if (done < n - 1) {
+      trd_clear_tail_k<<<1, 256, 0, c->stream>>>(n, done, d, e, tau, 1);
+      DMRG_CHECK_HIP(hipGetLastError());
+    }
+    for (int j = 0; j < done; ++j) ps.bytes += 8.0 * (double)(n - j - 1) * (n - j) / 2.0;
+    return done;
+  }
   const size_t vwv = (size_t)n * TRD_P;   // the [V | W | V] panel store
   const int gmax1 = (n + TRD_ROWS1 - 1) / TRD_ROWS1;
   const int gmax2 = (n + TRD_ROWS2 - 1) / TRD_ROWS2;
