@@ -37,7 +37,9 @@ __device__ __forceinline__ void xcd_tile(int nbx, int nby, int& tr, int& tc) {
 template <typename T, int TM, int TN, bool TA, bool TB, int TAG, typename CT = T>
 __global__ __launch_bounds__(256) void gemm_fast(const T* __restrict__ A, const T* __restrict__ B,
                                                  CT* __restrict__ C, GemmArgs g) {
-  constexpr int BM = 32 * TM, BN = 32 * TN, BK = 16;
+  // k per tile: 16, or 32 where 16 would not give every thread whole vectors
+  constexpr int BM = 32 * TM, BN = 32 * TN;
+  constexpr int BK = (BM * 16) % (Vec<T>::W * 256) == 0 && (BN * 16) % (Vec<T>::W * 256) == 0 ? 16 : 32;
   constexpr int PAD = 16 / sizeof(T);     // keeps rows 16-byte aligned
   constexpr int VW = Vec<T>::W;
   typedef typename Vec<T>::type vec_t;
@@ -202,25 +204,28 @@ __global__ __launch_bounds__(256) void gemm_fast(const T* __restrict__ A, const 
   for (int k0 = 0; k0 < K; k0 += BK) {
     const bool more = k0 + BK < K;
     if (more) load_regs(k0 + BK);
-    T fa[TM][4], fb[TN][4];
 #pragma unroll
-    for (int a = 0; a < TM; ++a) {
-      const int row = wm * TM * 16 + a * 16 + li;
+    for (int kk = 0; kk < BK; kk += 16) {
+      T fa[TM][4], fb[TN][4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) fa[a][t] = TA ? As[cur][lk * 4 + t][row] : As[cur][row][lk * 4 + t];
+      for (int a = 0; a < TM; ++a) {
+        const int row = wm * TM * 16 + a * 16 + li;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) fa[a][t] = TA ? As[cur][kk + lk * 4 + t][row] : As[cur][row][kk + lk * 4 + t];
+      }
+#pragma unroll
+      for (int b = 0; b < TN; ++b) {
+        const int col = wn * TN * 16 + b * 16 + li;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) fb[b][t] = TB ? Bs[cur][col][kk + lk * 4 + t] : Bs[cur][kk + lk * 4 + t][col];
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+          for (int b = 0; b < TN; ++b) acc[a][b] = Mfma<T>::op(fa[a][t], fb[b][t], acc[a][b]);
     }
-#pragma unroll
-    for (int b = 0; b < TN; ++b) {
-      const int col = wn * TN * 16 + b * 16 + li;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) fb[b][t] = TB ? Bs[cur][col][lk * 4 + t] : Bs[cur][lk * 4 + t][col];
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b) acc[a][b] = Mfma<T>::op(fa[a][t], fb[b][t], acc[a][b]);
     if (more) store_regs(cur ^ 1);
     __syncthreads();
     cur ^= 1;
@@ -613,8 +618,8 @@ static void launch_fast(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C
   else launch_fast_tagged<T, TM, TN, true, true, CT>(c, d, A, B, C);
 }
 
-// Which kernel a real product takes.  The LDS kernel runs 128 x 128 (FP32)
-// or 64 x 64 tiles; products whose 64 x 64 tiles would leave the 256 CUs idle
+// Which kernel a real product takes.  The LDS kernel runs square tiles
+// of 64 (FP32 also 96 and 128); products whose 64 x 64 tiles would leave the 256 CUs idle
 // or badly balanced go to the direct-load kernel (gemm_direct.hip), which
 // spreads 16 x 16 / 32 x 32 tiles and splits the inner dimension.  Measured
 // (LDS 64 x 64 / direct, us):
@@ -631,14 +636,32 @@ static bool use_direct(const GemmDesc& d, bool f64) {
   return tiles64 < (f64 ? (d.K <= 200 ? 160 : 512) : 200);
 }
 
-// FP32 tile of the LDS kernel: 128 x 128 where its tiles fill whole rounds of
-// the 256 CUs to three quarters (3918 x 11696 x 653: 522 us against 571 with
-// 64 x 64; 10448 x 731 x 4386, 492 tiles: 578 against 663), 64 x 64 otherwise
-// (857 x 857 x 3380 x 6, 294 tiles: 325 against 458; 4800 x 300 x 1800, 114
-// tiles: 80 against 135).
-static bool use_tile128(const GemmDesc& d) {
-  const long long t = (long long)((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
-  return 4 * t >= 3 * 256 * ((t + 255) / 256);
+// FP32 tile of the LDS kernel: 128, 96 or 64 square, whichever is estimated
+// fastest: rounds of the 256 CUs x tile area x the time per area and k, which
+// measured 4.2 / 4.45 / 4.75 e-6 us (smaller tiles read LDS more per MFMA);
+// a single round (two of 64 x 64) has too few workgroups per CU to hide its
+// loads and measured 1.1 / 1.25 / 1.17 times that.  Measured (us, 128 / 96 / 64):
+//   857 x 857 x 3380 x 6     464 / 280 / 323     1500^3               114 / 75 / 92
+//   5070 x 3428 x 845        291 / 273 / 279     2200 x 2200 x 1100   150 / 135 / 110
+//   10448 x 731 x 4386       579 / 685 / 662     700 x 700 x 2800 x 6 224 / 231 / 166
+//   6144 x 16384 x 1024     1581 / 1663 / 1837   4800 x 300 x 1800    136 / 90 / 82
+static int fast_tile(const GemmDesc& d) {
+  auto cost = [&](int tile, double per_area, int few, double penalty) {
+    const long long t = (long long)((d.M + tile - 1) / tile) * ((d.N + tile - 1) / tile) * d.batch;
+    const long long rounds = (t + 255) / 256;
+    return (double)rounds * tile * tile * per_area * (rounds <= few ? penalty : 1.0);
+  };
+  const double c128 = cost(128, 1.0, 1, 1.1), c96 = cost(96, 1.07, 1, 1.25), c64 = cost(64, 1.14, 2, 1.17);
+  return c128 <= c96 && c128 <= c64 ? 128 : (c96 <= c64 ? 96 : 64);
+}
+
+template <typename CT>
+static void launch_fast_f32(Ctx* c, const GemmDesc& d, const float* A, const float* B, CT* C) {
+  switch (fast_tile(d)) {
+    case 128: launch_fast<float, 4, 4, CT>(c, d, A, B, C); break;
+    case 96: launch_fast<float, 3, 3, CT>(c, d, A, B, C); break;
+    default: launch_fast<float, 2, 2, CT>(c, d, A, B, C);
+  }
 }
 
 // Real FP32 GEMM writing an FP64 result (the R-step of the FP32 H_eff apply
@@ -648,8 +671,7 @@ void gemm_f32_c64(Ctx* c, const GemmDesc& d, const float* A, const float* B, dou
   check_desc(d);
   if (d.M == 0 || d.N == 0) return;
   if (use_direct(d, false)) gemm_direct_f32_c64(c, d, A, B, C);
-  else if (use_tile128(d)) launch_fast<float, 4, 4, double>(c, d, A, B, C);
-  else launch_fast<float, 2, 2, double>(c, d, A, B, C);
+  else launch_fast_f32(c, d, A, B, C);
 }
 
 void gemm_f64(Ctx* c, const GemmDesc& d, const double* A, const double* B, double* C) {
@@ -663,8 +685,7 @@ void gemm_f32(Ctx* c, const GemmDesc& d, const float* A, const float* B, float* 
   check_desc(d);
   if (d.M == 0 || d.N == 0) return;
   if (d.field == CPLX || use_direct(d, false)) gemm_direct_f32(c, d, A, B, C);
-  else if (use_tile128(d)) launch_fast<float, 4, 4>(c, d, A, B, C);
-  else launch_fast<float, 2, 2>(c, d, A, B, C);
+  else launch_fast_f32(c, d, A, B, C);
 }
 
 // C[i][j] = conj(C[j][i]) for j > i (n x n, row pitch ld, imaginary plane at

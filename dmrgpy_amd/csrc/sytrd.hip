@@ -1,9 +1,9 @@
 // Householder tridiagonalisation of a real symmetric matrix (LAPACK dsytrd,
 // lower storage conventions), two kernel launches per column.  Real orders up
-// to 128 are reduced by one workgroup (trd_single.hip).  Orders whose rows fit the register files (real 3072, complex 1792) are reduced there in
-// one launch instead (trd_resident.hip); this path reduces larger matrices
-// down to that order by panels, and any order when the resident kernel gives
-// up.
+// to 128 are reduced by one workgroup (trd_single.hip), other orders whose rows
+// fit the register files (real 3072, complex 1792) across workgroups in one
+// launch (trd_resident.hip); this path reduces larger matrices down to that
+// order by panels, and any order when the resident kernel gives up.
 //
 // The dense symmetric eigensolver behind every Gram-route split spends most
 // of its time reducing the matrix to tridiagonal form, one column at a time.
