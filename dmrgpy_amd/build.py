@@ -5,7 +5,8 @@
 Objects go to dmrgpy_amd/_build/, the shared library to
 dmrgpy_amd/libdmrg_hip.so.  Every HIP source is compiled with packed-FP32
 instructions disabled (-packed-fp32-ops) and linked against rocBLAS /
-rocSOLVER (the latter provides the dense symmetric eigensolver of the SVD).
+rocSOLVER (the full SVD of small or ill-conditioned splits, and the dense
+eigensolvers the own one is compared with).
 """
 
 import os

@@ -98,9 +98,9 @@ struct Ctx {
   double prof_bytes[5] = {0, 0, 0, 0, 0};   // algorithmic HBM bytes
   long long prof_calls[5] = {0, 0, 0, 0, 0};
   long long matvecs = 0;
-  // dense eigensolver of the Gram route: 1 (default) = own two-launch
-  // tridiagonalisation (real or complex Hermitian; a real reduction stops
-  // once the trailing block is below TRD_STOP_TOL |G|_F) + rocSOLVER stedc +
+  // dense eigensolver of the Gram route: 1 (default) = own
+  // tridiagonalisation (real or complex Hermitian, stopping once the
+  // trailing block is below TRD_STOP_TOL |G|_F) + own divide and conquer +
   // the library's blocked back-transformation of the kept eigenvectors;
   // 3 = the same with the reduction always complete; 2 = complete reduction
   // with rocSOLVER ormtr / unmtr for the back-transformation; 0 = rocSOLVER

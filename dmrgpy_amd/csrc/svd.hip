@@ -3,8 +3,9 @@
 //            E = top-keep eigenvectors (rows, descending), U = E^dag,
 //            S Vh = E M  (so a right-moving split needs no scaling at all)
 //   m >  n:  G = M^dag M, Vh = E, U S = M E^dag
-// The dense symmetric eigen-decomposition is rocSOLVER's syevd/heevd.  The
-// keep count follows the cutoff / maxdim / mindim rule of the reference's
+// The dense symmetric eigen-decomposition is the library's own
+// (sytrd.hip, trd_resident.hip, trd_single.hip, tridiag_dc.hip).  The keep
+// count follows the cutoff / maxdim / mindim rule of the reference's
 // _truncate (src/dmrgpy/pyitensor/svd.py:32-68) on the host, and the same
 // fallback to a full SVD (rocSOLVER gesvd) applies when the matrix is small
 // (min(m,n) < 16) or the smallest kept singular value is below 1e-7 of the
@@ -937,8 +938,8 @@ int svd_split_entry(Ctx* c, int field, const double* M, int m, int n, double cut
 
 // All eigenpairs of a real symmetric matrix (row-major = column-major):
 // w ascending, Z[k][:] the eigenvector of w[k] (rows of the row-major Z).
-// modes 1 and 3: own tridiagonalisation (always complete here) + stedc + own
-// back-transformation, mode 2: the same with rocSOLVER's ormtr, mode 0:
+// modes 1 and 3: own tridiagonalisation (always complete here), divide and
+// conquer and back-transformation, mode 2: the same with rocSOLVER's ormtr, mode 0:
 // syevd.  A is overwritten.
 int sym_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
   DMRG_REQUIRE(n >= 2, "sym_eig: order must be at least 2");
@@ -975,7 +976,7 @@ int sym_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
 
 // All eigenpairs of a Hermitian matrix A (row-major, planar complex, plane
 // stride n*n): w ascending, Z planar with Z[k][:] the eigenvector of w[k].
-// modes 1 and 3: own reduction + stedc + own back-transformation, mode 2:
+// modes 1 and 3: own reduction, divide and conquer, back-transformation, mode 2:
 // the same with rocSOLVER's unmtr, mode 0: heevd.  A is overwritten.
 // The column-major view of the buffer is conj(A); its eigenvectors come out
 // as rows of the interleaved buffer and are conjugated on the way out.

@@ -230,7 +230,7 @@ class Engine:
 
     def set_eigensolver(self, mode):
         """Eigensolver of the Gram-route splits.  1 (default): own
-        tridiagonalisation (real or Hermitian) + rocSOLVER stedc + the
+        tridiagonalisation (real or Hermitian) and divide and conquer + the
         library's blocked back-transformation of the kept eigenvectors, the
         reduction stopping once its trailing block is below 2e-15 of
         the Gram matrix in Frobenius norm (orders above 96); 3: as 1 with

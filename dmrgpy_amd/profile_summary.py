@@ -97,10 +97,10 @@ def calibration(path, counter, nbytes):
 
 
 CATEGORIES = (
-    ("trd", "own Householder tridiagonalisation (real: trd_col_k, trd_symv_k, trd_fin_k; complex Hermitian: "
-            "trc_col_k, trc_symv_k, trc_fin_k; its panel GEMMs count as SVD GEMMs)"),
-    ("eigensolver", "rocSOLVER/rocBLAS: tridiagonal divide and conquer (stedc), back-transformation (ormtr), "
-                    "syevd/heevd where used, and the library GEMMs they call"),
+    ("trd", "own Householder tridiagonalisation (trd_single_k, trd_resident_k; by panels trd_col_k, trd_symv_k, "
+            "trd_fin_k, complex trc_*; its panel GEMMs count as SVD GEMMs)"),
+    ("eigensolver", "own tridiagonal divide and conquer (dc_*) and T factors (bt_*); rocSOLVER/rocBLAS: full SVDs, "
+                    "stedc, ormtr, syevd/heevd where used, and the library GEMMs they call"),
     ("heff", "H_eff GEMMs (L- and R-step)"),
     ("smallop", "small operator (MPO W) passes"),
     ("svd", "SVD GEMMs (Gram, factors, Loewdin, guided subspace)"),
@@ -116,14 +116,15 @@ CATEGORIES = (
 def _category(name):
     if "trd_" in name or "trc_" in name:
         return "trd"
-    if "rocsolver" in name or "rocblas" in name or name.startswith("Cijk_"):
+    if "rocsolver" in name or "rocblas" in name or name.startswith("Cijk_") or "dmrg::dc_" in name \
+            or "dmrg::bt_" in name or "dmrg::btc_" in name:
         return "eigensolver"
     if name.startswith("void dmrg::gemm"):
         tag = _gemm_tag(name)
         return {"1": "heff", "2": "heff", "3": "env", "4": "svd", "5": "grad"}.get(tag, "other")
     if "smallop" in name:
         return "smallop"
-    if any(k in name for k in ("dot_block", "sub_block", "reduce_rows", "combine_k", "scale_copy", "axpy")):
+    if any(k in name for k in ("kry_", "dot_block", "sub_block", "reduce_rows", "combine_k", "scale_copy", "axpy")):
         return "krylov"
     if any(k in name for k in ("convert", "split_rows", "split_transpose")):
         return "convert"

@@ -170,13 +170,14 @@ int dmrg_svd_split_guided(dmrg_ctx* ctx, int field, const double* M, int m, int 
 /* Dense eigensolver of the Gram route (the np.linalg.eigh call of
  * _svd_truncated, src/dmrgpy/pyitensor/svd.py:134): mode 1 (the default)
  * reduces the real symmetric or complex Hermitian Gram matrix to a real
- * tridiagonal with this library's two-launch-per-column Householder
- * kernels, runs rocSOLVER's divide and conquer on the tridiagonal and
- * back-transforms only the eigenvectors the truncation keeps with this
- * library's blocked compact-WY GEMMs.  For a real Gram matrix of order
- * above 96, mode 1 stops the reduction after the first full panel (at or
- * past column 64) whose trailing block has Frobenius norm at most 2e-15
- * of the Gram matrix's: that block's eigenvalues are then taken as zero
+ * tridiagonal with this library's Householder kernels (in registers up to
+ * order 3072 real, 1792 complex; larger orders by panels down to that),
+ * solves the tridiagonal with this library's divide and conquer (rocSOLVER's
+ * past order 4032) and back-transforms only the eigenvectors the truncation
+ * keeps with this library's blocked compact-WY GEMMs.  For a real Gram matrix of order
+ * above 96, mode 1 checks the trailing block every 32 columns from column
+ * 64 on and stops the reduction one check after the first at which its
+ * Frobenius norm is at most 2e-15 of the Gram matrix's: that block's eigenvalues are then taken as zero
  * (they lie below the FP64 rounding of forming the Gram matrix), its trace
  * is counted as discarded weight, and the divide and conquer runs on the
  * reduced order; a split that would keep more values than the reduced
@@ -196,7 +197,7 @@ int dmrg_sym_eig(dmrg_ctx* ctx, int mode, double* A, int n, double* w, double* Z
  * complex: real plane then imaginary plane, plane stride n*n; overwritten):
  * w ascending, row k of Z (planar, same layout) the eigenvector of w[k].
  * mode 1 (the split's default): this library's reduction to a real
- * tridiagonal (zhetrd conventions), rocSOLVER dstedc and this library's
+ * tridiagonal (zhetrd conventions), its divide and conquer and its
  * blocked back-transformation; mode 2: the same with rocSOLVER zunmtr for
  * the back-transformation; mode 0: rocSOLVER zheevd.  The
  * eigensolver of the complex dmrg_svd_split exposed for its parity tests;
