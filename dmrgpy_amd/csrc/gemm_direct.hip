@@ -1,6 +1,6 @@
 // MFMA GEMM for complex products and for products with few output tiles (the
 // H_eff, environment and split GEMMs at small and mid bond dimensions): each
-// workgroup computes one 16 x 16 or 32 x 32 tile, its waves split the inner
+// workgroup computes one 16 x 16, 32 x 16 or 32 x 32 tile, its waves split the inner
 // dimension, and every wave loads its MFMA fragments straight from global
 // memory one k-step ahead, with no LDS staging and no barrier in the k-loop.
 // What bounds such a product is the chain of k-steps of the few workgroups it
@@ -15,10 +15,10 @@
 
 namespace dmrg {
 
-template <typename T, bool CX, int W, bool TA, bool TB, int TAG, typename CT>
+template <typename T, bool CX, int WM, int WN, bool TA, bool TB, int TAG, typename CT>
 __global__ __launch_bounds__(256) void gemm_direct(const T* __restrict__ A, const T* __restrict__ B,
                                                    CT* __restrict__ C, GemmArgs g) {
-  constexpr int WM = W, WN = W, TS = 16 * W, NP = CX ? 2 : 1;
+  constexpr int TM = 16 * WM, TN = 16 * WN, NP = CX ? 2 : 1;
   constexpr int STG = 2;   // k-steps of fragments per wave: one multiplied, one in flight
   typedef typename Mfma<T>::acc_t acc_t;
   extern __shared__ double smem[];
@@ -32,11 +32,11 @@ __global__ __launch_bounds__(256) void gemm_direct(const T* __restrict__ A, cons
   if (g.lower) {   // Hermitian C: row-major tiles, as every XCD then has an even share below the diagonal
     tr = blockIdx.x / g.nbx;
     tc = blockIdx.x % g.nbx;
-    if (tile_above_diagonal(tr, tc, TS, TS)) return;
+    if (tile_above_diagonal(tr, tc, TM, TN)) return;
   } else {
     xcd_tile_of(blockIdx.x, 0, g.nbx, g.nby, tr, tc);
   }
-  const int m0 = tr * TS, n0 = tc * TS;
+  const int m0 = tr * TM, n0 = tc * TN;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), KS = blockDim.x >> 6;
   const int li = lane & 15, lk = lane >> 4;
@@ -215,15 +215,15 @@ __global__ __launch_bounds__(256) void gemm_direct(const T* __restrict__ A, cons
       }
 }
 
-template <typename T, bool CX, int W, bool TA, bool TB, typename CT>
+template <typename T, bool CX, int WM, int WN, bool TA, bool TB, typename CT>
 static void launch_direct_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, int ks) {
-  constexpr int TS = 16 * W;
-  const GemmArgs g = make_args(d, TS, TS);
+  constexpr int TM = 16 * WM, TN = 16 * WN;
+  const GemmArgs g = make_args(d, TM, TN);
   const dim3 grid((unsigned)g.nbx * g.nby, 1, d.batch);
-  const size_t lds = (size_t)(ks / 2) * (CX ? 2 : 1) * TS * TS * sizeof(T);
+  const size_t lds = (size_t)(ks / 2) * (CX ? 2 : 1) * TM * TN * sizeof(T);
   switch (d.tag) {
 #define CASE(t) \
-  case t: gemm_direct<T, CX, W, TA, TB, t, CT><<<grid, 64 * ks, lds, c->stream>>>(A, B, C, g); break;
+  case t: gemm_direct<T, CX, WM, WN, TA, TB, t, CT><<<grid, 64 * ks, lds, c->stream>>>(A, B, C, g); break;
     DMRG_GEMM_TAGS(CASE)
 #undef CASE
     default: throw Error("gemm: bad tag");
@@ -231,29 +231,42 @@ static void launch_direct_tagged(Ctx* c, const GemmDesc& d, const T* A, const T*
   DMRG_CHECK_HIP(hipGetLastError());
 }
 
-template <typename T, bool CX, int W, typename CT>
+template <typename T, bool CX, int WM, int WN, typename CT>
 static void launch_direct_tt(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, int ks) {
-  if (!d.transA && !d.transB) launch_direct_tagged<T, CX, W, false, false, CT>(c, d, A, B, C, ks);
-  else if (d.transA && !d.transB) launch_direct_tagged<T, CX, W, true, false, CT>(c, d, A, B, C, ks);
-  else if (!d.transA && d.transB) launch_direct_tagged<T, CX, W, false, true, CT>(c, d, A, B, C, ks);
-  else launch_direct_tagged<T, CX, W, true, true, CT>(c, d, A, B, C, ks);
+  if (!d.transA && !d.transB) launch_direct_tagged<T, CX, WM, WN, false, false, CT>(c, d, A, B, C, ks);
+  else if (d.transA && !d.transB) launch_direct_tagged<T, CX, WM, WN, true, false, CT>(c, d, A, B, C, ks);
+  else if (!d.transA && d.transB) launch_direct_tagged<T, CX, WM, WN, false, true, CT>(c, d, A, B, C, ks);
+  else launch_direct_tagged<T, CX, WM, WN, true, true, CT>(c, d, A, B, C, ks);
 }
 
-// Tile and split.  16 x 16 tiles up to 192 tiles of 32 x 32 (256 x 64 x 320:
-// 5 us against 10; 256 x 256 x 1024: 11 against 21; 760 x 187 x 935: 18.4
-// against 19.8), 32 x 32 above (1024 x 256 x 1280: 24 against 33).  Four
-// waves share a tile's inner dimension where tiles are few or the dimension
-// long (complex 2259 x 256 x 1280: 137 us against 172 with one wave per tile;
-// 8 waves were no faster anywhere), one wave otherwise (complex
-// 2400 x 6400 x 400: 759 against 831).
+// Tile and split.  Four waves share a tile's inner dimension where tiles are
+// few or the dimension long (complex 2259 x 256 x 1280: 137 us against 172
+// with one wave per tile; 8 waves were no faster anywhere), one wave otherwise
+// (complex 2400 x 6400 x 400: 759 against 831, on 32 x 32 tiles).
+// Up to 192 tiles of 32 x 32 the time is the latency of one tile's chain, and
+// 16 x 16 is shortest (256 x 64 x 320: 5 us against 10; 256 x 256 x 1024: 11
+// against 21; 760 x 187 x 935: 18.5 against 20).  Above, four waves fill a
+// CU's matrix cores, so the time goes by rounds of the 256 CUs times the
+// tile's size; smaller tiles load more per MFMA, 1.1 and 1.25 times the time
+// per area.  Measured (us, 32 x 32 / 32 x 16 / 16 x 16):
+//   complex  2259 x 256 x 1280  150 / 129 / 131    1620 x 180 x 900  76 / 58 / 54
+//            600^3               52 /  41 /  45    3600 x 400 x 2000 404 / 439 / 473
+//            256 x 256 x 768 x 5 61 /  52 /  47
+//   FP64     1024 x 256 x 1280   22 /  30 /  34    650^3             24 / 28 / 29
+//   FP32     2400 x 150 x 900    21 /  18 /  19
 template <typename T, bool CX, typename CT>
 static void launch_direct(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C) {
-  const long long tiles = (long long)((d.M + 31) / 32) * ((d.N + 31) / 32) * d.batch;
+  auto tiles = [&](int tm, int tn) { return (long long)((d.M + tm - 1) / tm) * ((d.N + tn - 1) / tn) * d.batch; };
+  auto rounds = [&](int tm, int tn) { return (double)((tiles(tm, tn) + 255) / 256); };
   const int steps = (d.K + 15) / 16;
-  int ks = tiles < 1024 || d.K >= 800 ? 4 : 1;
+  int ks = tiles(32, 32) < 1024 || d.K >= 800 ? 4 : 1;
+  const bool one = ks == 1;
   while (ks > 1 && steps < ks) ks >>= 1;
-  if (tiles <= 192) launch_direct_tt<T, CX, 1, CT>(c, d, A, B, C, ks);
-  else launch_direct_tt<T, CX, 2, CT>(c, d, A, B, C, ks);
+  const double c22 = 2.0 * rounds(32, 32), c21 = 1.1 * rounds(32, 16), c11 = 0.625 * rounds(16, 16);
+  if (tiles(32, 32) <= 192) launch_direct_tt<T, CX, 1, 1, CT>(c, d, A, B, C, ks);
+  else if (one || (c22 <= c21 && c22 <= c11)) launch_direct_tt<T, CX, 2, 2, CT>(c, d, A, B, C, ks);
+  else if (c21 <= c11) launch_direct_tt<T, CX, 2, 1, CT>(c, d, A, B, C, ks);
+  else launch_direct_tt<T, CX, 1, 1, CT>(c, d, A, B, C, ks);
 }
 
 void gemm_direct_f64(Ctx* c, const GemmDesc& d, const double* A, const double* B, double* C) {
