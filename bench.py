@@ -750,7 +750,7 @@ def main():
         out["roofline_tridiagonalisation"] = {
             "bound": "hbm", "achieved": gbs, "peak": 8000.0, "unit": "GB/s", "frac": gbs / 8000.0, "traffic": None,
             "algorithmic_bytes": res["trd_bytes"] / res["trd_calls"],
-            "kernel": "own Householder tridiagonalisation of the Gram matrices (trd_col_k + trd_symv_k per column, "
+            "kernel": "own Householder tridiagonalisation of the Gram matrices (in registers up to order 3072, one exchange per column; "
                       "panel GEMMs), {} reductions per sweep, {:.2f} ms average, {:.2f} s per sweep".format(
                           int(res["trd_calls"] / args.steps), res["trd_ms"] / res["trd_calls"],
                           res["trd_ms"] / 1e3 / args.steps)}
