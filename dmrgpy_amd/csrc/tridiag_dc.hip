@@ -26,6 +26,7 @@
 // ms here.  Blocks of at most 12: QL runs about 0.4 us per rotation, 418 us
 // for blocks of 32, 38 for 8, and a level of merges costs 30.
 #include "dmrg_internal.h"
+#include "secular_root.h"
 #include "wave_reduce.h"
 
 #include <algorithm>
@@ -338,11 +339,7 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
   }
 }
 
-// Root j of 1/rho + sum_i z_i^2 / (d_i - x): between poles j and j + 1 (the last
-// one past the last pole), as the distance tau from the nearer pole, so that
-// every difference d_i - x is formed without cancellation.  Two-pole rational
-// steps (the weights of Li's middle way) inside a bracket, bisection where a
-// step leaves it.
+// Every root of the secular equation (secular_root.h), one wave per root
 __global__ __launch_bounds__(256) void dc_secular_k(DcLevel L) {
   const int m = blockIdx.y, lane = threadIdx.x & 63;
   const int j = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -353,71 +350,31 @@ __global__ __launch_bounds__(256) void dc_secular_k(DcLevel L) {
   const double* zl = L.zl + o;
   const double rinv = 0.5 / fabs(L.e[m * L.N + L.S - 1] / L.scale[0]);
   const bool end = j == K - 1;
-  double psi, dpsi, phi, dphi, f;
-  double origin = dl[j];
-  auto eval = [&](double tau) {   // psi, phi: poles up to j, past j
-    psi = dpsi = phi = dphi = 0.0;
+  double z2 = 0.0;
+  if (end) {
+    double u1 = 0.0, u2 = 0.0, u3 = 0.0;
+    for (int i = lane; i < K; i += 64) z2 += zl[i] * zl[i];
+    wave_sums4(z2, u1, u2, u3);
+  }
+  const int jn = end ? j : j + 1;
+  const SecularRoot r = secular_root(end, dl[j], dl[jn], zl[j], zl[jn], z2, rinv, [&](double origin, double tau) {
+    SecularSums s = {0.0, 0.0, 0.0, 0.0};
     for (int i = lane; i < K; i += 64) {
       const double z = zl[i], t = z / ((dl[i] - origin) - tau);
       if (i <= j) {
-        psi += z * t;
-        dpsi += t * t;
+        s.psi += z * t;
+        s.dpsi += t * t;
       } else {
-        phi += z * t;
-        dphi += t * t;
+        s.phi += z * t;
+        s.dphi += t * t;
       }
     }
-    wave_sums4(psi, dpsi, phi, dphi);
-    f = rinv + psi + phi;
-  };
-  int org = j;
-  double lo = 0.0, hi, tau;
-  if (end) {
-    double z2 = 0.0, u1 = 0.0, u2 = 0.0, u3 = 0.0;
-    for (int i = lane; i < K; i += 64) z2 += zl[i] * zl[i];
-    wave_sums4(z2, u1, u2, u3);
-    hi = z2 / rinv;
-    tau = 0.5 * hi;
-    eval(tau);
-    hi *= 1.0 + 16.0 * DC_EPS;
-  } else {
-    const double gap = dl[j + 1] - dl[j];
-    tau = 0.5 * gap;
-    hi = tau;
-    eval(tau);
-    if (f < 0.0) {   // nearer the right pole
-      org = j + 1;
-      origin = dl[j + 1];
-      lo = -tau;
-      hi = 0.0;
-      tau = -tau;
-    }
-  }
-  for (int it = 0; it < 50; ++it) {
-    if (!(fabs(f) > 8.0 * DC_EPS * (rinv + fabs(psi) + fabs(phi)))) break;
-    if (f < 0.0) lo = fmax(lo, tau);
-    else hi = fmin(hi, tau);
-    const double dj = (dl[j] - origin) - tau;
-    double next;
-    if (end) {   // one pole with the slope of all
-      const double c = f - dpsi * dj;
-      next = tau + dj + dpsi * dj * dj / c;
-    } else {
-      const double dk = (dl[j + 1] - origin) - tau;
-      const double c = f - dj * dpsi - dk * dphi;
-      const double a = (dj + dk) * f - dj * dk * (dpsi + dphi);
-      const double b = dj * dk * f;
-      const double disc = sqrt(fabs(a * a - 4.0 * b * c));
-      next = tau + (a <= 0.0 ? (a - disc) / (2.0 * c) : 2.0 * b / (a + disc));
-    }
-    if (!(next > lo && next < hi) || (it >= 15 && (it & 1))) next = 0.5 * (lo + hi);
-    if (next == tau) break;
-    tau = next;
-    eval(tau);
-  }
+    wave_sums4(s.psi, s.dpsi, s.phi, s.dphi);
+    return s;
+  });
   if (lane == 0) {
-    L.tau[o + j] = tau;
-    L.org[o + j] = org;
+    L.tau[o + j] = r.tau;
+    L.org[o + j] = j + r.next;
   }
 }
 
