@@ -87,10 +87,11 @@ void trd_single(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
                 double* dropped);
 int trd_single_max();
 // Divide and conquer on a real symmetric tridiagonal matrix (tridiag_dc.hip):
-// eigenvalues ascending into w (w may be d), then the rows of Zt (keep x n,
+// eigenvalues ascending into w (w may be d) and *info (device) nonzero where
+// they could not be found (NaN or infinity in d or e among the causes), then the rows of Zt (keep x n,
 // pitch ldz) as the eigenvectors of the `keep` largest ones, ascending
 bool tridiag_dc_ok(int n);
-void tridiag_dc_values(Ctx* c, int n, const double* d, const double* e, double* w);
+void tridiag_dc_values(Ctx* c, int n, const double* d, const double* e, double* w, int* info);
 void tridiag_dc_vectors(Ctx* c, int n, const double* e, int keep, double* Zt, int ldz);
 // rows of Zt (keep x n, row-major: eigenvectors of the tridiagonal) <- rows
 // of Q Y for the first nrefl reflectors sytrd_lower left in A (all n - 1 by

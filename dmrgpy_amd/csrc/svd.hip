@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "dmrg_internal.h"
 #include "keep_rule.h"
@@ -403,7 +404,7 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
   double* ev = (double*)ws_get(c, WS_SVD_EV, sizeof(double) * (2 * (size_t)g + 16));
   double* ework = ev + g;
   double* amax_dev = ev + 2 * (size_t)g + 8;
-  rocblas_int* info = (rocblas_int*)ws_get(c, WS_SVD_INFO, 64);
+  rocblas_int* info = (rocblas_int*)(amax_dev + 1);   // beside max|M|: one copy brings both to the host
   double* Gsolve = nullptr;
   double *trd_Z = nullptr, *trd_tau = nullptr, *trd_refl = nullptr, *trd_Zs = nullptr;
   int trd_nrefl = g - 1, trd_m = g;   // reflectors computed, order of the tridiagonal solved
@@ -415,7 +416,7 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
   auto solve_tridiagonal = [&]() {
     own_dc = tridiag_dc_ok(trd_m);
     if (own_dc) {
-      tridiag_dc_values(c, trd_m, ev, ework, ev);
+      tridiag_dc_values(c, trd_m, ev, ework, ev, info);
     } else if (trd_m < g) {
       trd_Zs = (double*)ws_get(c, WS_TRD_ZS, sizeof(double) * (size_t)trd_m * trd_m);
       check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, trd_m, ev, ework, trd_Zs, trd_m, info), "dstedc");
@@ -483,16 +484,17 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
     }
   }
   std::vector<double> evh(g, 0.0);
-  int hinfo = 0;
-  double hmax = 0.0;
+  double hm[2] = {0.0, 0.0};
   // ascending; a reduction that stopped early leaves g - trd_m exact zeros
   // below the trd_m computed values
   DMRG_CHECK_HIP(hipMemcpyAsync(evh.data() + (g - trd_m), ev, sizeof(double) * trd_m, hipMemcpyDeviceToHost,
                                 c->stream));
-  if (!own_dc) DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  DMRG_CHECK_HIP(hipMemcpyAsync(&hmax, amax_dev, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  DMRG_CHECK_HIP(hipMemcpyAsync(hm, amax_dev, sizeof(hm), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  DMRG_REQUIRE(hinfo == 0, "syevd/heevd did not converge");
+  int hinfo;
+  std::memcpy(&hinfo, &hm[1], sizeof(hinfo));
+  DMRG_REQUIRE(hinfo == 0, "svd: the Gram eigenproblem did not converge (NaN or infinity in the matrix?)");
+  const double hmax = hm[0];
   const double scale = hmax > 0.0 ? hmax : 1.0;
   svals.resize(rank);
   for (int i = 0; i < rank; ++i) svals[i] = scale * std::sqrt(std::max(evh[g - 1 - i], 0.0));
@@ -951,7 +953,7 @@ int sym_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
     sytrd_lower(c, A, n, w, ework, tauv);
     own_dc = tridiag_dc_ok(n);
     if (own_dc) {
-      tridiag_dc_values(c, n, w, ework, w);
+      tridiag_dc_values(c, n, w, ework, w, info);
       tridiag_dc_vectors(c, n, ework, n, Z, n);
     } else {
       check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, n, w, ework, Z, n, info), "dstedc");
@@ -968,7 +970,7 @@ int sym_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
     DMRG_CHECK_HIP(hipMemcpyAsync(Z, A, sizeof(double) * n * n, hipMemcpyDeviceToDevice, c->stream));
   }
   int hinfo = 0;
-  if (!own_dc) DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
   DMRG_REQUIRE(hinfo == 0, "sym_eig: eigensolver did not converge");
   return 0;
@@ -994,7 +996,7 @@ int herm_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
     hetrd_lower(c, A, n, w, ework, tauv);
     own_dc = tridiag_dc_ok(n);
     if (own_dc) {
-      tridiag_dc_values(c, n, w, ework, w);
+      tridiag_dc_values(c, n, w, ework, w, info);
       tridiag_dc_vectors(c, n, ework, n, Zr, n);
     } else {
       check_rb(rocsolver_dstedc(c->blas, rocblas_evect_tridiagonal, n, w, ework, Zr, n, info), "dstedc");
@@ -1025,7 +1027,7 @@ int herm_eig_entry(Ctx* c, int mode, double* A, int n, double* w, double* Z) {
   inter_to_planar_conj_k<<<g1(nn), 256, 0, c->stream>>>(Zc, nn, Z);
   DMRG_CHECK_HIP(hipGetLastError());
   int hinfo = 0;
-  if (!own_dc) DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  DMRG_CHECK_HIP(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
   DMRG_REQUIRE(hinfo == 0, "herm_eig: eigensolver did not converge");
   return 0;

@@ -25,6 +25,9 @@
 // 480 us per level in its secular equations), against 0.15 / 0.2 / 0.4 / 0.4
 // ms here.  Blocks of at most 12: QL runs about 0.4 us per rotation, 418 us
 // for blocks of 32, 38 for 8, and a level of merges costs 30.
+//
+// A NaN or infinity in the matrix, or an iteration that runs out of steps, is
+// reported through a status word and leaves every eigenvalue NaN.
 #include "dmrg_internal.h"
 #include "secular_root.h"
 #include "wave_reduce.h"
@@ -35,6 +38,7 @@ namespace dmrg {
 
 constexpr int DC_LEAF = 12, DC_MAX = 4096;
 constexpr double DC_EPS = 1.1102230246251565e-16;   // 2^-53
+constexpr double DC_FAIL = 1e-10;                    // relative residual of a root that was not found
 constexpr double DC_PAD = -3.5;                      // below every eigenvalue of the scaled matrix (|lambda| <= 3)
 
 // One level's merges; every array holds `merges` rows of N entries (N = 2 S)
@@ -57,6 +61,7 @@ struct DcLevel {
   int *ichain, *ipos;          // index -> first rotation of its chain (-1: none), position in it
   int* col;                    // ascending position -> survivor j or N + deflated k
   int *K, *nrot;               // per merge
+  int* stat;                   // [blocks] nonzero: failed
 };
 
 // ---------------------------------------------------------------------------
@@ -65,13 +70,26 @@ struct DcLevel {
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, const double* __restrict__ e, int n,
                                                 int B, double* __restrict__ D, double* __restrict__ Q,
-                                                double* __restrict__ scale) {
+                                                double* __restrict__ scale, int* __restrict__ stat) {
   __shared__ double sd[DC_LEAF], se[DC_LEAF + 1], Z[DC_LEAF][DC_LEAF + 1];
   const int lane = threadIdx.x, b0 = blockIdx.x * B;
   double mx = 0.0;
+  bool finite = true;
   for (int i = lane; i < n; i += 64) {
     mx = fmax(mx, fabs(d[i]));
-    if (i < n - 1) mx = fmax(mx, fabs(e[i]));
+    finite &= isfinite(d[i]);
+    if (i < n - 1) {
+      mx = fmax(mx, fabs(e[i]));
+      finite &= isfinite(e[i]);
+    }
+  }
+  if (__any(!finite)) {   // in every block alike
+    if (lane < B) D[b0 + lane] = __builtin_nan("");
+    if (lane == 0) {
+      stat[blockIdx.x] = 1;
+      if (blockIdx.x == 0) scale[0] = 1.0;
+    }
+    return;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
@@ -94,14 +112,17 @@ __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, co
     for (int k = 0; k < B; ++k) Z[lane][k] = k == lane ? 1.0 : 0.0;
   }
   __syncthreads();
+  bool failed = false;
   for (int l = 0; l < B; ++l) {
+    bool found = false;
     for (int iter = 0; iter < 60; ++iter) {
       int m = l;
       for (; m < B - 1; ++m) {
         const double t = fabs(sd[m]) + fabs(sd[m + 1]);
         if (fabs(se[m]) <= DC_EPS * t) break;
       }
-      if (m == l) break;
+      found = m == l;
+      if (found) break;
       double p = (sd[l + 1] - sd[l]) / (2.0 * se[l]);
       double r = sqrt(p * p + 1.0);
       if (!(fabs(p) < 1e150)) r = fabs(p);
@@ -145,7 +166,9 @@ __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, co
       }
       __syncthreads();
     }
+    failed |= !found;
   }
+  if (lane == 0) stat[blockIdx.x] = failed;
   // ascending order by rank
   if (lane < B) {
     const double x = sd[lane];
@@ -373,6 +396,7 @@ __global__ __launch_bounds__(256) void dc_secular_k(DcLevel L) {
     return s;
   });
   if (lane == 0) {
+    if (!(r.residual < DC_FAIL)) L.stat[0] = 1;   // not found: the iteration's own ends leave a rounding's worth
     L.tau[o + j] = r.tau;
     L.org[o + j] = j + r.next;
   }
@@ -471,11 +495,17 @@ __global__ __launch_bounds__(256) void dc_vectors_k(DcLevel L, int first, int ro
   }
 }
 
-// eigenvalues past the padding, scaled back
-__global__ void dc_values_k(const double* __restrict__ lam, int np, int n, const double* __restrict__ scale,
-                            double* __restrict__ w) {
+// eigenvalues past the padding, scaled back (all NaN after a failure), and the
+// status of the whole solve
+__global__ __launch_bounds__(256) void dc_values_k(const double* __restrict__ lam, int np, int n,
+                                                   const double* __restrict__ scale, double* __restrict__ w,
+                                                   const int* __restrict__ stat, int blocks, int* __restrict__ info) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) w[i] = lam[np - n + i] * scale[0];
+  int bad = 0;
+  for (int b = threadIdx.x; b < blocks; b += 256) bad |= stat[b];
+  bad = __syncthreads_or(bad);
+  if (i < n) w[i] = bad ? __builtin_nan("") : lam[np - n + i] * scale[0];
+  if (i == 0) *info = bad;
 }
 
 // Zt[r][i] = Q[i][first + r]: the vectors of a matrix that is one block
@@ -493,6 +523,9 @@ static size_t dc_deflate_lds(int N) {
 }
 
 bool tridiag_dc_ok(int n) { return n >= 1 && n <= DC_MAX - 64; }
+
+// [Q ping][Q pong][Ut][D ping][D pong][arrays of a level][scale][status of up to 512 blocks]
+static size_t dc_ws_bytes(int np) { return sizeof(double) * (3 * (size_t)np * np + 18 * (size_t)np + 64 + 256); }
 
 static DcLevel dc_level(int n, const double* e, int S, double* ws, int np) {
   DcLevel L;
@@ -512,27 +545,30 @@ static DcLevel dc_level(int n, const double* e, int S, double* ws, int np) {
 
 // Eigenvalues (ascending, into w[n], device) of the tridiagonal matrix d, e
 // (device, read only); keeps what tridiag_dc_vectors needs in the context's
-// workspace.
-void tridiag_dc_values(Ctx* c, int n, const double* d, const double* e, double* w) {
+// workspace.  *info (device): 0, or 1 when the matrix holds NaN or infinity or
+// an iteration did not converge.
+void tridiag_dc_values(Ctx* c, int n, const double* d, const double* e, double* w, int* info) {
   DMRG_REQUIRE(tridiag_dc_ok(n), "tridiag_dc: order out of range");
   int levels = 0;
   while ((DC_LEAF << levels) < n) ++levels;
   const int blocks = 1 << levels, B = (n + blocks - 1) / blocks, np = B * blocks;
-  // [Q ping][Q pong][Ut][D ping][D pong][arrays of a level][scale]
   const size_t nq = (size_t)np * np;
-  double* ws = (double*)ws_get(c, WS_TRD_DC, sizeof(double) * (3 * nq + 18 * (size_t)np + 64));
+  double* ws = (double*)ws_get(c, WS_TRD_DC, dc_ws_bytes(np));
   double* Q[2] = {ws, ws + nq};
   double* Ut = Q[1] + nq;
   double* D[2] = {Ut + nq, Ut + nq + np};
   double* arr = D[1] + np;
   double* scale = arr + 16 * (size_t)np;
-  dc_leaf_k<<<blocks, 64, 0, c->stream>>>(d, e, n, B, D[0], Q[0], scale);
+  int* stat = (int*)(scale + 64);
+  DMRG_REQUIRE(blocks <= 512, "tridiag_dc: too many blocks");
+  dc_leaf_k<<<blocks, 64, 0, c->stream>>>(d, e, n, B, D[0], Q[0], scale, stat);
   DMRG_CHECK_HIP(hipGetLastError());
   int cur = 0;
   for (int l = 0; l < levels; ++l) {
     const int S = B << l, N = 2 * S, merges = blocks >> (l + 1);
     DcLevel L = dc_level(n, e, S, arr, np);
     L.scale = scale;
+    L.stat = stat;
     L.D = D[cur];
     L.Q = Q[cur];
     L.lam = D[cur ^ 1];
@@ -560,7 +596,7 @@ void tridiag_dc_values(Ctx* c, int n, const double* d, const double* e, double* 
     }
     cur ^= 1;
   }
-  dc_values_k<<<(n + 255) / 256, 256, 0, c->stream>>>(D[cur], np, n, scale, w);
+  dc_values_k<<<(n + 255) / 256, 256, 0, c->stream>>>(D[cur], np, n, scale, w, stat, blocks, info);
   DMRG_CHECK_HIP(hipGetLastError());
   c->dc_n = n;
 }
@@ -573,7 +609,7 @@ void tridiag_dc_vectors(Ctx* c, int n, const double* e, int keep, double* Zt, in
   while ((DC_LEAF << levels) < n) ++levels;
   const int blocks = 1 << levels, B = (n + blocks - 1) / blocks, np = B * blocks;
   const size_t nq = (size_t)np * np;
-  double* ws = (double*)ws_get(c, WS_TRD_DC, sizeof(double) * (3 * nq + 18 * (size_t)np + 64));
+  double* ws = (double*)ws_get(c, WS_TRD_DC, dc_ws_bytes(np));
   double* Q[2] = {ws, ws + nq};
   double* Ut = Q[1] + nq;
   double* arr = Ut + nq + 2 * (size_t)np;
