@@ -38,6 +38,12 @@ namespace dmrg {
 
 constexpr int DC_LEAF = 12, DC_MAX = 4096;
 constexpr double DC_EPS = 1.1102230246251565e-16;   // 2^-53
+// Couplings of the scaled matrix below this are taken as zero (a part that far
+// below the rest is diagonal then), and poles or weights of a merge below
+// DC_FLOOR of its size are deflated.  A root then lies at least 1e-120 of the
+// merge's size from its pole, so that the squares of z / (d - x), at most
+// 1e300, stay in range.
+constexpr double DC_TINY = 1e-70, DC_FLOOR = 1e-40;
 constexpr double DC_FAIL = 1e-10;                    // relative residual of a root that was not found
 constexpr double DC_PAD = -3.5;                      // below every eigenvalue of the scaled matrix (|lambda| <= 3)
 
@@ -63,6 +69,11 @@ struct DcLevel {
   int *K, *nrot;               // per merge
   int* stat;                   // [blocks] nonzero: failed
 };
+
+__device__ __forceinline__ double dc_coupling(double e, double scale) {
+  const double x = e / scale;
+  return fabs(x) < DC_TINY ? 0.0 : x;
+}
 
 // ---------------------------------------------------------------------------
 // Blocks: implicit QL with shifts, one wave per block.  Every lane runs the
@@ -93,13 +104,13 @@ __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, co
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-  const double sc = mx > 0.0 ? mx : 1.0, inv = 1.0 / sc;
+  const double sc = mx > 0.0 ? mx : 1.0;
   if (blockIdx.x == 0 && lane == 0) scale[0] = sc;
-  auto off = [&](int i) { return i >= 0 && i < n - 1 ? e[i] * inv : 0.0; };   // coupling of i and i + 1
+  auto off = [&](int i) { return i >= 0 && i < n - 1 ? dc_coupling(e[i], sc) : 0.0; };   // of i and i + 1
   // a block graded downwards is turned upside down: QL keeps the small
   // eigenvalues' accuracy when the small entries come first
   auto diag = [&](int i) {
-    double x = i < n ? d[i] * inv : DC_PAD;
+    double x = i < n ? d[i] / sc : DC_PAD;
     if (i == b0) x -= fabs(off(b0 - 1));               // tearing at the block's two ends
     if (i == b0 + B - 1) x -= fabs(off(b0 + B - 1));
     return x;
@@ -132,8 +143,15 @@ __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, co
       for (int i = m - 1; i >= l; --i) {
         const double f = s * se[i], bb = c * se[i];
         const double di1 = sd[i + 1], di = sd[i];
-        const double r2 = f * f + gg * gg, rin = r2 > 0.0 ? rsqrt(r2) : 0.0;
-        r = r2 * rin;
+        double fu = f, gu = gg, dn = 1.0, r2 = f * f + gg * gg;
+        if (r2 < 1e-280) {   // squares out of range: by a power of two
+          fu *= 0x1p500;
+          gu *= 0x1p500;
+          dn = 0x1p-500;
+          r2 = fu * fu + gu * gu;
+        }
+        const double rin = r2 > 0.0 ? rsqrt(r2) : 0.0;
+        r = r2 * rin * dn;
         __syncthreads();   // every lane has read what lane 0 now replaces
         if (lane == 0) se[i + 1] = r;
         if (r == 0.0) {
@@ -145,8 +163,8 @@ __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, co
           __syncthreads();
           break;
         }
-        s = f * rin;
-        c = gg * rin;
+        s = fu * rin;
+        c = gu * rin;
         const double h = di1 - q;
         const double t = (di - h) * s + 2.0 * c * bb;
         q = s * t;
@@ -196,9 +214,9 @@ __device__ __forceinline__ int block_rank(bool flag, int& base, int* sh) {
 }
 
 // Two poles p < n too close to tell apart: rotating z_p away leaves an
-// off-diagonal entry below the rounding of the two poles themselves
-__device__ __forceinline__ bool dc_close(double dp, double zp, double dn, double zn) {
-  return fabs((dn - dp) * zp * zn) <= DC_EPS * (fabs(dp) + fabs(dn)) * (zp * zp + zn * zn);
+// off-diagonal entry below the rounding of the two poles themselves, or the floor
+__device__ __forceinline__ bool dc_close(double dp, double zp, double dn, double zn, double floor) {
+  return fabs((dn - dp) * zp * zn) <= (DC_EPS * (fabs(dp) + fabs(dn)) + floor) * (zp * zp + zn * zn);
 }
 
 __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
@@ -216,7 +234,7 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
   const double* Q1 = L.Q + (size_t)(2 * m) * S * S;
   const double* Q2 = Q1 + (size_t)S * S;
   const int cut = m * N + S;   // first row of the lower block
-  const double beta = cut < L.n ? L.e[cut - 1] / L.scale[0] : 0.0;
+  const double beta = cut < L.n ? dc_coupling(L.e[cut - 1], L.scale[0]) : 0.0;
   const double rho = 2.0 * fabs(beta), sg = beta < 0.0 ? -0.70710678118654752440 : 0.70710678118654752440;
   for (int i = tid; i < N; i += 256) {   // every slot valid whatever the values (NaN) do to the order
     sd[i] = sz[i] = 0.0;
@@ -255,14 +273,13 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
   // Deflation is relative to the pole it concerns, not to the matrix norm as
   // in LAPACK: Gram matrices are graded, and their small eigenvalues (the
   // ones a truncation decides on) keep their own accuracy.  It costs little
-  // here, where the products take the full order anyway; the floor keeps z^2
-  // from underflowing.
-  const double floor_z = 1e-40 * md;
+  // here, where the products take the full order anyway.
+  const double floor = DC_FLOOR * fmax(md, rho);
   // ---- poles the update hardly touches
   int nc = 0, nd = 0;
   for (int b = 0; b < N; b += 256) {
     const int i = b + tid;
-    const bool in = i < N, cand = in && rho * fabs(sz[in ? i : 0]) > fmax(DC_EPS * fabs(sd[in ? i : 0]), floor_z);
+    const bool in = i < N, cand = in && rho * fabs(sz[in ? i : 0]) > fmax(DC_EPS * fabs(sd[in ? i : 0]), floor);
     const int c0 = block_rank(cand, nc, sh);
     const int d0 = block_rank(in && !cand, nd, sh);
     if (cand) sc[c0] = i;
@@ -277,7 +294,7 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
   // rotated one after the other (a rotation changes the pair that follows it)
   for (int b = 0; b < nc; b += 256) {
     const int j = b + tid;
-    const bool f = j > 0 && j < nc && dc_close(sd[sc[j - 1]], sz[sc[j - 1]], sd[sc[j]], sz[sc[j]]);
+    const bool f = j > 0 && j < nc && dc_close(sd[sc[j - 1]], sz[sc[j - 1]], sd[sc[j]], sz[sc[j]], floor);
     const unsigned long long w = __ballot(f);
     if ((tid & 63) == 0) fl[j >> 6] = w;
   }
@@ -295,7 +312,7 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
         const int base = nr;
         while (j < nc) {
           const int a = sc[j - 1], b = sc[j];
-          if (!dc_close(sd[a], sz[a], sd[b], sz[b])) break;
+          if (!dc_close(sd[a], sz[a], sd[b], sz[b], floor)) break;
           const double t = sqrt(sz[a] * sz[a] + sz[b] * sz[b]);
           const double c = sz[b] / t, s = -sz[a] / t;
           const double da = sd[a], db = sd[b];
