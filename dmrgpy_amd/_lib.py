@@ -58,6 +58,8 @@ SIGNATURES = {
                                       c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int, P_int, P_double,
                                       P_double, P_int, P_double]),
     "dmrg_set_eigensolver": (c_int, [c_void_p, c_int]),
+    "dmrg_set_reduction": (c_int, [c_void_p, c_int, c_double]),
+    "dmrg_reduction_counts": (c_int, [c_void_p, P_ll]),
     "dmrg_sym_eig": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p]),
     "dmrg_herm_eig": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p]),
     "dmrg_mpo_grad": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,

@@ -318,6 +318,22 @@ int dmrg_set_eigensolver(dmrg_ctx* ctx, int mode) {
   API_END
 }
 
+int dmrg_set_reduction(dmrg_ctx* ctx, int in_registers, double wait_ms) {
+  API_BEGIN
+  DMRG_REQUIRE(ctx, "set_reduction: null context");
+  DMRG_REQUIRE(wait_ms >= 0.0 && wait_ms <= 1000.0, "set_reduction: the wait must be 0 to 1000 ms");
+  ctx->c.trd_registers = in_registers != 0;
+  ctx->c.trd_wait = (long long)(wait_ms * 1e5);
+  API_END
+}
+
+int dmrg_reduction_counts(dmrg_ctx* ctx, long long* counts) {
+  API_BEGIN
+  DMRG_REQUIRE(ctx && counts, "reduction_counts: null argument");
+  for (int i = 0; i < 4; ++i) counts[i] = ctx->c.trd_counts[i];
+  API_END
+}
+
 int dmrg_sym_eig(dmrg_ctx* ctx, int mode, double* A, int n, double* w, double* Z) {
   API_BEGIN
   DMRG_REQUIRE(ctx && A && w && Z, "sym_eig: null argument");

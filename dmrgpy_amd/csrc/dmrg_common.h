@@ -106,6 +106,12 @@ struct Ctx {
   // with rocSOLVER ormtr / unmtr for the back-transformation; 0 = rocSOLVER
   // syevd / heevd
   int eig_mode = 1;
+  // tridiagonalisation: in-register reductions allowed, the longest wait of one
+  // for its workgroups in wall-clock ticks (100 MHz), and how reductions ran:
+  // one workgroup, across workgroups, given up, by panels
+  bool trd_registers = true;
+  long long trd_wait = 5000000;
+  long long trd_counts[4] = {0, 0, 0, 0};
   int dc_n = 0;   // order of the tridiagonal whose divide and conquer the workspace holds
   hipEvent_t trd_ev[2] = {nullptr, nullptr};   // early-stop checks of the reduction in flight
   // allocation-free calls (dmrg_heff_apply_noalloc): while `noalloc` is set,

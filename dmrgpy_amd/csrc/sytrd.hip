@@ -3,7 +3,8 @@
 // to 128 are reduced by one workgroup (trd_single.hip), other orders whose rows
 // fit the register files (real 3072, complex 1792) across workgroups in one
 // launch (trd_resident.hip); this path reduces larger matrices down to that
-// order by panels, and any order when the resident kernel gives up.
+// order by panels, and any order when the resident kernel gives up or the
+// context asks for panels only.
 //
 // The dense symmetric eigensolver behind every Gram-route split spends most
 // of its time reducing the matrix to tridiagonal form, one column at a time.
@@ -441,8 +442,9 @@ static double trailing_sumsq_wait(Ctx* c, int slot) {
 constexpr int TRD_STOP_MIN = 64;
 int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, double stop_tol, double* dropped) {
   DMRG_REQUIRE(n >= 2, "sytrd: order must be at least 2");
-  if (n <= trd_single_max()) {   // one workgroup holds the matrix (trd_single.hip)
+  if (c->trd_registers && n <= trd_single_max()) {   // one workgroup holds the matrix (trd_single.hip)
     ProfScope ps(c, 4, 0.0, 0.0);
+    ++c->trd_counts[0];
     int done = n - 1;
     trd_single(c, A, n, d, e, tau, n > TRD_STOP_MIN + TRD_NB ? stop_tol : 0.0, &done, dropped);
     if (done < n - 1) {
@@ -477,8 +479,8 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
   int pend = -1;      // slot of a trailing-norm check in flight
   // up to the order whose rows fit the register files the matrix is reduced
   // there (trd_resident.hip); larger ones by panels down to that order
-  bool resident = n <= trd_resident_max(REAL);
-  if (resident && trd_resident(c, REAL, A, n, 0, d, e, tau, early ? stop_tol : 0.0, -1.0, &done, dropped)) {
+  const bool fits = n <= trd_resident_max(REAL);
+  if (c->trd_registers && fits && trd_resident(c, REAL, A, n, 0, d, e, tau, early ? stop_tol : 0.0, -1.0, &done, dropped)) {
     if (done < n - 1) {
       trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 1);
       DMRG_CHECK_HIP(hipGetLastError());
@@ -486,13 +488,14 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
     for (int j = 0; j < done; ++j) ps.bytes += 8.0 * (double)(n - j - 1) * (n - j) / 2.0;
     return done;
   }
-  resident = !resident;   // try once
+  bool resident = c->trd_registers && !fits;   // to be tried once
   double total2 = 0.0;
   if (early) {
     trailing_sumsq_async(c, A, n, 0, 1, part1, sq_cap, sq_out, 0);
     total2 = trailing_sumsq_wait(c, 0);
     stop2 = stop_tol * stop_tol * total2;
   }
+  ++c->trd_counts[3];
   int g2prev = 1;
   bool in_registers = false;
   for (int j0 = 0; j0 < n - 1; j0 += TRD_NB) {
@@ -978,8 +981,8 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
   int done = n - 1;
   int pend = -1;
   // as in sytrd_lower: in registers where the order allows, panels down to it
-  bool resident = n <= trd_resident_max(CPLX);
-  if (resident && trd_resident(c, CPLX, A, n, 0, d, e, tau, early ? stop_tol : 0.0, -1.0, &done, dropped)) {
+  const bool fits = n <= trd_resident_max(CPLX);
+  if (c->trd_registers && fits && trd_resident(c, CPLX, A, n, 0, d, e, tau, early ? stop_tol : 0.0, -1.0, &done, dropped)) {
     if (done < n - 1) {
       trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 2);
       DMRG_CHECK_HIP(hipGetLastError());
@@ -987,13 +990,14 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
     for (int j = 0; j < done; ++j) ps.bytes += 16.0 * (double)(n - j - 1) * (n - j) / 2.0;
     return done;
   }
-  resident = !resident;   // try once
+  bool resident = c->trd_registers && !fits;   // to be tried once
   double total2 = 0.0;
   if (early) {
     trailing_sumsq_async(c, A, n, 0, 2, part1, sq_cap, sq_out, 0);
     total2 = trailing_sumsq_wait(c, 0);
     stop2 = stop_tol * stop_tol * total2;
   }
+  ++c->trd_counts[3];
   int g2prev = 1;
   bool in_registers = false;
   for (int j0 = 0; j0 < n - 1; j0 += TRD_NB) {

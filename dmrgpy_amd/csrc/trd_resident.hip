@@ -29,9 +29,9 @@
 // validity, so no fence, flag or cache write-back is needed.  Measured with
 // 16 / 32 / 64 / 128 / 256 workgroups exchanging 760 words: 1.6 / 2.1 / 2.5 /
 // 3.0 / 3.2 us.  All waits are bounded: a workgroup that waits longer than
-// the limit (other work holding the CUs its peers need) gives up, as then do
-// the others, the input is untouched and the caller runs the
-// launch-per-column reduction instead.
+// the context's limit (other work holding the CUs its peers need) gives up and
+// says so, the others leave their next long wait, the input is untouched and
+// the caller runs the launch-per-column reduction instead.
 //
 // Measured per column, launch-per-column / resident (us): real order 128
 // 8.7 / 2.45, 380 9.8 / 2.6, 2588 (930 columns reduced) 16.2 / 6.0; complex
@@ -48,7 +48,6 @@ namespace dmrg {
 
 constexpr unsigned long long RES_EMPTY = ~0ull;                  // a NaN no arithmetic produces; see publish()
 constexpr unsigned long long RES_NAN = 0x7FF8000000000000ull;
-constexpr long long RES_LIMIT = 5000000;                          // wall-clock ticks (100 MHz): 50 ms
 constexpr int RES_CHECK = 32, RES_CHECK_MIN = 64;                 // early-stop checks: every 32 columns from 64 on
 
 struct ResArgs {
@@ -62,6 +61,7 @@ struct ResArgs {
   double *d, *e, *tau;         // at col0 (tau interleaved when complex)
   int early;
   double tol2, total2;         // stop once |trailing|_F^2 <= tol2 * total2 (total2 < 0: of this matrix)
+  long long limit;             // longest wait, wall-clock ticks; 0: none, the first unmet word gives up
   int* status;                 // [0] 1 = gave up, [1] columns reduced
   double* trace;               // trace of the block left when stopped early
 };
@@ -75,18 +75,23 @@ __device__ __forceinline__ unsigned long long peek(const unsigned long long* p) 
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Words published by other workgroups, loaded in batches until all of a batch
-// are there; false after RES_LIMIT ticks
+// One wait for words published by other workgroups: over() after each look
+// that missed some; true once the limit has passed or another workgroup gave
+// up (workgroups that start late then leave at once, not after a limit each)
 struct Patience {
   int spin = 0;
   long long t0 = 0;
-  __device__ __forceinline__ bool over() {
+  __device__ __forceinline__ bool over(const ResArgs& g) {
+    if (g.limit == 0) return true;
     if ((++spin & 63) != 0) return false;
     const long long t = wall_clock64();
     if (t0 == 0) t0 = t;
-    return t - t0 > RES_LIMIT;
+    return t - t0 > g.limit || __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
   }
 };
+__device__ __forceinline__ void give_up(const ResArgs& g) {
+  __hip_atomic_store(g.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // T threads, thread t holds columns t, t + T, ... (CC of them) of RW rows.
 template <bool CX, int T, int CC, int RW>
@@ -304,7 +309,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
           y0 = peek(ck + o);
           y1 = peek(ck + G + o);
           if (y0 != RES_EMPTY && y1 != RES_EMPTY) break;
-          if (wait.over()) {
+          if (wait.over(g)) {
             s_bad = 1;
             break;
           }
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       const bool bad = s_bad != 0;
       __syncthreads();
       if (bad) {
-        if (tid == 0) g.status[0] = 1;
+        if (tid == 0) give_up(g);
         return;
       }
       if (first) {
@@ -426,7 +431,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
 #pragma unroll
           for (int k = 0; k < CC; ++k) miss |= uq[p][k] == RES_EMPTY;
         }
-        if (miss && wait.over()) ok = false;
+        if (miss && wait.over(g)) ok = false;
       } while (miss && ok);
       do {
         miss = false;
@@ -443,7 +448,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
               uc[p][k] = peek(Xc + p * mp + idx[k]);
             }
         }
-        if (miss && wait.over()) ok = false;
+        if (miss && wait.over(g)) ok = false;
       } while (miss && ok);
       if (!ok) s_bad = 1;
 #pragma unroll
@@ -483,7 +488,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
     }
     __syncthreads();
     if (s_bad) {
-      if (tid == 0) g.status[0] = 1;
+      if (tid == 0) give_up(g);
       return;
     }
     sr = si = 0.0;
@@ -590,6 +595,7 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
   g.early = stop_tol > 0.0 ? 1 : 0;
   g.tol2 = stop_tol * stop_tol;
   g.total2 = total2;
+  g.limit = c->trd_wait;
   trd_resident_fill_k<<<2048, 256, 0, c->stream>>>(g.X, nx, g.chk, nc, g.status, m);
   DMRG_CHECK_HIP(hipGetLastError());
   bool ok = false;
@@ -617,7 +623,11 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
   DMRG_CHECK_HIP(hipStreamSynchronize(c->stream));
   int st[2];
   std::memcpy(st, c->host_scalars + 36, sizeof(st));
-  if (st[0] != 0) return false;
+  if (st[0] != 0) {
+    ++c->trd_counts[2];
+    return false;
+  }
+  ++c->trd_counts[1];
   trd_resident_store_k<<<st[1], 256, 0, c->stream>>>(g.R, m, st[1], A + (long long)s0 * n + s0, n, g.pA, np);
   DMRG_CHECK_HIP(hipGetLastError());
   *done = s0 + st[1];

@@ -238,6 +238,19 @@ class Engine:
         back-transformation; 0: rocSOLVER syevd/heevd."""
         check(self.lib.dmrg_set_eigensolver(self.ctx, int(mode)), "dmrg_set_eigensolver")
 
+    def set_reduction(self, in_registers=True, wait_ms=50.0):
+        """Tridiagonalisation of the eigensolver: with the matrix in registers
+        where its order allows, or always by panels; wait_ms: how long
+        workgroups wait for each other before panels take over (0: not)."""
+        check(self.lib.dmrg_set_reduction(self.ctx, int(bool(in_registers)), float(wait_ms)), "dmrg_set_reduction")
+
+    def reduction_counts(self):
+        """Reductions so far: (one workgroup, across workgroups, attempts given
+        up, by panels)."""
+        n = (ctypes.c_longlong * 4)()
+        check(self.lib.dmrg_reduction_counts(self.ctx, n), "dmrg_reduction_counts")
+        return tuple(n)
+
     def herm_eig(self, A, mode=1):
         """Eigenpairs of a Hermitian device matrix given as planar float64
         [2, n, n] (copied): (w ascending [n], Z [2, n, n] planar with row k

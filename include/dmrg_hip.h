@@ -187,6 +187,18 @@ int dmrg_svd_split_guided(dmrg_ctx* ctx, int field, const double* M, int m, int 
  * dsyevd / zheevd. */
 int dmrg_set_eigensolver(dmrg_ctx* ctx, int mode);
 
+/* How the eigensolver's tridiagonalisation runs.  in_registers 1 (the default):
+ * with the matrix in registers where its order allows; 0: by panels, at every
+ * order.  Reductions across workgroups wait for each other on the device; where
+ * other work holds the compute units they need, a wait longer than wait_ms
+ * (default 50, at most 1000; 0: the first look that finds a word missing) ends
+ * the attempt and the panels run from the untouched input.
+ * dmrg_reduction_counts: this context's reductions so far, counts[0] in one
+ * workgroup, [1] across workgroups, [2] attempts given up, [3] by panels (a
+ * large order that starts in panels and ends in registers counts in both). */
+int dmrg_set_reduction(dmrg_ctx* ctx, int in_registers, double wait_ms);
+int dmrg_reduction_counts(dmrg_ctx* ctx, long long* counts);
+
 /* All eigenpairs of the real symmetric n x n matrix A (device, row-major;
  * overwritten): w ascending, row k of Z the eigenvector of w[k].  mode as
  * in dmrg_set_eigensolver.  The eigensolver of dmrg_svd_split exposed for
