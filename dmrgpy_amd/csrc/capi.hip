@@ -324,6 +324,7 @@ int dmrg_set_reduction(dmrg_ctx* ctx, int in_registers, double wait_ms) {
   DMRG_REQUIRE(wait_ms >= 0.0 && wait_ms <= 1000.0, "set_reduction: the wait must be 0 to 1000 ms");
   ctx->c.trd_registers = in_registers != 0;
   ctx->c.trd_wait = (long long)(wait_ms * 1e5);
+  ctx->c.trd_backoff = dmrg::Backoff();
   API_END
 }
 

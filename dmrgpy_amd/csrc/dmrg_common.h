@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 
+#include "backoff.h"
 #include "dmrg_error.h"
 
 #include <cstdint>
@@ -112,6 +113,7 @@ struct Ctx {
   bool trd_registers = true;
   long long trd_wait = 5000000;
   long long trd_counts[4] = {0, 0, 0, 0};
+  Backoff trd_backoff;   // attempts across workgroups, after one was given up
   int dc_n = 0;   // order of the tridiagonal whose divide and conquer the workspace holds
   hipEvent_t trd_ev[2] = {nullptr, nullptr};   // early-stop checks of the reduction in flight
   // allocation-free calls (dmrg_heff_apply_noalloc): while `noalloc` is set,

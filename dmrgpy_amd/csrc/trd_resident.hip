@@ -31,7 +31,10 @@
 // 3.0 / 3.2 us.  All waits are bounded: a workgroup that waits longer than
 // the context's limit (other work holding the CUs its peers need) gives up and
 // says so, the others leave their next long wait, the input is untouched and
-// the caller runs the launch-per-column reduction instead.
+// the caller runs the launch-per-column reduction instead.  Where the other
+// work stays, every attempt would cost a wait, so after a failure the context
+// passes over the next reductions (1, 2, 4 ... 64, until one succeeds): a
+// wasted wait of 50 ms is as long as 5000 columns by panels.
 //
 // Measured per column, launch-per-column / resident (us): real order 128
 // 8.7 / 2.45, 380 9.8 / 2.6, 2588 (930 columns reduced) 16.2 / 6.0; complex
@@ -560,13 +563,14 @@ int trd_resident_max(int field) { return field == CPLX ? 256 * 7 : 256 * 12; }
 
 // Reduces A[s0:, s0:] of the n x n matrix A (in place: reflectors into its
 // rows) as sytrd_lower / hetrd_lower do; false (nothing changed) when the
-// order is out of range, the workgroups do not all fit, or a wait ran out.
+// order is out of range, the workgroups do not all fit, or a wait ran out (now
+// or shortly before).
 // *done: absolute number of columns reduced; *dropped: trace of the rest.
 bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double* e, double* tau, double stop_tol,
                   double total2, int* done, double* dropped) {
   const bool cx = field == CPLX;
   const int m = n - s0, np = cx ? 2 : 1;
-  if (m < 3 || m > trd_resident_max(field)) return false;
+  if (m < 3 || m > trd_resident_max(field) || !c->trd_backoff.allowed()) return false;
   // workgroup size and rows per workgroup: 13 rows (7 complex) fill the
   // 16-value reduction; larger orders take 12 so that the rows fit the
   // registers (512 threads, 256 registers each)
@@ -625,9 +629,11 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
   std::memcpy(st, c->host_scalars + 36, sizeof(st));
   if (st[0] != 0) {
     ++c->trd_counts[2];
+    c->trd_backoff.failed();
     return false;
   }
   ++c->trd_counts[1];
+  c->trd_backoff.succeeded();
   trd_resident_store_k<<<st[1], 256, 0, c->stream>>>(g.R, m, st[1], A + (long long)s0 * n + s0, n, g.pA, np);
   DMRG_CHECK_HIP(hipGetLastError());
   *done = s0 + st[1];

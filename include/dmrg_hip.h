@@ -192,7 +192,9 @@ int dmrg_set_eigensolver(dmrg_ctx* ctx, int mode);
  * order.  Reductions across workgroups wait for each other on the device; where
  * other work holds the compute units they need, a wait longer than wait_ms
  * (default 50, at most 1000; 0: the first look that finds a word missing) ends
- * the attempt and the panels run from the untouched input.
+ * the attempt and the panels run from the untouched input, as they do at once
+ * for the next 1, 2, 4 ... 64 reductions after attempts in a row that failed
+ * (this call forgets them).
  * dmrg_reduction_counts: this context's reductions so far, counts[0] in one
  * workgroup, [1] across workgroups, [2] attempts given up, [3] by panels (a
  * large order that starts in panels and ends in registers counts in both). */

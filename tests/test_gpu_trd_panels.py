@@ -62,7 +62,19 @@ def test_early_stop(engine, reduction, field, shape, setting):
     reduction(**setting)
     single, registers, given_up, panels = _counted(engine, lambda: early_stop_matches(engine, field, shape))
     assert (single, registers, panels) == (0, 0, 4)   # two splits in each of two modes
-    assert given_up == (4 if "wait_ms" in setting else 0)
+    assert given_up == (2 if "wait_ms" in setting else 0)   # the second and fourth come after a failure
+
+
+def test_back_off(engine, reduction):
+    """After a failure the next 1, 2, 4 ... reductions go to the panels at once,
+    until a setting or a success forgets it."""
+    import torch
+    A = torch.from_numpy(_graded(np.random.default_rng(0), 150, False)).to(engine.device)
+    reduction(wait_ms=0.0)
+    tried = [_counted(engine, lambda: engine.sym_eig(A, 1))[2] for _ in range(12)]
+    assert tried == [1, 0, 1, 0, 0, 1, 0, 0, 0, 0, 1, 0]
+    reduction()
+    assert _counted(engine, lambda: engine.sym_eig(A, 1)) == (0, 1, 0, 0)
 
 
 @pytest.mark.parametrize("field,shape", [(0, (3300, 3200)), (0, (3400, 3500)), (1, (2000, 2100))])
