@@ -29,12 +29,12 @@
 // validity, so no fence, flag or cache write-back is needed.  Measured with
 // 16 / 32 / 64 / 128 / 256 workgroups exchanging 760 words: 1.6 / 2.1 / 2.5 /
 // 3.0 / 3.2 us.  All waits are bounded: a workgroup that waits longer than
-// the context's limit (other work holding the CUs its peers need) gives up and
-// says so, the others leave their next long wait, the input is untouched and
-// the caller runs the launch-per-column reduction instead.  Where the other
-// work stays, every attempt would cost a wait, so after a failure the context
-// passes over the next reductions (1, 2, 4 ... 64, until one succeeds): a
-// wasted wait of 50 ms is as long as 5000 columns by panels.
+// the context's limit (other work holding the CUs its peers need) gives up, as
+// then do the others (at once where they had not started), the input is
+// untouched and the caller runs the launch-per-column reduction instead.  Where
+// the other work stays, every attempt would cost a wait, so after a failure the
+// context passes over the next reductions (1, 2, 4 ... 64, until one succeeds):
+// a wasted wait of 50 ms is as long as 5000 columns by panels.
 //
 // Measured per column, launch-per-column / resident (us): real order 128
 // 8.7 / 2.45, 380 9.8 / 2.6, 2588 (930 columns reduced) 16.2 / 6.0; complex
@@ -79,17 +79,19 @@ __device__ __forceinline__ unsigned long long peek(const unsigned long long* p) 
 }
 
 // One wait for words published by other workgroups: over() after each look
-// that missed some; true once the limit has passed or another workgroup gave
-// up (workgroups that start late then leave at once, not after a limit each)
+// that missed some, true once the limit has passed (ANY: the argument's, else
+// the default one; see resident_launch)
+constexpr long long RES_DEFAULT = 5000000;   // wall-clock ticks (100 MHz): 50 ms, as Ctx::trd_wait
+template <bool ANY>
 struct Patience {
   int spin = 0;
   long long t0 = 0;
   __device__ __forceinline__ bool over(const ResArgs& g) {
-    if (g.limit == 0) return true;
+    if (ANY && g.limit == 0) return true;
     if ((++spin & 63) != 0) return false;
     const long long t = wall_clock64();
     if (t0 == 0) t0 = t;
-    return t - t0 > g.limit || __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    return t - t0 > (ANY ? g.limit : RES_DEFAULT);
   }
 };
 __device__ __forceinline__ void give_up(const ResArgs& g) {
@@ -97,7 +99,7 @@ __device__ __forceinline__ void give_up(const ResArgs& g) {
 }
 
 // T threads, thread t holds columns t, t + T, ... (CC of them) of RW rows.
-template <bool CX, int T, int CC, int RW>
+template <bool CX, int T, int CC, int RW, bool ANY>
 __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
   constexpr int NP = CX ? 2 : 1, NW = T / 64, NS = NP * RW;
   // 16 sums per column: A x of the own rows, |x|^2 at NS and, real, w.x and v.x
@@ -113,7 +115,11 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
   const int wg = blockIdx.x, G = gridDim.x, m = g.m, mp = g.mp;
   const int row0 = wg * RW, last = min(row0 + RW, m) - 1;
   const bool writer = wg == G - 1;
-  if (tid == 0) s_bad = 0;
+  // an attempt already given up before this workgroup found a place: leave at
+  // once, or workgroups that run one after the other would each wait a limit
+  if (tid == 0) s_bad = __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (s_bad) return;
 
   // own rows (conj(buffer) when complex: the reduction works on the column-major view)
   double M[NP][RW][CC], a[NP][CC], v[NP][CC], w[NP][CC];
@@ -307,7 +313,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
       double f2 = 0.0, tc = 0.0;
       for (int o = J / RW + tid; o < G; o += T) {   // the workgroups that hold rows from J on
         unsigned long long y0, y1;
-        Patience wait;
+        Patience<ANY> wait;
         for (;;) {
           y0 = peek(ck + o);
           y1 = peek(ck + G + o);
@@ -418,7 +424,7 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
 #pragma unroll
         for (int k = 0; k < CC; ++k) uc[p][k] = peek(Xc + p * mp + idx[k]);
       }
-      Patience wait;
+      Patience<ANY> wait;
       bool ok = true, miss;
       do {
         miss = false;
@@ -547,14 +553,18 @@ __global__ __launch_bounds__(256) void trd_resident_store_k(const double* __rest
       A[(long long)p * pA + (long long)j * lda + c] = R[((long long)p * m + j) * m + c];
 }
 
-template <bool CX, int T, int CC, int RW>
+// ANY = false keeps the default limit as a constant.  The two variants that fill
+// the registers (real 6, complex 4 columns per thread) have it both ways, since
+// one more argument takes them from 5.57 to 5.9 us per column at order 2588,
+// from 6.58 to 6.7 at 1700.
+template <bool CX, int T, int CC, int RW, bool ANY = true>
 static bool resident_launch(Ctx* c, const ResArgs& g, int G) {
   // every workgroup must be resident at once: they wait for each other
   int per_cu = 0, cus = 0;
-  DMRG_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trd_resident_k<CX, T, CC, RW>, T, 0));
+  DMRG_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trd_resident_k<CX, T, CC, RW, ANY>, T, 0));
   DMRG_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
   if ((long long)per_cu * cus < G) return false;
-  trd_resident_k<CX, T, CC, RW><<<G, T, 0, c->stream>>>(g);
+  trd_resident_k<CX, T, CC, RW, ANY><<<G, T, 0, c->stream>>>(g);
   DMRG_CHECK_HIP(hipGetLastError());
   return true;
 }
@@ -611,7 +621,10 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
       case 3: ok = resident_launch<false, 512, 3, 12>(c, g, G); break;
       case 4: ok = resident_launch<false, 512, 4, 12>(c, g, G); break;
       case 5: ok = resident_launch<false, 512, 5, 12>(c, g, G); break;
-      case 6: ok = resident_launch<false, 512, 6, 12>(c, g, G); break;
+      case 6:
+        ok = g.limit == RES_DEFAULT ? resident_launch<false, 512, 6, 12, false>(c, g, G)
+                                    : resident_launch<false, 512, 6, 12>(c, g, G);
+        break;
     }
   } else {
     if (T == 256) ok = resident_launch<true, 256, 1, 7>(c, g, G);
@@ -619,7 +632,10 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
       case 1: ok = resident_launch<true, 512, 1, 7>(c, g, G); break;
       case 2: ok = resident_launch<true, 512, 2, 7>(c, g, G); break;
       case 3: ok = resident_launch<true, 512, 3, 7>(c, g, G); break;
-      case 4: ok = resident_launch<true, 512, 4, 7>(c, g, G); break;
+      case 4:
+        ok = g.limit == RES_DEFAULT ? resident_launch<true, 512, 4, 7, false>(c, g, G)
+                                    : resident_launch<true, 512, 4, 7>(c, g, G);
+        break;
     }
   }
   if (!ok) return false;
