@@ -14,6 +14,8 @@
 #include "gemm_kernels.h"
 #include "tile_order.h"
 
+#include <type_traits>
+
 namespace dmrg {
 
 // ---------------------------------------------------------------------------
@@ -596,13 +598,13 @@ static void check_desc(const GemmDesc& d) {
 }
 
 // Launch helpers: pick the instantiation for (transA, transB, tag).
-template <typename T, int TM, int TN, bool TA, bool TB, typename CT = T>
-static void launch_fast_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C) {
+template <typename T, int TM, int TN, bool TA, bool TB>
+static void launch_fast_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, T* C) {
   const GemmArgs g = make_args(d, 32 * TM, 32 * TN);
   const dim3 grid((unsigned)g.nbx * g.nby, 1, d.batch);
   switch (d.tag) {
 #define CASE(t) \
-  case t: gemm_fast<T, TM, TN, TA, TB, t, CT><<<grid, 256, 0, c->stream>>>(A, B, C, g); break;
+  case t: gemm_fast<T, TM, TN, TA, TB, t><<<grid, 256, 0, c->stream>>>(A, B, C, g); break;
     DMRG_GEMM_TAGS(CASE)
 #undef CASE
     default: throw Error("gemm: bad tag");
@@ -612,10 +614,14 @@ static void launch_fast_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B
 
 template <typename T, int TM, int TN, typename CT = T>
 static void launch_fast(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C) {
-  if (!d.transA && !d.transB) launch_fast_tagged<T, TM, TN, false, false, CT>(c, d, A, B, C);
-  else if (d.transA && !d.transB) launch_fast_tagged<T, TM, TN, true, false, CT>(c, d, A, B, C);
-  else if (!d.transA && d.transB) launch_fast_tagged<T, TM, TN, false, true, CT>(c, d, A, B, C);
-  else launch_fast_tagged<T, TM, TN, true, true, CT>(c, d, A, B, C);
+  if constexpr (!std::is_same<T, CT>::value) {   // gemm_f32_c64
+    const GemmArgs g = make_args(d, 32 * TM, 32 * TN);
+    gemm_fast<T, TM, TN, false, false, 2, CT><<<dim3((unsigned)g.nbx * g.nby, 1, d.batch), 256, 0, c->stream>>>(A, B, C, g);
+    DMRG_CHECK_HIP(hipGetLastError());
+  } else if (!d.transA && !d.transB) launch_fast_tagged<T, TM, TN, false, false>(c, d, A, B, C);
+  else if (d.transA && !d.transB) launch_fast_tagged<T, TM, TN, true, false>(c, d, A, B, C);
+  else if (!d.transA && d.transB) launch_fast_tagged<T, TM, TN, false, true>(c, d, A, B, C);
+  else launch_fast_tagged<T, TM, TN, true, true>(c, d, A, B, C);
 }
 
 // Which kernel a real product takes.  The LDS kernel runs square tiles
@@ -664,10 +670,12 @@ static void launch_fast_f32(Ctx* c, const GemmDesc& d, const float* A, const flo
   }
 }
 
-// Real FP32 GEMM writing an FP64 result (the R-step of the FP32 H_eff apply
-// writes y straight into the FP64 Krylov vector, with no conversion pass).
+// Real FP32 GEMM writing an FP64 result: the R-step of the FP32 H_eff apply
+// writes y straight into the FP64 Krylov vector, with no conversion pass.
+// Built for that caller only (no transposes, tag 2).
 void gemm_f32_c64(Ctx* c, const GemmDesc& d, const float* A, const float* B, double* C) {
-  DMRG_REQUIRE(d.field == REAL && d.beta == 0.0, "gemm_f32_c64: real field and beta = 0 only");
+  DMRG_REQUIRE(d.field == REAL && d.beta == 0.0 && !d.transA && !d.transB && d.tag == 2,
+               "gemm_f32_c64: real field, beta = 0, no transposes and tag 2 only");
   check_desc(d);
   if (d.M == 0 || d.N == 0) return;
   if (use_direct(d, false)) gemm_direct_f32_c64(c, d, A, B, C);

@@ -13,6 +13,8 @@
 #include "gemm_kernels.h"
 #include "tile_order.h"
 
+#include <type_traits>
+
 namespace dmrg {
 
 template <typename T, bool CX, int WM, int WN, bool TA, bool TB, int TAG, typename CT>
@@ -215,28 +217,34 @@ __global__ __launch_bounds__(256) void gemm_direct(const T* __restrict__ A, cons
       }
 }
 
-template <typename T, bool CX, int WM, int WN, bool TA, bool TB, typename CT>
-static void launch_direct_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, int ks) {
+template <typename T, bool CX, int WM, int WN, bool TA, bool TB, int TAG, typename CT>
+static void launch_direct_as(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, int ks) {
   constexpr int TM = 16 * WM, TN = 16 * WN;
   const GemmArgs g = make_args(d, TM, TN);
   const dim3 grid((unsigned)g.nbx * g.nby, 1, d.batch);
   const size_t lds = (size_t)(ks / 2) * (CX ? 2 : 1) * TM * TN * sizeof(T);
+  gemm_direct<T, CX, WM, WN, TA, TB, TAG, CT><<<grid, 64 * ks, lds, c->stream>>>(A, B, C, g);
+  DMRG_CHECK_HIP(hipGetLastError());
+}
+
+template <typename T, bool CX, int WM, int WN, bool TA, bool TB>
+static void launch_direct_tagged(Ctx* c, const GemmDesc& d, const T* A, const T* B, T* C, int ks) {
   switch (d.tag) {
 #define CASE(t) \
-  case t: gemm_direct<T, CX, WM, WN, TA, TB, t, CT><<<grid, 64 * ks, lds, c->stream>>>(A, B, C, g); break;
+  case t: launch_direct_as<T, CX, WM, WN, TA, TB, t, T>(c, d, A, B, C, ks); break;
     DMRG_GEMM_TAGS(CASE)
 #undef CASE
     default: throw Error("gemm: bad tag");
   }
-  DMRG_CHECK_HIP(hipGetLastError());
 }
 
 template <typename T, bool CX, int WM, int WN, typename CT>
 static void launch_direct_tt(Ctx* c, const GemmDesc& d, const T* A, const T* B, CT* C, int ks) {
-  if (!d.transA && !d.transB) launch_direct_tagged<T, CX, WM, WN, false, false, CT>(c, d, A, B, C, ks);
-  else if (d.transA && !d.transB) launch_direct_tagged<T, CX, WM, WN, true, false, CT>(c, d, A, B, C, ks);
-  else if (!d.transA && d.transB) launch_direct_tagged<T, CX, WM, WN, false, true, CT>(c, d, A, B, C, ks);
-  else launch_direct_tagged<T, CX, WM, WN, true, true, CT>(c, d, A, B, C, ks);
+  if constexpr (!std::is_same<T, CT>::value) launch_direct_as<T, CX, WM, WN, false, false, 2, CT>(c, d, A, B, C, ks);
+  else if (!d.transA && !d.transB) launch_direct_tagged<T, CX, WM, WN, false, false>(c, d, A, B, C, ks);
+  else if (d.transA && !d.transB) launch_direct_tagged<T, CX, WM, WN, true, false>(c, d, A, B, C, ks);
+  else if (!d.transA && d.transB) launch_direct_tagged<T, CX, WM, WN, false, true>(c, d, A, B, C, ks);
+  else launch_direct_tagged<T, CX, WM, WN, true, true>(c, d, A, B, C, ks);
 }
 
 // Tile and split.  Four waves share a tile's inner dimension where tiles are

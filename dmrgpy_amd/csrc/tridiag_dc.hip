@@ -66,7 +66,7 @@ struct DcLevel {
   int *rbase, *rlen;           // rotation -> first of its chain; at a chain's first, its length
   int *ichain, *ipos;          // index -> first rotation of its chain (-1: none), position in it
   int* col;                    // ascending position -> survivor j or N + deflated k
-  int *K, *nrot;               // per merge
+  int* K;                      // survivors per merge
   int* stat;                   // [blocks] nonzero: failed
 };
 
@@ -340,7 +340,6 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
         if (nr > base) L.rlen[o + base] = nr - base;
       }
     }
-    L.nrot[m] = nr;
   }
   __syncthreads();
   // ---- survivors
@@ -556,7 +555,7 @@ static DcLevel dc_level(int n, const double* e, int S, double* ws, int np) {
   int* q = (int*)p;
   auto itg = [&]() { int* r = q; q += np; return r; };
   L.org = itg(); L.sidx = itg(); L.rep = itg(); L.didx = itg(); L.drot = itg(); L.rbase = itg(); L.rlen = itg();
-  L.ichain = itg(); L.ipos = itg(); L.col = itg(); L.K = itg(); L.nrot = itg();
+  L.ichain = itg(); L.ipos = itg(); L.col = itg(); L.K = itg();
   return L;
 }
 
