@@ -70,10 +70,7 @@ struct DcLevel {
   int* stat;                   // [blocks] nonzero: failed
 };
 
-__device__ __forceinline__ double dc_coupling(double e, double scale) {
-  const double x = e / scale;
-  return fabs(x) < DC_TINY ? 0.0 : x;
-}
+__device__ __forceinline__ double dc_coupling(double e) { return fabs(e) < DC_TINY ? 0.0 : e; }
 
 // ---------------------------------------------------------------------------
 // Blocks: implicit QL with shifts, one wave per block.  Every lane runs the
@@ -104,13 +101,13 @@ __global__ __launch_bounds__(64) void dc_leaf_k(const double* __restrict__ d, co
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-  const double sc = mx > 0.0 ? mx : 1.0;
+  const double sc = mx > 0.0 ? fmax(mx, 1e-300) : 1.0, inv = 1.0 / sc;
   if (blockIdx.x == 0 && lane == 0) scale[0] = sc;
-  auto off = [&](int i) { return i >= 0 && i < n - 1 ? dc_coupling(e[i], sc) : 0.0; };   // of i and i + 1
+  auto off = [&](int i) { return i >= 0 && i < n - 1 ? dc_coupling(e[i] * inv) : 0.0; };   // of i and i + 1
   // a block graded downwards is turned upside down: QL keeps the small
   // eigenvalues' accuracy when the small entries come first
   auto diag = [&](int i) {
-    double x = i < n ? d[i] / sc : DC_PAD;
+    double x = i < n ? d[i] * inv : DC_PAD;
     if (i == b0) x -= fabs(off(b0 - 1));               // tearing at the block's two ends
     if (i == b0 + B - 1) x -= fabs(off(b0 + B - 1));
     return x;
@@ -234,7 +231,7 @@ __global__ __launch_bounds__(256) void dc_deflate_k(DcLevel L) {
   const double* Q1 = L.Q + (size_t)(2 * m) * S * S;
   const double* Q2 = Q1 + (size_t)S * S;
   const int cut = m * N + S;   // first row of the lower block
-  const double beta = cut < L.n ? dc_coupling(L.e[cut - 1], L.scale[0]) : 0.0;
+  const double beta = cut < L.n ? dc_coupling(L.e[cut - 1] / L.scale[0]) : 0.0;
   const double rho = 2.0 * fabs(beta), sg = beta < 0.0 ? -0.70710678118654752440 : 0.70710678118654752440;
   for (int i = tid; i < N; i += 256) {   // every slot valid whatever the values (NaN) do to the order
     sd[i] = sz[i] = 0.0;
@@ -538,6 +535,7 @@ static size_t dc_deflate_lds(int N) {
   return (size_t)N * (2 * sizeof(double) + 2 * sizeof(int)) + 32 * (size_t)((N + 255) / 256);
 }
 
+// orders up to 4096 would pad to the arrays' limit; 4032 is the largest one tested
 bool tridiag_dc_ok(int n) { return n >= 1 && n <= DC_MAX - 64; }
 
 // [Q ping][Q pong][Ut][D ping][D pong][arrays of a level][scale][status of up to 512 blocks]
