@@ -201,6 +201,7 @@ def run_sweeps(ch, psi, K, prec_name, maxdim):
     prec = PREC_NAMES[prec_name]
     stats = alg.Stats()
     eng.prof_enable(True)
+    cols = eng.reduction_counts()[4]
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(K):
@@ -209,6 +210,7 @@ def run_sweeps(ch, psi, K, prec_name, maxdim):
     dt = time.perf_counter() - t0
     tms, flops, calls = eng.prof_read()
     nbytes = eng.prof_read_bytes()
+    cols = eng.reduction_counts()[4] - cols
     eng.prof_enable(False)
     nrm = alg.overlap(eng, psi, psi).real
     e = (alg.expectation(eng, psi, ch.H, psi) / nrm).real
@@ -219,7 +221,7 @@ def run_sweeps(ch, psi, K, prec_name, maxdim):
             "heff_ms": tms[0], "heff_flops": flops[0], "heff_calls": calls[0],
             "heff_bytes": nbytes[0],
             "env_ms": tms[1], "svd_ms": tms[2], "svd_calls": calls[2],
-            "trd_ms": tms[4], "trd_calls": calls[4], "trd_bytes": nbytes[4],
+            "trd_ms": tms[4], "trd_calls": calls[4], "trd_columns": cols,
             "vec_ms": tms[3], "vec_calls": calls[3], "vec_bytes": nbytes[3],
             "iters_per_bond": sum(stats.lanczos_iters) / max(1, len(stats.lanczos_iters)),
             "svd_guided_fraction": sum(stats.svd_guided) / max(1, len(stats.svd_guided)),
@@ -744,14 +746,16 @@ def main():
                         "kernel": "H_eff two-site apply at Dl = Dr = {} with the model's bulk MPO tensors and random "
                                   "environments, 10 applies".format(D)}
     if res["trd_calls"] > 0 and res["trd_ms"] > 0:
-        # the Gram eigensolver's tridiagonalisation, the largest cost of a sweep:
-        # algorithmic bytes = the lower triangle of the trailing matrix once per column
-        gbs = res["trd_bytes"] / (res["trd_ms"] * 1e-3) / 1e9
+        # the Gram eigensolver's tridiagonalisation, the largest cost of a sweep: with the matrix in registers a
+        # column moves two vectors between the workgroups, so its floor is that exchange (2.5 us measured alone
+        # with 64 workgroups, 3.2 with 256)
+        us = 1e3 * res["trd_ms"] / max(1, res["trd_columns"])
         out["roofline_tridiagonalisation"] = {
-            "bound": "hbm", "achieved": gbs, "peak": 8000.0, "unit": "GB/s", "frac": gbs / 8000.0, "traffic": None,
-            "algorithmic_bytes": res["trd_bytes"] / res["trd_calls"],
-            "kernel": "own Householder tridiagonalisation of the Gram matrices (in registers up to order 3072, one exchange per column; "
-                      "panel GEMMs), {} reductions per sweep, {:.2f} ms average, {:.2f} s per sweep".format(
+            "bound": "latency", "achieved": us, "peak": 3.2, "unit": "us per column", "frac": 3.2 / us, "traffic": None,
+            "columns_per_reduction": res["trd_columns"] / res["trd_calls"],
+            "kernel": "own Householder tridiagonalisation of the Gram matrices (in registers up to order 3072, one "
+                      "exchange per column; larger orders by panels down to that), {} reductions per sweep, {:.2f} ms "
+                      "average, {:.2f} s per sweep".format(
                           int(res["trd_calls"] / args.steps), res["trd_ms"] / res["trd_calls"],
                           res["trd_ms"] / 1e3 / args.steps)}
     if res["vec_calls"] > 0 and res["vec_ms"] > 0:

@@ -331,7 +331,7 @@ int dmrg_set_reduction(dmrg_ctx* ctx, int in_registers, double wait_ms) {
 int dmrg_reduction_counts(dmrg_ctx* ctx, long long* counts) {
   API_BEGIN
   DMRG_REQUIRE(ctx && counts, "reduction_counts: null argument");
-  for (int i = 0; i < 4; ++i) counts[i] = ctx->c.trd_counts[i];
+  for (int i = 0; i < 5; ++i) counts[i] = ctx->c.trd_counts[i];
   API_END
 }
 

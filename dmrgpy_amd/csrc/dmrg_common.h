@@ -109,10 +109,10 @@ struct Ctx {
   int eig_mode = 1;
   // tridiagonalisation: in-register reductions allowed, the longest wait of one
   // for its workgroups in wall-clock ticks (100 MHz), and how reductions ran:
-  // one workgroup, across workgroups, given up, by panels
+  // one workgroup, across workgroups, given up, by panels; columns reduced
   bool trd_registers = true;
   long long trd_wait = 5000000;
-  long long trd_counts[4] = {0, 0, 0, 0};
+  long long trd_counts[5] = {0, 0, 0, 0, 0};
   Backoff trd_backoff;   // attempts across workgroups, after one was given up
   int dc_n = 0;   // order of the tridiagonal whose divide and conquer the workspace holds
   hipEvent_t trd_ev[2] = {nullptr, nullptr};   // early-stop checks of the reduction in flight

@@ -5,7 +5,7 @@
 //
 // Vector work per iteration k (n elements per plane, sizeof = 8): three
 // kernels after the apply (kry_alpha_k, kry_project_k, kry_clean_k), about
-// (2k + 7) * n * 8 bytes of HBM traffic -- bandwidth bound for long vectors,
+// (2k + 8) * n * 8 bytes of HBM traffic -- bandwidth bound for long vectors,
 // launch bound for short ones.
 #include "dmrg_internal.h"
 #include "host_eig.h"

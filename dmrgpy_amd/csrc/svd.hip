@@ -445,8 +445,8 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
     mirror_lower(c, Gplanar, g, g, (long long)g * g, field);
     if (cx && c->eig_mode >= 1) {
       // complex Hermitian: own reduction to a real tridiagonal (stopping
-      // early in mode 1 as the real one does), rocSOLVER's divide and
-      // conquer on it; unmtr on the kept columns after keep
+      // early in mode 1 as the real one does) and divide and conquer on it;
+      // the back-transformation of the kept columns waits for keep
       trd_Z = (double*)ws_get(c, WS_TRD_Z, sizeof(double) * ((size_t)g * g + 2 * (size_t)g + 16));
       trd_tau = trd_Z + (size_t)g * g;
       trd_nrefl = hetrd_lower(c, Gplanar, g, ev, ework, trd_tau, c->eig_mode == 1 ? TRD_STOP_TOL : 0.0,
@@ -463,8 +463,8 @@ static SvdOut svd_gram(Ctx* c, int field, const double* M, int m, int n, double 
                "zheevd");
       Gsolve = Gi;
     } else if (c->eig_mode >= 1 && g >= 32) {
-      // tridiagonalise here, eigenpairs of the tridiagonal by rocSOLVER's
-      // divide and conquer; the back-transformation waits for keep.  In
+      // tridiagonalise here, eigenvalues of the tridiagonal by divide and
+      // conquer; vectors and back-transformation wait for keep.  In
       // mode 1 the reduction stops once the trailing block is below
       // TRD_STOP_TOL |G|_F (sytrd_lower), and divide and conquer then runs
       // on the leading order-(nrefl + 1) tridiagonal only; the rest of the

@@ -30,7 +30,8 @@
 // matrix-vector products read whole rows).  Outputs match dsytrd(uplo = 'L')
 // on the column-major view (the matrix is symmetric, so the row-major buffer
 // is the same matrix): d, e, tau, and reflector j in row j, columns j+2..,
-// ready for rocsolver_dstedc and the back-transformation below.  All sums
+// ready for the divide and conquer (tridiag_dc.hip) and the back-transformation
+// below.  All sums
 // run in a fixed order (deterministic).
 #include "dmrg_internal.h"
 #include "gemm_kernels.h"
@@ -423,6 +424,13 @@ static double trailing_sumsq_wait(Ctx* c, int slot) {
   return c->host_scalars[32 + slot];
 }
 
+// `done` columns of an order-n reduction: their count, and as algorithmic bytes
+// the lower triangle of the trailing matrix (es bytes an entry) once per column
+static void trd_account(Ctx* c, ProfScope& ps, int n, int done, double es) {
+  c->trd_counts[4] += done;
+  for (int j = 0; j < done; ++j) ps.bytes += es * (double)(n - j - 1) * (n - j) / 2.0;
+}
+
 // A (n x n, symmetric, row-major = column-major) -> d[n], e[n-1], tau[n-1]
 // and reflectors in place (dsytrd, uplo 'L').  Returns the number of
 // reflectors computed: n - 1, or, with stop_tol > 0, possibly fewer -- after
@@ -451,7 +459,7 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
       trd_clear_tail_k<<<1, 256, 0, c->stream>>>(n, done, d, e, tau, 1);
       DMRG_CHECK_HIP(hipGetLastError());
     }
-    for (int j = 0; j < done; ++j) ps.bytes += 8.0 * (double)(n - j - 1) * (n - j) / 2.0;
+    trd_account(c, ps, n, done, 8.0);
     return done;
   }
   const size_t vwv = (size_t)n * TRD_P;   // the [V | W | V] panel store
@@ -485,7 +493,7 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
       trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 1);
       DMRG_CHECK_HIP(hipGetLastError());
     }
-    for (int j = 0; j < done; ++j) ps.bytes += 8.0 * (double)(n - j - 1) * (n - j) / 2.0;
+    trd_account(c, ps, n, done, 8.0);
     return done;
   }
   bool resident = c->trd_registers && !fits;   // to be tried once
@@ -563,8 +571,7 @@ int sytrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
   if (done == n - 1 && !in_registers)
     DMRG_CHECK_HIP(hipMemcpyAsync(d + (n - 1), A + (size_t)(n - 1) * n + (n - 1), sizeof(double),
                                   hipMemcpyDeviceToDevice, c->stream));
-  // algorithmic bytes: the lower triangle of the trailing matrix, once per reduced column
-  for (int j = 0; j < done; ++j) ps.bytes += 8.0 * (double)(n - j - 1) * (n - j) / 2.0;
+  trd_account(c, ps, n, done, 8.0);
   return done;
 }
 
@@ -987,7 +994,7 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
       trd_clear_tail_k<<<(n - done + 255) / 256, 256, 0, c->stream>>>(n, done, d, e, tau, 2);
       DMRG_CHECK_HIP(hipGetLastError());
     }
-    for (int j = 0; j < done; ++j) ps.bytes += 16.0 * (double)(n - j - 1) * (n - j) / 2.0;
+    trd_account(c, ps, n, done, 16.0);
     return done;
   }
   bool resident = c->trd_registers && !fits;   // to be tried once
@@ -1062,8 +1069,7 @@ int hetrd_lower(Ctx* c, double* A, int n, double* d, double* e, double* tau, dou
   if (done == n - 1 && !in_registers)
     DMRG_CHECK_HIP(hipMemcpyAsync(d + (n - 1), A + (size_t)(n - 1) * n + (n - 1), sizeof(double),
                                   hipMemcpyDeviceToDevice, c->stream));
-  // algorithmic bytes: the lower triangle of the trailing matrix (both planes) once per reduced column
-  for (int j = 0; j < done; ++j) ps.bytes += 16.0 * (double)(n - j - 1) * (n - j) / 2.0;
+  trd_account(c, ps, n, done, 16.0);
   return done;
 }
 

@@ -354,7 +354,8 @@ __global__ __launch_bounds__(T) void trd_resident_k(ResArgs g) {
         passed = f2 <= g.tol2 * total2;
       }
     }
-    // ---- reflector of column J (every workgroup, the same sums in the same order)
+    // ---- reflector of column J (every workgroup, the same sums in the same order;
+    // |x|^2 is the plain sum of squares, as in the panels)
     const double xn2 = lane_value(tot, NS);
     const double a0r = s_a0[0], a0i = CX ? s_a0[NP - 1] : 0.0;
     double beta;

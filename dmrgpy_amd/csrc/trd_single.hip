@@ -216,7 +216,9 @@ __global__ __launch_bounds__(256) void trd_single_k(SingleArgs g) {
     double beta;
     {
       const double h2 = a0 * a0 + xx;
-      // powers of two out of the range where squares can over- or underflow
+      // powers of two keep a0^2 and the root in range; xx is the plain sum of
+      // squares, as in the panels: entries of x below 1e-154 lose digits in
+      // it, and below 1e-162 they count as zero
       const double up = h2 > 1e-280 ? (h2 < 1e280 ? 1.0 : 0x1p-600) : 0x1p600;
       const double dn = h2 > 1e-280 ? (h2 < 1e280 ? 1.0 : 0x1p600) : 0x1p-600;
       const double b = a0 * up;

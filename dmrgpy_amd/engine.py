@@ -246,8 +246,8 @@ class Engine:
 
     def reduction_counts(self):
         """Reductions so far: (one workgroup, across workgroups, attempts given
-        up, by panels)."""
-        n = (ctypes.c_longlong * 4)()
+        up, by panels), and the columns they reduced."""
+        n = (ctypes.c_longlong * 5)()
         check(self.lib.dmrg_reduction_counts(self.ctx, n), "dmrg_reduction_counts")
         return tuple(n)
 

@@ -174,17 +174,18 @@ int dmrg_svd_split_guided(dmrg_ctx* ctx, int field, const double* M, int m, int 
  * order 3072 real, 1792 complex; larger orders by panels down to that),
  * solves the tridiagonal with this library's divide and conquer (rocSOLVER's
  * past order 4032) and back-transforms only the eigenvectors the truncation
- * keeps with this library's blocked compact-WY GEMMs.  For a real Gram matrix of order
- * above 96, mode 1 checks the trailing block every 32 columns from column
- * 64 on and stops the reduction one check after the first at which its
- * Frobenius norm is at most 2e-15 of the Gram matrix's: that block's eigenvalues are then taken as zero
- * (they lie below the FP64 rounding of forming the Gram matrix), its trace
+ * keeps with this library's blocked compact-WY GEMMs.  For a Gram matrix of
+ * order above 96, mode 1 checks the trailing block every 32 columns from
+ * column 64 on and stops the reduction one check after the first at which its
+ * Frobenius norm is at most 2e-15 of the Gram matrix's: that block's
+ * eigenvalues are then taken as zero (they lie below the FP64 rounding of forming the Gram matrix), its trace
  * is counted as discarded weight, and the divide and conquer runs on the
  * reduced order; a split that would keep more values than the reduced
  * order falls back to the full SVD.  Mode 3
  * is mode 1 with the complete reduction; mode 2 is mode 3 with rocSOLVER's
  * dormtr / zunmtr for the back-transformation; mode 0 calls rocSOLVER
- * dsyevd / zheevd. */
+ * dsyevd / zheevd.  A matrix that holds NaN or infinity, and an iteration that
+ * does not converge, make the split and the calls below return an error. */
 int dmrg_set_eigensolver(dmrg_ctx* ctx, int mode);
 
 /* How the eigensolver's tridiagonalisation runs.  in_registers 1 (the default):
@@ -197,7 +198,8 @@ int dmrg_set_eigensolver(dmrg_ctx* ctx, int mode);
  * (this call forgets them).
  * dmrg_reduction_counts: this context's reductions so far, counts[0] in one
  * workgroup, [1] across workgroups, [2] attempts given up, [3] by panels (a
- * large order that starts in panels and ends in registers counts in both). */
+ * large order that starts in panels and ends in registers counts in both), and
+ * [4] the columns they reduced. */
 int dmrg_set_reduction(dmrg_ctx* ctx, int in_registers, double wait_ms);
 int dmrg_reduction_counts(dmrg_ctx* ctx, long long* counts);
 

@@ -28,7 +28,7 @@ def reduction(engine):
 def _counted(engine, fn):
     before = engine.reduction_counts()
     fn()
-    return tuple(b - a for a, b in zip(before, engine.reduction_counts()))
+    return tuple(b - a for a, b in zip(before, engine.reduction_counts()))[:4]
 
 
 def _eig(engine, n, cplx):
