@@ -80,7 +80,7 @@ __device__ __forceinline__ unsigned long long peek(const unsigned long long* p) 
 
 // One wait for words published by other workgroups: over() after each look
 // that missed some, true once the limit has passed (ANY: the argument's, else
-// the default one; see resident_launch)
+// the default one; see either_launch)
 constexpr long long RES_DEFAULT = 5000000;   // wall-clock ticks (100 MHz): 50 ms, as Ctx::trd_wait
 template <bool ANY>
 struct Patience {
@@ -554,10 +554,6 @@ __global__ __launch_bounds__(256) void trd_resident_store_k(const double* __rest
       A[(long long)p * pA + (long long)j * lda + c] = R[((long long)p * m + j) * m + c];
 }
 
-// ANY = false keeps the default limit as a constant.  The two variants that fill
-// the registers (real 6, complex 4 columns per thread) have it both ways, since
-// one more argument takes them from 5.57 to 5.9 us per column at order 2588,
-// from 6.58 to 6.7 at 1700.
 template <bool CX, int T, int CC, int RW, bool ANY = true>
 static bool resident_launch(Ctx* c, const ResArgs& g, int G) {
   // every workgroup must be resident at once: they wait for each other
@@ -568,6 +564,14 @@ static bool resident_launch(Ctx* c, const ResArgs& g, int G) {
   trd_resident_k<CX, T, CC, RW, ANY><<<G, T, 0, c->stream>>>(g);
   DMRG_CHECK_HIP(hipGetLastError());
   return true;
+}
+
+// The default limit as a constant of the code (ANY = false) where the variant
+// fills the registers: as one more argument it takes order 2588 from 5.57 to 5.9
+// us per column, complex 1700 from 6.58 to 6.7 and 1200 from 5.61 to 5.67.
+template <bool CX, int T, int CC, int RW>
+static bool either_launch(Ctx* c, const ResArgs& g, int G) {
+  return g.limit == RES_DEFAULT ? resident_launch<CX, T, CC, RW, false>(c, g, G) : resident_launch<CX, T, CC, RW>(c, g, G);
 }
 
 int trd_resident_max(int field) { return field == CPLX ? 256 * 7 : 256 * 12; }
@@ -622,21 +626,15 @@ bool trd_resident(Ctx* c, int field, double* A, int n, int s0, double* d, double
       case 3: ok = resident_launch<false, 512, 3, 12>(c, g, G); break;
       case 4: ok = resident_launch<false, 512, 4, 12>(c, g, G); break;
       case 5: ok = resident_launch<false, 512, 5, 12>(c, g, G); break;
-      case 6:
-        ok = g.limit == RES_DEFAULT ? resident_launch<false, 512, 6, 12, false>(c, g, G)
-                                    : resident_launch<false, 512, 6, 12>(c, g, G);
-        break;
+      case 6: ok = either_launch<false, 512, 6, 12>(c, g, G); break;
     }
   } else {
     if (T == 256) ok = resident_launch<true, 256, 1, 7>(c, g, G);
     else switch (CC) {
       case 1: ok = resident_launch<true, 512, 1, 7>(c, g, G); break;
       case 2: ok = resident_launch<true, 512, 2, 7>(c, g, G); break;
-      case 3: ok = resident_launch<true, 512, 3, 7>(c, g, G); break;
-      case 4:
-        ok = g.limit == RES_DEFAULT ? resident_launch<true, 512, 4, 7, false>(c, g, G)
-                                    : resident_launch<true, 512, 4, 7>(c, g, G);
-        break;
+      case 3: ok = either_launch<true, 512, 3, 7>(c, g, G); break;
+      case 4: ok = either_launch<true, 512, 4, 7>(c, g, G); break;
     }
   }
   if (!ok) return false;
