@@ -37,7 +37,7 @@
 // a wasted wait of 50 ms is as long as 5000 columns by panels.
 //
 // Measured per column, launch-per-column / resident (us): real order 128
-// 8.7 / 2.45, 380 9.8 / 2.6, 2588 (930 columns reduced) 16.2 / 6.0; complex
+// 8.7 / 2.45, 380 9.8 / 2.6, 2588 (930 columns reduced) 16.2 / 5.9; complex
 // order 1200 14.5 / 5.6 (with the update and the reflector before the
 // publication: 2.8, 2.9, 6.3, 5.7).  What bounds a column is the exchange,
 // then the chain of two workgroup-wide reductions.
